@@ -229,8 +229,6 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_wshift);
   dev_free(&c->d_lneed);
   dev_free(&c->d_trace);
-  dev_free(&c->d_node_obs);
-  dev_free(&c->d_node_nobs);
   dev_free(&c->d_off);
   dev_free(&c->d_st);
   dev_free(&c->d_start);
@@ -243,9 +241,8 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_targets);
   dev_free(&c->d_sel_q);
   dev_free(&c->d_sel);
-  dev_free(&c->d_geo);
-  dev_free(&c->d_sweep);
-  dev_free(&c->d_srange);
+  dev_free(&c->d_st4);
+  dev_free(&c->d_prec);
   dev_free(&c->d_act);
   dev_free(&c->d_act32);
   dev_free(&c->d_goalidx);
@@ -344,31 +341,35 @@ int dp_upload_primitives(dp_ctx* c, const dp_prims* pr, int32_t max_motions) {
   // translation leaves orientation unchanged, so cos/sin and the trailer's
   // offset from the state position are per-primitive constants.
   const int nbox = c->nbox;
-  std::vector<double> geo;
+  std::vector<double> st4, prec;
   std::vector<double> sweep((size_t)4 * P);
   if (!quad) {
-    geo.assign((size_t)4 * nbox * S, 0.0);
+    st4.resize((size_t)4 * nbox * S);
+    double* trl = st4.data() + (size_t)4 * S;  // the trailer's block
     const double hitch = c->desc.hitch;
     for (int32_t s = 0; s < S; ++s) {
       const double* x = st + (int64_t)s * nx;
       double c0 = std::cos(x[2]), s0 = std::sin(x[2]);
-      geo[(size_t)2 * S + s] = c0;
-      geo[(size_t)3 * S + s] = s0;
+      st4[(size_t)4 * s] = x[0];
+      st4[(size_t)4 * s + 1] = x[1];
+      st4[(size_t)4 * s + 2] = c0;
+      st4[(size_t)4 * s + 3] = s0;
       if (nbox > 1) {
         double c1 = std::cos(x[3]), s1 = std::sin(x[3]);
-        geo[(size_t)4 * S + s] = -(hitch * c1);
-        geo[(size_t)5 * S + s] = -(hitch * s1);
-        geo[(size_t)6 * S + s] = c1;
-        geo[(size_t)7 * S + s] = s1;
+        trl[(size_t)4 * s] = -(hitch * c1);
+        trl[(size_t)4 * s + 1] = -(hitch * s1);
+        trl[(size_t)4 * s + 2] = c1;
+        trl[(size_t)4 * s + 3] = s1;
       }
     }
     for (int32_t j = 0; j < P; ++j) {
       double lo0 = INFINITY, hi0 = -INFINITY, lo1 = INFINITY, hi1 = -INFINITY;
       for (int32_t s = off[j]; s < off[j + 1]; ++s) {
         for (int b = 0; b < nbox; ++b) {
-          double cx = st[(int64_t)s * nx] + (b ? geo[(size_t)4 * S + s] : 0.0);
-          double cy = st[(int64_t)s * nx + 1] + (b ? geo[(size_t)5 * S + s] : 0.0);
-          double cc = std::fabs(geo[(size_t)(4 * b + 2) * S + s]), ss = std::fabs(geo[(size_t)(4 * b + 3) * S + s]);
+          const double* g4 = b ? trl + (size_t)4 * s : st4.data() + (size_t)4 * s;
+          double cx = st[(int64_t)s * nx] + (b ? g4[0] : 0.0);
+          double cy = st[(int64_t)s * nx + 1] + (b ? g4[1] : 0.0);
+          double cc = std::fabs(g4[2]), ss = std::fabs(g4[3]);
           double hl = b ? c->desc.trailer_half[0] : c->desc.body_half[0];
           double hw = b ? c->desc.trailer_half[1] : c->desc.body_half[1];
           double ex = hl * cc + hw * ss, ey = hl * ss + hw * cc;
@@ -416,20 +417,28 @@ int dp_upload_primitives(dp_ctx* c, const dp_prims* pr, int32_t max_motions) {
   // "no state out of bounds" from it without reading the states.  A NaN
   // component gives a NaN range, which fails every comparison and so never
   // proves anything.
-  std::vector<double> srange((size_t)2 * nx * P);
-  for (int32_t j = 0; j < P; ++j) {
-    for (int k = 0; k < nx; ++k) {
-      double mn = INFINITY, mx = -INFINITY;
-      bool nan = false;
-      for (int32_t s = off[j]; s < off[j + 1]; ++s) {
-        const double v = st[(int64_t)s * nx + k];
-        nan = nan || v != v;
-        mn = std::min(mn, v);
-        mx = std::max(mx, v);
+  if (!quad) {
+    prec.assign((size_t)DP_PREC * P, 0.0);
+    for (int32_t j = 0; j < P; ++j) {
+      double* r = prec.data() + (size_t)DP_PREC * j;
+      for (int k = 0; k < 4; ++k) r[k] = sweep[(size_t)k * P + j];
+      for (int k = 0; k < nx; ++k) {
+        double mn = INFINITY, mx = -INFINITY;
+        bool nan = false;
+        for (int32_t s = off[j]; s < off[j + 1]; ++s) {
+          const double v = st[(int64_t)s * nx + k];
+          nan = nan || v != v;
+          mn = std::min(mn, v);
+          mx = std::max(mx, v);
+        }
+        if (nan) mn = mx = NAN;
+        r[DP_PREC_RANGE + 2 * k] = mn;
+        r[DP_PREC_RANGE + 2 * k + 1] = mx;
+        r[DP_PREC_START + k] = start[(size_t)k * P + j];
+        r[DP_PREC_LAST + k] = last[(size_t)k * P + j];
       }
-      if (nan) mn = mx = NAN;
-      srange[(size_t)k * P + j] = mn;
-      srange[((size_t)nx + k) * P + j] = mx;
+      const int32_t sl[2] = {off[j], off[j + 1] - off[j]};
+      std::memcpy(r + DP_PREC_S0, sl, sizeof(sl));
     }
   }
   int rc;
@@ -438,8 +447,6 @@ int dp_upload_primitives(dp_ctx* c, const dp_prims* pr, int32_t max_motions) {
   if ((rc = dev_alloc(&c->d_start, (int64_t)nx * P))) return rc;
   if ((rc = dev_alloc(&c->d_last, (int64_t)nx * P))) return rc;
   if ((rc = dev_alloc(&c->d_cost, P))) return rc;
-  if ((rc = dev_alloc(&c->d_sweep, (int64_t)4 * P))) return rc;
-  if ((rc = dev_alloc(&c->d_srange, (int64_t)2 * nx * P))) return rc;
   if ((rc = dev_alloc(&c->d_goalidx, (int64_t)8 * P))) return rc;
   HIP_CHECK(hipMemcpy(c->d_off, off.data(), sizeof(int32_t) * (P + 1), hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(c->d_st, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
@@ -455,11 +462,11 @@ int dp_upload_primitives(dp_ctx* c, const dp_prims* pr, int32_t max_motions) {
   HIP_CHECK(hipMemcpy(c->d_cost, cost.data(), sizeof(double) * P, hipMemcpyHostToDevice));
   dev_free(&c->d_order);  // a pair order refers to the previous primitive count
   c->order_rows = 0;
-  HIP_CHECK(hipMemcpy(c->d_sweep, sweep.data(), sizeof(double) * sweep.size(), hipMemcpyHostToDevice));
-  HIP_CHECK(hipMemcpy(c->d_srange, srange.data(), sizeof(double) * srange.size(), hipMemcpyHostToDevice));
   if (!quad) {
-    if ((rc = dev_alloc(&c->d_geo, (int64_t)geo.size()))) return rc;
-    HIP_CHECK(hipMemcpy(c->d_geo, geo.data(), sizeof(double) * geo.size(), hipMemcpyHostToDevice));
+    if ((rc = dev_alloc(&c->d_st4, (int64_t)st4.size()))) return rc;
+    HIP_CHECK(hipMemcpy(c->d_st4, st4.data(), sizeof(double) * st4.size(), hipMemcpyHostToDevice));
+    if ((rc = dev_alloc(&c->d_prec, (int64_t)prec.size()))) return rc;
+    HIP_CHECK(hipMemcpy(c->d_prec, prec.data(), sizeof(double) * prec.size(), hipMemcpyHostToDevice));
   } else {
     const int nu = c->desc.nu;
     const int64_t A = (int64_t)S - P;
@@ -635,8 +642,6 @@ int dp_reserve(dp_ctx* c, int32_t max_nodes, int64_t max_pairs) {
     if ((rc = dev_alloc(&c->d_node_count, max_nodes))) return rc;
     if ((rc = dev_alloc(&c->d_chunk, (int64_t)max_nodes + 1))) return rc;
     if ((rc = dev_alloc(&c->d_nshort, max_nodes))) return rc;
-    if ((rc = dev_alloc(&c->d_node_obs, (int64_t)DP_NODE_OBS * max_nodes))) return rc;
-    if ((rc = dev_alloc(&c->d_node_nobs, max_nodes))) return rc;
     c->N_cap = max_nodes;
   }
   if (max_pairs > c->pair_cap) {

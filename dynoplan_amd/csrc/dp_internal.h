@@ -10,8 +10,15 @@
 
 // Largest obstacle count staged in LDS by one workgroup.
 #define DP_MAX_OBS 1024
-// obstacles listed per frontier node for the swept-box cull of its pairs
-#define DP_NODE_OBS 128
+// Planar primitive record, DP_PREC doubles (two cache lines): what the check
+// reads of a pair's primitive.  First line: swept box (lo x, hi x, lo y,
+// hi y), min and max of each component, first state and state count (two
+// int32); second line: first and last state.
+#define DP_PREC 32
+#define DP_PREC_RANGE 4
+#define DP_PREC_S0 14
+#define DP_PREC_START 16
+#define DP_PREC_LAST 21
 // Per-pair resolution value while undecided (ordered duplicate resolution).
 #define DP_R_UNDECIDED 0x7f
 // Pair flag set by the pre-resolution: every earlier contender is decided
@@ -180,9 +187,8 @@ struct dp_ctx {
   float* d_start32 = nullptr;    // [nx][P] FP32 copies of the keys (exact rejections with margins)
   float* d_last32 = nullptr;
   double* d_cost = nullptr;      // [P] motion cost (given, or ref_dt per action)
-  double* d_geo = nullptr;       // [4*nbox][S] : relx rely c s (per box)
-  double* d_sweep = nullptr;     // [4][P] canonical swept footprint box (planar) / centre box (quad)
-  double* d_srange = nullptr;    // [2][nx][P] per-primitive min / max of each state component (canonical)
+  double* d_st4 = nullptr;       // planar: [nbox][S][4] (x, y, cos, sin), then the trailer's (offset x, y, cos, sin)
+  double* d_prec = nullptr;      // planar: [P][DP_PREC] primitive records
   double* d_act = nullptr;       // [A][nu] (quadrotor: nu = 4, 32-byte rows)
   float* d_act32 = nullptr;      // [A][nu] (16-byte rows)
   int32_t* d_goalidx = nullptr;  // [8][P]
@@ -279,8 +285,6 @@ struct dp_ctx {
   bool select_mode = false;         // set while dp_expand_select enqueues its kernels
   double select_radius = 0.0, select_cost_jump = 0.0;
   int32_t select_first = 0;
-  int16_t* d_node_obs = nullptr;    // [N_cap][DP_NODE_OBS] obstacles within a node's reach box
-  int32_t* d_node_nobs = nullptr;   // [N_cap] their count (-1: more than DP_NODE_OBS)
   dp_mlp mlp;
   int32_t round_limit = 0;          // limit_branching_factor of the batch in flight
   dp_expand_params round_params{};  // parameters of the batch in flight

@@ -345,17 +345,15 @@ struct dp_check_args {
   const int32_t* off;
   const double* st;
   int32_t S;
-  const double* geo;
-  int32_t nbox;
-  const double* sweep;
-  const double* srange;  // [2][NX][P] per-primitive min / max of each component
+  const double4* st4;    // [boxes][S] per state: (x, y, cos, sin) of the body, then the trailer's (offset x, y, cos, sin)
+  const double* prec;    // [P][DP_PREC] what a pair reads of its primitive
+  double reach[4];       // union of the swept boxes relative to a node (lo x, hi x, lo y, hi y)
+  int32_t ppw;           // pairs per wave, 1 to 64 (0: from the pair count)
   int32_t P;
   const int32_t* goalidx;
   int32_t num_goal, check_goal;
   const double* obs;
   int32_t nobs;
-  const int16_t* node_obs;   // [Ncap][DP_NODE_OBS] ascending obstacle indices near each node
-  const int32_t* node_nobs;  // [Ncap] their count, -1 when the list overflowed (scan all)
   const double* vis;
   int64_t vstride;
   int64_t nv;
@@ -380,7 +378,6 @@ struct dp_check_args {
   // tdbastar's reverse search: placement offset = node - last position of
   // the primitive, new state = first placed state
   int32_t backward;
-  const double* last;  // [nx][P]
   // tdbastar constraints: times [ncon], then states [ncon][nx]
   int32_t ncon;
   const double* con;
@@ -399,50 +396,106 @@ __device__ __forceinline__ void load_translated(const dp_check_args& a, int64_t 
   for (int c = 2; c < NX; ++c) s[c] = a.st[(int64_t)c * a.S + sidx];
 }
 
+// Flattened items of a wave: segments of 0 or more items, numbered one after
+// another and dealt to the 64 lanes in turn.  A bitmap of the segments' first
+// items gives an item's segment by a bit count, kItemWindow items at a time.
+constexpr int kItemWindow = 4096;
 
-// Per frontier node, the obstacles that can touch any of its primitives: the
-// swept box of every primitive lies inside the union box `reach`, and the
-// pair test below uses the same rounding form with the larger box, so every
-// obstacle a pair's swept-box cull keeps is on its node's list.  One wave per
-// node; lists hold ascending indices.
-__global__ __launch_bounds__(256) void k_node_obs(const double* nodes, int32_t Ncap, int32_t N, const double* obs,
-                                                  int32_t nobs, double r0, double r1, double r2, double r3,
-                                                  int16_t* node_obs, int32_t* node_nobs) {
-  const int lane = threadIdx.x % 64;
-  for (int64_t i = (int64_t)blockIdx.x * kWaves + threadIdx.x / 64; i < N; i += (int64_t)gridDim.x * kWaves) {
-    const double ox = nodes[i], oy = nodes[(int64_t)Ncap + i];
-    const double bx0 = (r0 + ox) - DP_SWEEP_PAD, bx1 = (r1 + ox) + DP_SWEEP_PAD;
-    const double by0 = (r2 + oy) - DP_SWEEP_PAD, by1 = (r3 + oy) + DP_SWEEP_PAD;
-    int cnt = 0;
-    for (int ob = 0; ob < nobs; ob += 64) {
-      const int o = ob + lane;
-      bool hit = false;
-      if (o < nobs) {
-        const double* b = obs + 4 * o;
-        hit = !(b[0] + b[2] < bx0 || b[0] - b[2] > bx1 || b[1] + b[3] < by0 || b[1] - b[3] > by1);
-      }
-      const uint64_t m = __ballot(hit);
-      const int at = cnt + __popcll(m & ((1ull << lane) - 1ull));
-      if (hit && at < DP_NODE_OBS) node_obs[i * DP_NODE_OBS + at] = (int16_t)o;
-      cnt += __popcll(m);
+// Per-wave LDS of k_check_planar (6 KB for three components, 7 KB for five).
+template <int NX>
+struct check_wave {
+  uint64_t head[kItemWindow / 64];
+  // bounds and collision: per segment (a pair with states to test)
+  int32_t pre[64];           // its first item
+  int32_t st0[64];           // first state of the pair's primitive (complemented: bounds to be tested too)
+  int32_t bad[64], col[64];  // first offending / colliding state so far (constraints: bad = first violated one)
+  uint64_t mask[64];         // obstacles of the staged chunk that meet the pair's swept box
+  double ox[64], oy[64];     // placement offset
+  union {
+    struct {
+      int32_t len[64], reach[64];
+      float g[64];
+    } con;                   // constraints: per pair to test
+    struct {
+      double x[NX][64];      // state of the new node, per lane
+      int2 run[9 * 64];      // per non-empty run: the pair's lane, sorted position minus first item
+    } vis;
+  };
+};
+
+__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  return v;
+}
+
+// Calls set(window start) for each window of items (it marks the first items
+// of the segments in head[], relative to the window), then item(segment, f)
+// for every item f < T of it.
+template <typename Set, typename Item>
+__device__ __forceinline__ void for_items(uint64_t* head, int T, int lane, Set&& set, Item&& item) {
+  const uint64_t le = (2ull << lane) - 1ull;
+  int base = -1;
+  for (int w0 = 0; w0 < T; w0 += kItemWindow) {
+    head[lane] = 0ull;
+    wave_lds_sync();
+    set(w0);
+    wave_lds_sync();
+    for (int r = 0; r < 64 && w0 + 64 * r < T; ++r) {
+      const uint64_t h = head[r];
+      const int f = w0 + 64 * r + lane;
+      if (f < T) item(base + (int)__popcll(h & le), f);
+      base += __builtin_amdgcn_readfirstlane((int)__popcll(h));
     }
-    if (lane == 0) node_nobs[i] = cnt <= DP_NODE_OBS ? cnt : -1;
+    wave_lds_sync();
   }
 }
 
-// Planar translate systems (unicycle1/2, car+trailer), FP64.
-template <int NX, int LPP>
+__device__ __forceinline__ void mark_item(uint64_t* head, int f, int w0) {
+  const int r = f - w0;
+  if (r >= 0 && r < kItemWindow) atomicOr((unsigned long long*)&head[r >> 6], 1ull << (r & 63));
+}
+
+// Planar translate systems (unicycle1/2, car+trailer), FP64.  A wave takes
+// a.ppw consecutive pairs, one per lane, and spreads what varies in length
+// between pairs (states against obstacles, constraints, visited candidates)
+// over all 64 lanes as one flattened list, so that a pair's length costs its
+// share and the loads of 64 items are in flight together.
+//
+// It is bound by the latency of its chains of dependent loads (pair ->
+// primitive record -> states; final state -> cell starts -> candidates) at
+// three waves per SIMD.  A split of LPP lanes per pair, each lane one state,
+// did the once-per-pair work LPP times and ran every group to its longest
+// primitive.  Measured, 1.95M pairs of 5-30 states, 200 boxes, 100k visited:
+// 32 lanes per pair (the old rule for that length) 2.03 ms, the best split
+// (4) 0.69 ms, this form 0.32 ms, of which states against boxes 0.10, the
+// visited set 0.10, setting up and writing the pairs the rest.  0.50M car
+// pairs, 300 boxes: 1.07 -> 0.18 ms.
+//
+// Pairs per wave without a setting: about 2304 waves (9 per CU) over the
+// batch, read on the device.  Fewer pairs per wave leave fewer states to
+// one wave but idle lanes in the once-per-pair part: 24k pairs 64 / 16 / 4
+// per wave 50 / 33 / 58 us, 143k pairs 56 / 79 / 153 us.
+template <int NX>
 __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
-  static_assert(LPP >= 2 && 64 % LPP == 0, "a pair takes 2 to 64 lanes of a wave");
   extern __shared__ double smem[];
   // the system constants in LDS: read from global memory after the loop's
   // stores, each would be a load the wave waits for
   __shared__ dp_dev_sys s_sys;
+  __shared__ check_wave<NX> s_wave[kWaves];
   const dp_dev_sys& S = s_sys;
   const int nobs = a.nobs;
-  if ((int64_t)blockIdx.x * kWaves * (64 / LPP) >= (int64_t)*a.total) return;  // uniform per block
+  // a.ppw 0: about 9 waves per CU over the batch's pairs, 4 to 64 pairs each
+  int ppw = a.ppw;
+  if (ppw == 0) {
+    const int want = *a.total / 2304;
+    ppw = want <= 4 ? 4 : want <= 8 ? 8 : want <= 16 ? 16 : want <= 32 ? 32 : 64;
+  }
+  if ((int64_t)blockIdx.x * kWaves * ppw >= (int64_t)*a.total) return;  // uniform per block
   double* s_obs = smem;  // [nobs][4]
-  int16_t* s_cand = (int16_t*)(smem + 4 * nobs);
   for (int t = threadIdx.x; t < 4 * nobs; t += blockDim.x) s_obs[t] = a.obs[t];
   static_assert(sizeof(dp_dev_sys) % sizeof(double) == 0, "copied as doubles");
   for (int t = threadIdx.x; t < (int)(sizeof(dp_dev_sys) / sizeof(double)); t += blockDim.x)
@@ -452,44 +505,20 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
   if (threadIdx.x < 5) s_cnt[threadIdx.x] = 0ull;
   __syncthreads();
 
-  constexpr int SEG = 64 / LPP;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
-  const int seg = lane / LPP, k0 = lane % LPP;
-  const int shift = seg * LPP;
-  const uint64_t segbits = LPP == 64 ? ~0ull : ((1ull << LPP) - 1ull);
-  const uint64_t ltmask = (1ull << k0) - 1ull;
-  int16_t* cand = s_cand + (int64_t)(wave * SEG + seg) * nobs;
+  check_wave<NX>& W = s_wave[wave];
+  int16_t* list = (int16_t*)(smem + 4 * nobs) + (int64_t)wave * nobs;  // obstacles near the node being checked
+  const uint64_t lt = (1ull << lane) - 1ull;
   const int32_t total = *a.total;
-  const double Tdup = dp_pos_bound(S, a.r_dup);
-  long long c_b = 0, c_c = 0, c_f = 0, c_k = 0, c_x = 0;
-  // bounds and footprint held in registers: read inside the loops below
-  // (after the loop's stores) every bound would be a load and a wait
-  double blo[NX], bhi[NX];
-#pragma unroll
-  for (int c = 0; c < NX; ++c) {
-    blo[c] = S.lo[c];
-    bhi[c] = S.hi[c];
-  }
-  const double body_hl = S.body_hl, body_hw = S.body_hw, trailer_hl = S.trailer_hl, trailer_hw = S.trailer_hw;
+  const double Tdup = dp_pos_bound(S, a.r_dup), Tgoal = dp_pos_bound(S, a.goal_bound);
+  int c_b = 0, c_c = 0, c_f = 0, c_k = 0, c_x = 0;
 
-  for (int64_t q0 = ((int64_t)blockIdx.x * kWaves + wave) * SEG; q0 < total;
-       q0 += (int64_t)gridDim.x * kWaves * SEG) {
-    const int64_t q = q0 + seg;
-    const bool vp = q < total && !(a.surrogate && a.verdict[q] == DP_V_SURROGATE_REJECT);
+  for (int64_t q0 = ((int64_t)blockIdx.x * kWaves + wave) * ppw; q0 < total; q0 += (int64_t)gridDim.x * kWaves * ppw) {
+    const int64_t q = q0 + lane;
+    const bool vp = lane < ppw && q < total && !(a.surrogate && a.verdict[q] == DP_V_SURROGATE_REJECT);
     int32_t i = 0, j = 0, st0 = 0, L1 = 0;
     double ox = 0.0, oy = 0.0;
-    if (vp) {
-      i = a.pnode[q];
-      j = a.pprim[q];
-      st0 = a.off[j];
-      L1 = a.off[j + 1] - st0;
-      ox = a.nodes[i];
-      oy = a.nodes[(int64_t)a.Ncap + i];
-      if (a.backward) {  // offset - motion->traj.states.back().head(2), tdbastar.hpp:193-196
-        ox = ox - a.last[j];
-        oy = oy - a.last[(int64_t)a.P + j];
-      }
-    }
+    const double* rec = a.prec;
     // ---- is_state_valid on every translated state -----------------------
     // First from the primitive's component ranges: with the translation
     // rounded the same way, (min + offset) >= lo and (max + offset) <= hi
@@ -497,101 +526,138 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
     // compare their range directly.  Only pairs not cleared this way scan
     // their states for the first offending index.
     bool clear = true;
+    double bx0 = 0, bx1 = 0, by0 = 0, by1 = 0;
+    double tx0 = 0, tx1 = 0, ty0 = 0, ty1 = 0;  // range of the placed positions
     if (vp) {
+      i = a.pnode[q];
+      j = a.pprim[q];
+      rec = a.prec + (int64_t)j * DP_PREC;
+      const int2 sl = *reinterpret_cast<const int2*>(rec + DP_PREC_S0);
+      st0 = sl.x;
+      L1 = sl.y;
+      ox = a.nodes[i];
+      oy = a.nodes[(int64_t)a.Ncap + i];
+      if (a.backward) {  // offset - motion->traj.states.back().head(2), tdbastar.hpp:193-196
+        ox = ox - rec[DP_PREC_LAST];
+        oy = oy - rec[DP_PREC_LAST + 1];
+      }
+      bx0 = (rec[0] + ox) - DP_SWEEP_PAD;
+      bx1 = (rec[1] + ox) + DP_SWEEP_PAD;
+      by0 = (rec[2] + oy) - DP_SWEEP_PAD;
+      by1 = (rec[3] + oy) + DP_SWEEP_PAD;
 #pragma unroll
       for (int c = 0; c < NX; ++c) {
         const double o = c == 0 ? ox : (c == 1 ? oy : 0.0);
-        const double mn = a.srange[(int64_t)c * a.P + j], mx = a.srange[((int64_t)NX + c) * a.P + j];
+        const double mn = rec[DP_PREC_RANGE + 2 * c], mx = rec[DP_PREC_RANGE + 2 * c + 1];
         const double tmn = c < 2 ? mn + o : mn, tmx = c < 2 ? mx + o : mx;
-        clear = clear & (tmn >= blo[c]) & (tmx <= bhi[c]);
+        clear = clear & (tmn >= S.lo[c]) & (tmx <= S.hi[c]);
+        if (c == 0) tx0 = tmn, tx1 = tmx;
+        if (c == 1) ty0 = tmn, ty1 = tmx;
       }
     }
-    int first_bad = INT_MAX;
-    for (int kb = 0; __ballot(vp && !clear && kb < L1) != 0; kb += LPP) {
-      const int k = kb + k0;
-      bool bad = false;
-      if (vp && !clear && k < L1) {
-        const int64_t sidx = (int64_t)st0 + k;
-        double s[NX];
-        load_translated<NX>(a, sidx, ox, oy, s);
-#pragma unroll
-        for (int c = 0; c < NX; ++c) bad = bad | !((s[c] >= blo[c]) & (s[c] <= bhi[c]));
-      }
-      const uint64_t m = (__ballot(bad) >> shift) & segbits;
-      if (first_bad == INT_MAX && m) first_bad = kb + __ffsll((long long)m) - 1;
-    }
-    int8_t vd = first_bad != INT_MAX ? DP_V_BOUNDS : DP_V_FREE;
-    const bool need_col = vp && vd == DP_V_FREE;
+    int first_bad = INT_MAX, first_col = INT_MAX;
 
-    // ---- collision: swept-box cull, then SAT per state ------------------
-    int first_col = INT_MAX;
-    if (__ballot(need_col)) {
-      double bx0 = 0, bx1 = 0, by0 = 0, by1 = 0;
-      if (need_col) {
-        bx0 = (a.sweep[j] + ox) - DP_SWEEP_PAD;
-        bx1 = (a.sweep[(int64_t)a.P + j] + ox) + DP_SWEEP_PAD;
-        by0 = (a.sweep[2 * (int64_t)a.P + j] + oy) - DP_SWEEP_PAD;
-        by1 = (a.sweep[3 * (int64_t)a.P + j] + oy) + DP_SWEEP_PAD;
-      }
-      // scan the node's obstacle list (all obstacles when it overflowed)
+    // ---- bounds and collision, node by node of the wave's pairs ----------
+    for (uint64_t todo = __ballot(vp); todo;) {
+      const int src = __ffsll((long long)todo) - 1;
+      const int32_t node = __builtin_amdgcn_readlane(i, src);
+      const bool mine = vp && i == node;
+      todo &= ~__ballot(mine);
+      // Obstacles that can touch any of the node's primitives: every swept
+      // box lies inside the union box `reach` and both tests round the same
+      // way, so the list holds every obstacle that a pair's own box meets.
       int nlist = 0;
-      const int16_t* list = nullptr;
-      if (need_col) {
-        nlist = a.node_nobs[i];
-        if (nlist >= 0) list = a.node_obs + (int64_t)i * DP_NODE_OBS;
-        else nlist = nobs;
-      }
-      int ncand = 0;
-      for (int ob = 0; __ballot(need_col && ob < nlist) != 0; ob += LPP) {
-        const int t = ob + k0;
-        bool hit = false;
-        int o = 0;
-        if (need_col && t < nlist) {
-          o = list ? list[t] : t;
-          const double* b = s_obs + 4 * o;
-          hit = !(b[0] + b[2] < bx0 || b[0] - b[2] > bx1 || b[1] + b[3] < by0 || b[1] - b[3] > by1);
+      {
+        const double nox = a.nodes[node], noy = a.nodes[(int64_t)a.Ncap + node];
+        const double rx0 = (a.reach[0] + nox) - DP_SWEEP_PAD, rx1 = (a.reach[1] + nox) + DP_SWEEP_PAD;
+        const double ry0 = (a.reach[2] + noy) - DP_SWEEP_PAD, ry1 = (a.reach[3] + noy) + DP_SWEEP_PAD;
+        for (int ob = 0; ob < nobs; ob += 64) {
+          const int o = ob + lane;
+          bool hit = false;
+          if (o < nobs) {
+            const double* b = s_obs + 4 * o;
+            hit = !(b[0] + b[2] < rx0 || b[0] - b[2] > rx1 || b[1] + b[3] < ry0 || b[1] - b[3] > ry1);
+          }
+          const uint64_t m = __ballot(hit);
+          if (hit) list[nlist + __popcll(m & lt)] = (int16_t)o;
+          nlist += __popcll(m);
         }
-        const uint64_t m = (__ballot(hit) >> shift) & segbits;
-        if (hit) cand[ncand + __popcll(m & ltmask)] = (int16_t)o;
-        ncand += __popcll(m);
       }
       wave_lds_sync();
-      for (int kb = 0; __ballot(need_col && ncand > 0 && kb < L1) != 0; kb += LPP) {
-        const int k = kb + k0;
-        bool col = false;
-        if (need_col && ncand > 0 && k < L1 && first_col == INT_MAX) {
-          const int64_t sidx = (int64_t)st0 + k;
-          const double x = a.st[sidx] + ox;
-          const double y = a.st[(int64_t)a.S + sidx] + oy;
-          for (int bi = 0; bi < a.nbox && !col; ++bi) {
-            const double c = a.geo[(int64_t)(4 * bi + 2) * a.S + sidx];
-            const double s = a.geo[(int64_t)(4 * bi + 3) * a.S + sidx];
-            double cx = x, cy = y, hl = body_hl, hw = body_hw;
-            if (bi > 0) {
-              cx = x + a.geo[(int64_t)(4 * bi) * a.S + sidx];
-              cy = y + a.geo[(int64_t)(4 * bi + 1) * a.S + sidx];
-              hl = trailer_hl;
-              hw = trailer_hw;
-            }
-            for (int t = 0; t < ncand; ++t) {
-              const double* b = s_obs + 4 * cand[t];
-              if (dp_obb_aabb(cx, cy, c, s, hl, hw, b[0], b[1], b[2], b[3])) {
-                col = true;
-                break;
-              }
-            }
-          }
+      // 64 obstacles of the list at a time, one bit each
+      for (int c0 = 0; c0 == 0 || c0 < nlist; c0 += 64) {
+        const int nc = nlist - c0 < 64 ? nlist - c0 : 64;
+        uint64_t mask = 0ull;
+        for (int t = 0; t < nc; ++t) {
+          const double* b = s_obs + 4 * list[c0 + t];
+          const bool hit = !(b[0] + b[2] < bx0 || b[0] - b[2] > bx1 || b[1] + b[3] < by0 || b[1] - b[3] > by1);
+          mask |= hit ? 1ull << t : 0ull;
         }
-        const uint64_t m = (__ballot(col) >> shift) & segbits;
-        if (first_col == INT_MAX && m) first_col = kb + __ffsll((long long)m) - 1;
+        const bool scan = mine && (mask != 0ull || (c0 == 0 && !clear));
+        const int n = scan ? L1 : 0;
+        const int incl = wave_incl_scan(n, lane);
+        const int T = __builtin_amdgcn_readlane(incl, 63);
+        const int seg = __popcll(__ballot(scan) & lt);
+        if (scan) {
+          W.pre[seg] = incl - n;
+          W.mask[seg] = mask;
+          W.st0[seg] = clear ? st0 : ~st0;
+          W.ox[seg] = ox;
+          W.oy[seg] = oy;
+          W.bad[seg] = INT_MAX;
+          W.col[seg] = INT_MAX;
+        }
+        for_items(
+            W.head, T, lane,
+            [&](int w0) {
+              if (scan) mark_item(W.head, incl - n, w0);
+            },
+            [&](int p, int f) {
+              const int k = f - W.pre[p];
+              const int32_t s0 = W.st0[p];
+              const int64_t sidx = (int64_t)(s0 < 0 ? ~s0 : s0) + k;
+              const double4 s4 = a.st4[sidx];
+              const double x = s4.x + W.ox[p], y = s4.y + W.oy[p];
+              if (s0 < 0 && c0 == 0) {
+                bool bad = !((x >= S.lo[0]) & (x <= S.hi[0])) | !((y >= S.lo[1]) & (y <= S.hi[1]));
+#pragma unroll
+                for (int c = 2; c < NX; ++c) {
+                  const double v = a.st[(int64_t)c * a.S + sidx];
+                  bad = bad | !((v >= S.lo[c]) & (v <= S.hi[c]));
+                }
+                if (bad) atomicMin(&W.bad[p], k);
+              }
+              bool col = false;
+              const uint64_t m0 = W.mask[p];
+              for (uint64_t m = m0; m && !col; m &= m - 1ull) {
+                const double* b = s_obs + 4 * list[c0 + __ffsll((long long)m) - 1];
+                col = dp_obb_aabb(x, y, s4.z, s4.w, S.body_hl, S.body_hw, b[0], b[1], b[2], b[3]);
+              }
+              if constexpr (NX == 4) {  // the trailer's box, at its offset from the state position
+                if (m0 && !col) {
+                  const double4 t4 = a.st4[(int64_t)a.S + sidx];
+                  const double cx = x + t4.x, cy = y + t4.y;
+                  for (uint64_t m = m0; m && !col; m &= m - 1ull) {
+                    const double* b = s_obs + 4 * list[c0 + __ffsll((long long)m) - 1];
+                    col = dp_obb_aabb(cx, cy, t4.z, t4.w, S.trailer_hl, S.trailer_hw, b[0], b[1], b[2], b[3]);
+                  }
+                }
+              }
+              if (col) atomicMin(&W.col[p], k);
+            });
+        if (scan) {
+          first_bad = min(first_bad, W.bad[seg]);
+          first_col = min(first_col, W.col[seg]);
+        }
+        wave_lds_sync();
       }
-      wave_lds_sync();  // candidate list is rewritten by the next pair group
-      if (need_col && first_col != INT_MAX) vd = DP_V_COLLIDE;
     }
+    int8_t vd = first_bad != INT_MAX ? DP_V_BOUNDS : (first_col != INT_MAX ? DP_V_COLLIDE : DP_V_FREE);
 
     // ---- tdbastar constraints on a valid pair (tdbastar.cpp:408-443) -----
-    // LPP constraints at a time; the first violated one in list order wins.
-    if (a.ncon > 0 && __ballot(vp && vd == DP_V_FREE)) {
+    // (pair, constraint) items; the first violated constraint in list order
+    // wins.
+    if (a.ncon > 0) {
       const bool nc = vp && vd == DP_V_FREE;
       bool reaches = false;
       float gf = 0.0f;
@@ -601,66 +667,83 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
         reaches = dp_distance(S, s, a.goal) <= a.con_delta;
         gf = (float)a.gpar[i];  // best_node_gScore is passed as float
       }
-      int viol_k = -1;
-      for (int cb = 0; __ballot(nc && viol_k < 0 && cb < a.ncon) != 0; cb += LPP) {
-        const int ci = cb + k0;
-        bool viol = false;
+      // state that constraint ci selects for a pair, or -1
+      auto con_state = [&](int ci, float g_f, bool reach, int len) {
+        const float toff = (float)(a.con[ci] - (double)g_f);
+        const int ti = (int)lround((double)toff / S.dt);
         int k = -1;
-        if (nc && viol_k < 0 && ci < a.ncon) {
-          const float toff = (float)(a.con[ci] - (double)gf);
-          const int ti = (int)lround((double)toff / S.dt);
-          if (reaches && ti >= L1 - 1) k = L1 - 1;
-          if (ti >= 0 && ti < L1 - 1) k = ti;
-          if (k >= 0) {
-            double s[NX], cs[NX];
-            load_translated<NX>(a, (int64_t)st0 + k, ox, oy, s);
+        if (reach && ti >= len - 1) k = len - 1;
+        if (ti >= 0 && ti < len - 1) k = ti;
+        return k;
+      };
+      const uint64_t ncm = __ballot(nc);
+      const int np = __popcll(ncm), seg = __popcll(ncm & lt);
+      if (nc) {  // the pairs to test, packed
+        W.st0[seg] = st0;
+        W.ox[seg] = ox;
+        W.oy[seg] = oy;
+        W.bad[seg] = INT_MAX;  // first violated constraint
+        W.con.len[seg] = L1;
+        W.con.reach[seg] = reaches ? 1 : 0;
+        W.con.g[seg] = gf;
+      }
+      wave_lds_sync();
+      for (int64_t f = lane; f < (int64_t)np * a.ncon; f += 64) {
+        const int p = (int)(f / a.ncon), ci = (int)(f % a.ncon);
+        if (W.bad[p] < ci) continue;  // an earlier one is violated
+        const int k = con_state(ci, W.con.g[p], W.con.reach[p] != 0, W.con.len[p]);
+        if (k < 0) continue;
+        double s[NX], cs[NX];
+        load_translated<NX>(a, (int64_t)W.st0[p] + k, W.ox[p], W.oy[p], s);
 #pragma unroll
-            for (int c = 0; c < NX; ++c) cs[c] = a.con[a.ncon + (int64_t)ci * NX + c];
-            viol = dp_distance(S, s, cs) <= a.con_delta;
-          }
-        }
-        const uint64_t m = (__ballot(viol) >> shift) & segbits;
-        const int src = m ? shift + __ffsll((long long)m) - 1 : lane;
-        const int kk = __shfl(k, src);
-        if (nc && viol_k < 0 && m) viol_k = kk;
+        for (int c = 0; c < NX; ++c) cs[c] = a.con[a.ncon + (int64_t)ci * NX + c];
+        if (dp_distance(S, s, cs) <= a.con_delta) atomicMin(&W.bad[p], ci);
       }
-      if (nc && viol_k >= 0) {
+      wave_lds_sync();
+      if (nc && W.bad[seg] != INT_MAX) {
         vd = DP_V_CONSTRAINT;
-        first_col = viol_k;
+        first_col = con_state(W.bad[seg], gf, reaches, L1);
       }
+      wave_lds_sync();
     }
 
     // ---- FREE: check_goal, g, h, duplicate vs visited --------------------
     const bool fr = vp && vd == DP_V_FREE;
     int chosen = -1;
-    if (a.check_goal && !a.select && __ballot(fr)) {
-      // goal indices LPP at a time; the first in index order that hits wins
-      for (int gb = 0; gb < a.num_goal; gb += LPP) {
-        const int gk = gb + k0;
-        bool hit = false;
-        if (fr && chosen == -1 && gk < a.num_goal) {
+    if (a.check_goal && !a.select && fr) {
+      // The position range of the placed states against the goal: beyond the
+      // bound no state can reach it (the differences and their squares round
+      // monotonically, dp_pos_bound covers the root), so most pairs load none
+      // of the goal states.
+      const double dx = fmax(fmax(tx0 - a.goal[0], a.goal[0] - tx1), 0.0);
+      const double dy = fmax(fmax(ty0 - a.goal[1], a.goal[1] - ty1), 0.0);
+      double s2 = dx * dx;
+      s2 = s2 + dy * dy;
+      if (!(s2 > Tgoal))
+        for (int gk = 0; gk < a.num_goal && chosen == -1; ++gk) {
           const int idx = a.goalidx[(int64_t)gk * a.P + j];
           double s[NX];
           load_translated<NX>(a, (int64_t)st0 + idx, ox, oy, s);
-          hit = dp_within(S, s, a.goal, a.goal_bound);
+          if (dp_within(S, s, a.goal, a.goal_bound)) chosen = idx;
         }
-        const uint64_t m = (__ballot(hit) >> shift) & segbits;
-        if (fr && chosen == -1 && m) chosen = a.goalidx[(int64_t)(gb + __ffsll((long long)m) - 1) * a.P + j];
-      }
     }
     double xf[NX];
     double gq = 0.0, hq = 0.0;
     if (fr) {
       // the new node's state: the last placed state, or the first for the
       // reverse search (check_goal, tdbastar.cpp:453-458)
-      const int fi = chosen != -1 ? chosen : (a.backward ? 0 : L1 - 1);
-      load_translated<NX>(a, (int64_t)st0 + fi, ox, oy, xf);
-      hq = dp_lower_bound_time(S, xf, a.goal);
-      const double cm = chosen != -1 ? chosen * S.dt : (L1 - 1) * S.dt;
       double nd[NX], t0[NX];
 #pragma unroll
-      for (int c = 0; c < NX; ++c) nd[c] = a.nodes[(int64_t)c * a.Ncap + i];
-      load_translated<NX>(a, (int64_t)st0, ox, oy, t0);
+      for (int c = 0; c < NX; ++c) {
+        const double o = c == 0 ? ox : oy;
+        nd[c] = a.nodes[(int64_t)c * a.Ncap + i];
+        const double first = rec[DP_PREC_START + c], last = rec[DP_PREC_LAST + c];
+        t0[c] = c < 2 ? first + o : first;
+        xf[c] = a.backward ? t0[c] : (c < 2 ? last + o : last);
+      }
+      if (chosen != -1) load_translated<NX>(a, (int64_t)st0 + chosen, ox, oy, xf);
+      hq = dp_lower_bound_time(S, xf, a.goal);
+      const double cm = chosen != -1 ? chosen * S.dt : (L1 - 1) * S.dt;
       gq = a.gpar[i] + cm + a.cdf * dp_lower_bound_time(S, nd, t0);
     } else {
 #pragma unroll
@@ -668,13 +751,77 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
     }
     bool dupv = false;
     if (a.nv > 0 && !a.select && __ballot(fr)) {
-      bool hit = false;
-      // the 9 runs over the pair's lanes (one round from 16 lanes per pair)
-      for (int k = k0; fr && k < 9 && !hit; k += LPP)
-        hit = dp_grid_run_any<NX>(S, a.grid, a.vstart, a.vis, a.vstride, xf, k, a.r_dup, Tdup);
-      dupv = ((__ballot(hit) >> shift) & segbits) != 0;
+      // the 9 runs of each final state's 27-cell block (dp_grid_run_any's
+      // rules), their bounds loaded together
+      int32_t rb[9], rn[9];
+      int K = 0, nr = 0;
+#pragma unroll
+      for (int k = 0; k < 9; ++k) rb[k] = rn[k] = 0;
+      if (fr) {
+        const dp_grid_geom& G = a.grid;
+        int32_t c[3];
+        dp_cell_coords(G, xf, c);
+        const int32_t x0 = c[0] > 0 ? c[0] - 1 : 0, x1 = c[0] + 1 < G.dims[0] ? c[0] + 1 : G.dims[0] - 1;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          const int32_t n1 = c[1] + k % 3 - 1, d2 = k / 3 - 1;
+          int32_t n2 = c[2] + d2;
+          bool ok = n1 >= 0 && n1 < G.dims[1];
+          if (G.dims[2] == 1) {
+            ok = ok && d2 == 0;
+            n2 = 0;
+          } else if (G.periodic2) {
+            n2 = n2 < 0 ? n2 + G.dims[2] : (n2 >= G.dims[2] ? n2 - G.dims[2] : n2);
+          } else {
+            ok = ok && n2 >= 0 && n2 < G.dims[2];
+          }
+          const int64_t row = ok ? ((int64_t)n2 * G.dims[1] + n1) * G.dims[0] : 0;
+          rb[k] = a.vstart[ok ? row + x0 : 0];
+          rn[k] = a.vstart[ok ? row + x1 + 1 : 0];
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          rn[k] -= rb[k];
+          K += rn[k];
+          nr += rn[k] > 0 ? 1 : 0;
+        }
+      }
+      const int incl = wave_incl_scan(K, lane), run0 = wave_incl_scan(nr, lane) - nr;
+      const int T = __builtin_amdgcn_readlane(incl, 63);
+      {
+        int f = incl - K, at = run0;
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+          if (rn[k] > 0) {
+            W.vis.run[at++] = make_int2(lane, rb[k] - f);
+            f += rn[k];
+          }
+      }
+      W.bad[lane] = 0;
+#pragma unroll
+      for (int c = 0; c < NX; ++c) W.vis.x[c][lane] = xf[c];
+      for_items(
+          W.head, T, lane,
+          [&](int w0) {
+            int f = incl - K;
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+              if (rn[k] > 0) {
+                mark_item(W.head, f, w0);
+                f += rn[k];
+              }
+          },
+          [&](int run, int f) {
+            const int2 r = W.vis.run[run];
+            double x[NX];
+#pragma unroll
+            for (int c = 0; c < NX; ++c) x[c] = W.vis.x[c][r.x];
+            if (dp_within_col_pf<NX>(S, x, a.vis, a.vstride, (int64_t)f + r.y, a.r_dup, Tdup)) W.bad[r.x] = 1;
+          });
+      dupv = fr && W.bad[lane] != 0;
+      wave_lds_sync();
     }
-    if (vp && k0 == 0) {
+    if (vp) {
       a.verdict[q] = vd;
       a.firstk[q] = vd == DP_V_BOUNDS ? first_bad : (vd == DP_V_COLLIDE || vd == DP_V_CONSTRAINT ? first_col : -1);
       a.goal_out[q] = chosen;
@@ -686,14 +833,14 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
         a.gout[q] = gq;
         a.hout[q] = hq;
       }
-      c_b += vd == DP_V_BOUNDS;
-      c_c += vd == DP_V_COLLIDE;
-      c_x += vd == DP_V_CONSTRAINT;
-      c_f += fr;
-      c_k += vd != DP_V_BOUNDS;
     }
+    c_b += __popcll(__ballot(vp && vd == DP_V_BOUNDS));
+    c_c += __popcll(__ballot(vp && vd == DP_V_COLLIDE));
+    c_x += __popcll(__ballot(vp && vd == DP_V_CONSTRAINT));
+    c_f += __popcll(__ballot(fr));
+    c_k += __popcll(__ballot(vp && vd != DP_V_BOUNDS));
   }
-  if (k0 == 0) {
+  if (lane == 0) {
     if (c_x) atomicAdd(&s_cnt[0], (unsigned long long)c_x);
     if (c_b) atomicAdd(&s_cnt[1], (unsigned long long)c_b);
     if (c_c) atomicAdd(&s_cnt[2], (unsigned long long)c_c);
@@ -908,6 +1055,11 @@ int dp_launch_count(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     if (!c->no_events) DP_HIP_RET(hipEventRecord(ev_, s_)); \
   } while (0)
 
+// Pairs per wave of the planar check: 64 / lanes_per_pair when that is set.
+static int32_t planar_pairs_per_wave(const dp_ctx* c) {
+  return c->tiles.lanes_per_pair > 0 ? 64 / c->tiles.lanes_per_pair : 0;
+}
+
 int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   const int nx = c->desc.nx;
   const int32_t N = c->N;
@@ -959,18 +1111,15 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   a.off = c->d_off;
   a.st = c->d_st;
   a.S = c->S;
-  a.geo = c->d_geo;
-  a.nbox = c->nbox;
-  a.sweep = c->d_sweep;
-  a.srange = c->d_srange;
+  a.st4 = reinterpret_cast<const double4*>(c->d_st4);
+  a.prec = c->d_prec;
+  for (int k = 0; k < 4; ++k) a.reach[k] = c->forward ? c->reach_box[k] : c->reach_box_bwd[k];
   a.P = c->P;
   a.goalidx = c->d_goalidx;
   a.num_goal = p->num_check_goal;
   a.check_goal = p->check_intermediate_goal && p->num_check_goal > 0;
   a.obs = c->d_obs;
   a.nobs = c->nb;
-  a.node_obs = c->d_node_obs;
-  a.node_nobs = c->d_node_nobs;
   a.vis = c->d_vis_sorted;
   a.vstride = c->nv_cap;
   a.nv = c->nv;
@@ -995,7 +1144,6 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   a.surrogate = p->use_surrogate ? 1 : 0;
   a.counters = c->d_counters;
   a.backward = c->forward ? 0 : 1;
-  a.last = c->d_last;
   a.ncon = c->select_mode ? 0 : c->ncon;
   a.con = c->d_con;
   a.con_delta = (double)p->delta;
@@ -1012,37 +1160,20 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     c->timing_valid = !c->no_events && !c->defer_walk;
     return DP_OK;
   }
-  int lpp = c->tiles.lanes_per_pair > 0 ? c->tiles.lanes_per_pair
-                                       : (c->maxlen <= 16 ? 16 : (c->maxlen <= 32 ? 32 : 64));
-  // LDS: the obstacles plus one candidate list per pair group; narrow shapes
-  // widen until that fits a workgroup
-  auto lds_of = [&](int l) {
-    return sizeof(double) * 4 * c->nb + sizeof(int16_t) * (size_t)kWaves * (64 / l) * (c->nb > 0 ? c->nb : 1);
-  };
-  while (lpp < 64 && lds_of(lpp) > (size_t)DP_LDS_MAX - sizeof(dp_dev_sys)) lpp *= 2;
-  const int seg = 64 / lpp;
-  const size_t lds = lds_of(lpp);
+  a.ppw = planar_pairs_per_wave(c);
+  // LDS: the obstacles plus one list of obstacles near a node per wave
+  const size_t lds = (sizeof(double) * 4 + sizeof(int16_t) * kWaves) * (size_t)c->nb;
   // The pair count is on the device; size the grid from the bound N*P.
-  const int64_t groups = ((int64_t)N * c->P + seg - 1) / seg;
+  const int32_t least = a.ppw > 0 ? a.ppw : 4;
+  const int64_t groups = ((int64_t)N * c->P + least - 1) / least;
   const int blocks = dp_grid_blocks(groups, kWaves, c->tiles.check_blocks);
-  if (N > 0) {
-    const double* rb = c->forward ? c->reach_box : c->reach_box_bwd;
-    k_node_obs<<<dp_grid_blocks(N, kWaves, 1024), 256, 0, s>>>(c->d_nodes, c->N_cap, N, c->d_obs, c->nb, rb[0], rb[1],
-                                                              rb[2], rb[3], c->d_node_obs, c->d_node_nobs);
-    DP_HIP_RET(hipGetLastError());
-  }
   if ((rc = dp_record_event(c, 5, s))) return rc;
   rc = dispatch_nx(nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     if constexpr (NX == 13) {
       return DP_ERR_ARG;
     } else {
-      if (lpp == 2) k_check_planar<NX, 2><<<blocks, 256, lds, s>>>(a);
-      else if (lpp == 4) k_check_planar<NX, 4><<<blocks, 256, lds, s>>>(a);
-      else if (lpp == 8) k_check_planar<NX, 8><<<blocks, 256, lds, s>>>(a);
-      else if (lpp == 16) k_check_planar<NX, 16><<<blocks, 256, lds, s>>>(a);
-      else if (lpp == 32) k_check_planar<NX, 32><<<blocks, 256, lds, s>>>(a);
-      else k_check_planar<NX, 64><<<blocks, 256, lds, s>>>(a);
+      k_check_planar<NX><<<blocks, 256, lds, s>>>(a);
       return DP_OK;
     }
   });
