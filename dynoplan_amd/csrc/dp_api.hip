@@ -251,6 +251,8 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_vis_sorted);
   dev_free(&c->d_vis_cell);
   dev_free(&c->d_vis_perm);
+  dev_free(&c->d_vis_rank);
+  dev_free(&c->d_vis_count);
   dp_radius_free(c);
   dev_free(&c->d_vis_start);
   dev_free(&c->d_nodes);
@@ -269,14 +271,14 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_g);
   dev_free(&c->d_h);
   dev_free(&c->d_cont_start);
-  dev_free(&c->d_cont_cursor);
-  dev_free(&c->d_cont_idx);
+  dev_free(&c->d_cont_count);
+  dev_free(&c->d_cont_cell);
+  dev_free(&c->d_cont_item);
   dev_free(&c->d_cont_x);
   dev_free(&c->d_conf_cnt);
   dev_free(&c->d_conf);
   dev_free(&c->d_conf_ov);
   dev_free(&c->d_conf_pool);
-  dev_free(&c->d_tiles);
   dev_free(&c->d_node_cursor);
   dev_free(&c->d_node_count);
   dev_free(&c->d_chunk);
@@ -592,6 +594,7 @@ static int ensure_visited_cap(dp_ctx* c, int64_t need) {
   if ((rc = dev_alloc(&c->d_vis_sorted, (int64_t)nx * cap))) return rc;
   if ((rc = dev_alloc(&c->d_vis_cell, cap))) return rc;
   if ((rc = dev_alloc(&c->d_vis_perm, cap))) return rc;
+  if ((rc = dev_alloc(&c->d_vis_rank, cap))) return rc;
   c->nv_cap = cap;
   c->grid_dirty = true;
   return DP_OK;
@@ -657,8 +660,9 @@ int dp_reserve(dp_ctx* c, int32_t max_nodes, int64_t max_pairs) {
     if ((rc = dev_alloc(&c->d_final, (int64_t)nx * max_pairs))) return rc;
     if ((rc = dev_alloc(&c->d_g, max_pairs))) return rc;
     if ((rc = dev_alloc(&c->d_h, max_pairs))) return rc;
-    if ((rc = dev_alloc(&c->d_cont_idx, max_pairs))) return rc;
-    if ((rc = dev_alloc(&c->d_cont_x, (int64_t)nx * max_pairs))) return rc;
+    if ((rc = dev_alloc(&c->d_cont_cell, max_pairs))) return rc;
+    if ((rc = dev_alloc(&c->d_cont_item, 2 * max_pairs))) return rc;
+    if ((rc = dev_alloc(&c->d_cont_x, (int64_t)dp_cont_rec(nx) * max_pairs))) return rc;
     if ((rc = dev_alloc(&c->d_conf_cnt, max_pairs))) return rc;
     if ((rc = dev_alloc(&c->d_conf, (int64_t)DP_CONF_SLOTS * max_pairs))) return rc;
     if ((rc = dev_alloc(&c->d_conf_ov, max_pairs))) return rc;

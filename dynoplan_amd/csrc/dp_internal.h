@@ -21,9 +21,6 @@
 #define DP_PREC_LAST 21
 // Per-pair resolution value while undecided (ordered duplicate resolution).
 #define DP_R_UNDECIDED 0x7f
-// Pair flag set by the pre-resolution: every earlier contender is decided
-// and not NOVEL, so the pair is NOVEL unless its node's cap falls before it.
-#define DP_F_NUC 0x10
 // Pair flag (quadrotor): a FREE pair past its node's FP64 window; its FP64
 // rollout, final state, goal index, g and h are computed only if the node's
 // cap does not fall before it (the batch is then resolved again).
@@ -71,9 +68,11 @@ void dp_set_error(const std::string& msg);
 enum {
   DPC_PAIRS = 0, DPC_BOUNDS, DPC_COLLIDE, DPC_FREE, DPC_SURR, DPC_NOVEL, DPC_DUPV, DPC_DUPB,
   DPC_CAPPED, DPC_GOAL, DPC_CHECKED, DPC_RECHECK, DPC_ROUNDS, DPC_ERRFLAG, DPC_OVERFLOW,
-  DPC_NODES_LEFT, DPC_CONF, DPC_TICKET, DPC_CELLS, DPC_WINDOW_OVF, DPC_DEFERRED, DPC_Q64, DPC_CONSTRAINT,
+  DPC_NODES_LEFT, DPC_CONF, DPC_TICKET, DPC_SORTED, DPC_WINDOW_OVF, DPC_DEFERRED, DPC_Q64, DPC_CONSTRAINT,
   DPC_COUNT
 };
+// DPC_SORTED: contender records in cell order (low 32 bits) and conflict-wave
+// items (high 32 bits) reserved so far.
 // Sticky counters (never reset by a batch): resolutions finished by
 // host-launched rounds after a wave gave up, FP64 window overflows.
 enum { DPS_GIVEUP = 0, DPS_WINDOW = 1, DPS_COUNT = 4 };
@@ -88,7 +87,11 @@ struct dp_grid_geom {
   double inv_cell[3];
   int32_t dims[3];
   int32_t periodic2;
-  int64_t ncells;
+  // Cells of a row (axis 0) are consecutive, then one slot that stays empty:
+  // start[cell + 1] is the end of every cell, and a row's entries need not
+  // follow the previous row's (k_cell_rows gives each row its own range).
+  int32_t row;      // dims[0] + 1
+  int64_t nslots;   // row * dims[1] * dims[2]
 };
 
 __host__ __device__ inline int32_t dp_cell_axis(double x, double lo, double inv_cell, int32_t dim) {
@@ -112,7 +115,7 @@ __host__ __device__ inline void dp_cell_coords(const dp_grid_geom& G, const doub
 }
 
 __host__ __device__ inline int64_t dp_cell_linear(const dp_grid_geom& G, const int32_t* c) {
-  return ((int64_t)c[2] * G.dims[1] + c[1]) * G.dims[0] + c[0];
+  return ((int64_t)c[2] * G.dims[1] + c[1]) * G.row + c[0];
 }
 
 // Neighbour cq (0..26) of base cell c, or -1 when outside the grid (or a
@@ -130,7 +133,7 @@ __host__ __device__ inline int64_t dp_cell_neighbor(const dp_grid_geom& G, const
   } else if (n2 < 0 || n2 >= G.dims[2]) {
     return -1;
   }
-  return ((int64_t)n2 * G.dims[1] + n1) * G.dims[0] + n0;
+  return ((int64_t)n2 * G.dims[1] + n1) * G.row + n0;
 }
 
 // Learned surrogate state (k_mlp.hip).
@@ -206,7 +209,10 @@ struct dp_ctx {
   double* d_vis_sorted = nullptr;  // [nx][nv_cap] sorted by cell
   int32_t* d_vis_cell = nullptr;   // scratch [nv_cap]
   int32_t* d_vis_perm = nullptr;   // [nv_cap] position in d_vis_sorted -> append index
-  int32_t* d_vis_start = nullptr;  // [ncells+1]
+  int32_t* d_vis_rank = nullptr;   // scratch [nv_cap]
+  int32_t* d_vis_count = nullptr;  // scratch [nslots]
+  int64_t vis_count_cap = 0;
+  int32_t* d_vis_start = nullptr;  // [nslots]
   int64_t vis_cells_cap = 0;
   bool grid_dirty = true;
   dp_grid_geom grid{};
@@ -234,20 +240,20 @@ struct dp_ctx {
   double* d_h = nullptr;
 
   // contender grid (batch duplicates)
-  int32_t* d_cont_start = nullptr;  // [ncells+1]
-  int32_t* d_cont_cursor = nullptr; // [ncells]
-  int32_t* d_cont_idx = nullptr;    // [pair_cap]
-  int64_t cont_start_cap = 0, cont_cursor_cap = 0;
+  int32_t* d_cont_count = nullptr;  // [nslots] contenders per cell (-1: one, alone in its 27-cell block)
+  int32_t* d_cont_start = nullptr;  // [nslots] first record of each cell
+  int64_t cont_count_cap = 0, cont_start_cap = 0;
+  int32_t* d_cont_cell = nullptr;   // [pair_cap] grid cell of each contender
+  int32_t* d_cont_item = nullptr;   // [2 * pair_cap] conflict-wave items
   int32_t* d_node_novel = nullptr;  // [N_cap+1] NOVEL pairs per node, then offsets
-  double* d_cont_x = nullptr;       // [nx][pair_cap] contender final states sorted by cell
+  double* d_cont_x = nullptr;       // [pair_cap][dp_cont_rec(nx)] contender records, by cell
   int16_t* d_conf_cnt = nullptr;    // [pair_cap] stored earlier conflicts per pair (-1: scan)
   int32_t* d_conf = nullptr;        // [pair_cap][DP_CONF_SLOTS] earlier conflicting contenders
-  int32_t* d_conf_ov = nullptr;     // [pair_cap] offset of entries DP_CONF_SLOTS.. in the overflow pool
+  int32_t* d_conf_ov = nullptr;     // [pair_cap] place in the cell (until the scatter), then the offset of entries
+                                    // DP_CONF_SLOTS.. in the overflow pool
   int32_t* d_conf_pool = nullptr;   // [pool_cap] overflow entries (bump-allocated per batch)
   int64_t conf_pool_cap = 0;
   double round_r_dup = 0.0;         // duplicate radius of the batch in flight
-  int32_t* d_tiles = nullptr;       // [tiles+1] partial sums of the large scan
-  int64_t tiles_cap = 0;
   int32_t* d_node_cursor = nullptr; // [N_cap] first undecided pair per node
   int32_t* d_node_count = nullptr;  // [N_cap] NOVEL pairs decided per node
   long long* h_pinned = nullptr;    // pinned host words for device totals
@@ -350,22 +356,38 @@ int dp_ensure_u64(uint64_t** p, int64_t* cap, int64_t need);
 
 // ---- k_util.hip ---------------------------------------------------------
 void dp_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
-void dp_zero_counters(long long* c, hipStream_t s);
+// Clears the batch counters, a[0..na) and b[0..nb) in one launch.
+void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t nb, hipStream_t s);
 // Exclusive scan of data[0..n-1] into data[0..n]; data[n] = total.  Small n
 // (one workgroup).  total (optional) receives min(total, cap); counters[slot]
 // receives the total when slot >= 0.
 void dp_scan_small(int32_t* data, int64_t n, int32_t* total, int64_t cap, long long* counters, int slot,
                    hipStream_t s);
-// Same for large arrays: three passes over tiles of 4096 elements.  The
-// length is *n_dev (at most n_max) when n_dev is set, else n_max.
-int dp_scan_large(dp_ctx* c, int32_t* data, const int32_t* n_dev, int64_t n_max, long long* counters, int slot,
-                  hipStream_t s);
-
 // ---- k_grid.hip ---------------------------------------------------------
 dp_grid_geom dp_make_grid(const dp_ctx* c, double r);
 int dp_launch_visited_rebuild(dp_ctx* c, double radius, hipStream_t s);
 int dp_launch_visited_append_novel(dp_ctx* c, int64_t novel_total, hipStream_t s);
-int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, hipStream_t s);
+// counted: the check stage has counted the contenders into their cells (else
+// they are counted here).
+int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool counted, hipStream_t s);
+// Contender grid buffers for the current geometry (before the check stage).
+int dp_ensure_cont_grid(dp_ctx* c);
+// Doubles of a contender record: the state, its pair index (int32, bit 31:
+// it needs no list of its own), padded to 16 bytes.
+__host__ __device__ constexpr int dp_cont_rec(int nx) { return (nx + 2) / 2 * 2; }
+#define DP_CONT_NOLIST 0x80000000u
+
+// The pair counted into its cell of the contender grid (final state x); its
+// place in the cell is kept for the scatter.
+__device__ __forceinline__ void dp_count_contender(const dp_grid_geom& G, const double* x, int64_t q,
+                                                   int32_t* count, int32_t* cell_of, int32_t* place) {
+  int32_t c[3];
+  dp_cell_coords(G, x, c);
+  const int32_t cell = (int32_t)dp_cell_linear(G, c);
+  cell_of[q] = cell;
+  place[q] = atomicAdd(&count[cell], 1);
+}
+
 int dp_launch_more_rounds(dp_ctx* c, int rounds, hipStream_t s);
 // Resolution from scratch after a window overflow: every FREE pair
 // undecided again, resolution counters cleared, lists and walk rebuilt.
@@ -388,7 +410,8 @@ int dp_noalloc_init_device(int device);
 void dp_radius_free(dp_ctx* c);
 
 // ---- k_quad.hip ---------------------------------------------------------
-int dp_launch_quad(dp_ctx* c, const dp_expand_params* p, double goal_bound, double r_dup, hipStream_t s);
+// count: contenders are counted into their grid cells.
+int dp_launch_quad(dp_ctx* c, const dp_expand_params* p, double goal_bound, double r_dup, bool count, hipStream_t s);
 // FP64 rollout of the pairs deferred past their node's FP64 window (after a
 // window overflow), then their visited-set duplicate test.
 int dp_launch_quad_deferred(dp_ctx* c, hipStream_t s);
@@ -440,7 +463,7 @@ __device__ __forceinline__ bool dp_grid_run_any(const dp_dev_sys& S, const dp_gr
   } else if (n2 < 0 || n2 >= G.dims[2]) {
     return false;
   }
-  const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.dims[0];
+  const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.row;
   const int32_t x0 = c[0] > 0 ? c[0] - 1 : 0, x1 = c[0] + 1 < G.dims[0] ? c[0] + 1 : G.dims[0] - 1;
   const int32_t e = start[row + x1 + 1];
   for (int32_t p = start[row + x0]; p < e; ++p)

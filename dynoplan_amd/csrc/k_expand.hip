@@ -384,6 +384,11 @@ struct dp_check_args {
   double con_delta;
   // dbrrt selection: no goal check or duplicate test, resolution DP_R_NONE
   int32_t select;
+  // contender grid: cell counts, and each contender's cell and place in it
+  // (count null: not counted here)
+  int32_t* cont_count;
+  int32_t* cont_cell;
+  int32_t* cont_place;
 };
 
 namespace {
@@ -775,7 +780,7 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
           } else {
             ok = ok && n2 >= 0 && n2 < G.dims[2];
           }
-          const int64_t row = ok ? ((int64_t)n2 * G.dims[1] + n1) * G.dims[0] : 0;
+          const int64_t row = ok ? ((int64_t)n2 * G.dims[1] + n1) * G.row : 0;
           rb[k] = a.vstart[ok ? row + x0 : 0];
           rn[k] = a.vstart[ok ? row + x1 + 1 : 0];
         }
@@ -832,6 +837,8 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
         for (int c = 0; c < NX; ++c) a.fin[(int64_t)c * a.pcap + q] = xf[c];
         a.gout[q] = gq;
         a.hout[q] = hq;
+        if (a.cont_count && (chosen != -1 || !dupv))
+          dp_count_contender(a.grid, xf, q, a.cont_count, a.cont_cell, a.cont_place);
       }
     }
     c_b += __popcll(__ballot(vp && vd == DP_V_BOUNDS));
@@ -984,7 +991,7 @@ static app_bounds make_app_bounds(const dp_ctx* c, double r) {
   return B;
 }
 
-// Applicability masks and counts of the uploaded nodes (app cleared here).
+// Applicability masks and counts of the uploaded nodes (app is clear).
 template <int NX>
 static void launch_app(dp_ctx* c, const app_bounds& B, double r_app, hipStream_t s);
 
@@ -1022,7 +1029,6 @@ static bool app_per_node_order(const dp_ctx* c) { return c->d_order && c->order_
 template <int NX>
 static void launch_app(dp_ctx* c, const app_bounds& B, double r_app, hipStream_t s) {
   const int32_t N = c->N;
-  dp_fill_i32(c->d_app, N, 0, s);
   const double* keys = c->forward ? c->d_start : c->d_last;
   if (app_per_node_order(c)) {  // a pair order per node: one wave per node part
     k_app_count<NX><<<N * kAppParts, 64, 0, s>>>(c->d_sys, B, c->d_nodes, c->N_cap, N, keys, c->P, r_app, c->d_order,
@@ -1040,6 +1046,7 @@ int dp_launch_count(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   const double r_app = app_radius(c, p);
   const int32_t N = c->N;
   const app_bounds B = make_app_bounds(c, r_app);
+  dp_fill_i32(c->d_app, N, 0, s);
   return dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     launch_app<NX>(c, B, r_app, s);
@@ -1072,10 +1079,16 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     if (rc) return rc;
   }
 
+  // The check stage counts the contenders into their grid cells as it finds
+  // them; limit 0 takes pairs out again after it (k_precap_first), so there
+  // they are counted later.
+  const bool count = !c->select_mode && p->limit_branching_factor != 0;
+  int rc = c->select_mode ? DP_OK : dp_ensure_cont_grid(c);
+  if (rc) return rc;
   DP_EV(c->ev[0], s);
-  dp_zero_counters(c->d_counters, s);
+  dp_begin(c->d_counters, c->d_app, N, c->d_cont_count, count ? c->grid.nslots : 0, s);
   const app_bounds B = make_app_bounds(c, r_app);
-  int rc = dispatch_nx(nx, [&](auto NXc) -> int {
+  rc = dispatch_nx(nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     launch_app<NX>(c, B, r_app, s);
     dp_scan_small(c->d_app, N, c->d_total, c->pair_cap, c->d_counters, DPC_PAIRS, s);
@@ -1149,12 +1162,15 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   a.con_delta = (double)p->delta;
   a.select = c->select_mode ? 1 : 0;
   if (c->select_mode) a.nv = 0;
+  a.cont_count = count ? c->d_cont_count : nullptr;
+  a.cont_cell = c->d_cont_cell;
+  a.cont_place = c->d_conf_ov;
 
   if (c->desc.system == DP_SYS_QUADROTOR) {
-    rc = dp_launch_quad(c, p, goal_bound, r_dup, s);
+    rc = dp_launch_quad(c, p, goal_bound, r_dup, count, s);
     if (rc) return rc;
     DP_EV(c->ev[2], s);
-    rc = dp_launch_resolve(c, p, r_dup, s);
+    rc = dp_launch_resolve(c, p, r_dup, count, s);
     if (rc) return rc;
     DP_EV(c->ev[3], s);
     c->timing_valid = !c->no_events && !c->defer_walk;
@@ -1200,7 +1216,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     c->timing_valid = !c->no_events && !c->defer_walk;
     return DP_OK;
   }
-  rc = dp_launch_resolve(c, p, r_dup, s);
+  rc = dp_launch_resolve(c, p, r_dup, count, s);
   if (rc) return rc;
   DP_EV(c->ev[3], s);
   c->timing_valid = !c->no_events && !c->defer_walk;

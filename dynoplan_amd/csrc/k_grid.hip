@@ -65,7 +65,8 @@ dp_grid_geom dp_make_grid(const dp_ctx* c, double r) {
       n *= nth;
     }
     if (n <= max_cells) {
-      G.ncells = (int64_t)G.dims[0] * G.dims[1] * G.dims[2];
+      G.row = G.dims[0] + 1;
+      G.nslots = (int64_t)G.row * G.dims[1] * G.dims[2];
       break;
     }
     cell *= 1.5;  // coarser cells stay exact, only slower
@@ -87,24 +88,168 @@ __device__ __forceinline__ int64_t cell_of_soa(const dp_grid_geom& G, const doub
   return dp_cell_linear(G, c);
 }
 
+// ---- cells --------------------------------------------------------------
+// Contenders of one cell that one wave of k_conf_waves takes.  A wave's
+// serial work is its contenders times the candidate batches of the block
+// (K / batch), so the contenders of a crowded block are split over several
+// waves, about 16 contender-batches each.
+__device__ __forceinline__ int32_t cell_part_size(int32_t K, int32_t batch) {
+  const int32_t nb = (K + batch - 1) / batch;
+  const int32_t per = nb > 0 ? 16 / nb : 64;
+  return per < 1 ? 1 : (per > 64 ? 64 : per);
+}
+
+// Cell counts to cell starts, one wave per grid row.  The entries of a row
+// are consecutive (a 27-cell block reads runs of three cells of one row);
+// the rows themselves lie in any order, so a row needs only its own sum and
+// one reserved range instead of a scan of the whole grid (three launches over
+// 0.4M cells: 18 us, and 29 to 45 us more for the list of cells).  What
+// bounds it are the atomics that reserve the ranges, all on one address at
+// about 15 ns each: 16 rows share one, which returns both the records' and
+// the items' range (packed in 64 bits).  2.7k rows 15 us, 4.1k rows 16 us;
+// with two atomics per four rows 26 and 35 us.
+//
+// kItems (contender grid): also the work items of k_conf_waves.  A cell's
+// 27-cell count is the sum of three column sums of its nine rows, formed
+// from coalesced loads of the counts, 62 cells at a time (a lane on each
+// side holds the neighbours' columns).  A contender alone in its block has
+// no conflict: its cell gets no entry, and count -1 tells the scatter.  An
+// item is int2(cell | (contenders - 1) << 26, first record).
+constexpr int kRowWaves = 16;  // rows per workgroup
+
+template <bool kItems>
+__global__ __launch_bounds__(64 * kRowWaves) void k_cell_rows(dp_grid_geom G, int32_t* __restrict__ count,
+                                                   int32_t* __restrict__ start, int32_t batch, int2* __restrict__ items,
+                                                   long long* __restrict__ counters) {
+  __shared__ int32_t s_sum[kRowWaves], s_items[kRowWaves];
+  __shared__ unsigned long long s_base;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int32_t rows = G.dims[1] * G.dims[2];
+  const int32_t r = blockIdx.x * kRowWaves + wave;
+  const int32_t n1 = r < rows ? r % G.dims[1] : 0, n2 = r < rows ? r / G.dims[1] : 0;
+  const int64_t base = (int64_t)r * G.row;
+  const int32_t d0 = r < rows ? G.dims[0] : 0;
+  // cells x0 .. x0 + 61 on lanes 1 .. 62
+  auto block_count = [&](int32_t x0, int32_t own) -> int32_t {
+    int32_t col = own;
+    const int32_t x = x0 - 1 + lane;
+    const bool in = x >= 0 && x < d0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      if (k == 4) continue;
+      const int32_t m1 = n1 + k % 3 - 1, e2 = k / 3 - 1;
+      int32_t m2 = n2 + e2;
+      bool ok = in && m1 >= 0 && m1 < G.dims[1];
+      if (G.dims[2] == 1) {
+        ok = ok && e2 == 0;
+        m2 = 0;
+      } else if (G.periodic2) {
+        m2 = m2 < 0 ? m2 + G.dims[2] : (m2 >= G.dims[2] ? m2 - G.dims[2] : m2);
+      } else {
+        ok = ok && m2 >= 0 && m2 < G.dims[2];
+      }
+      const int32_t v = count[ok ? ((int64_t)m2 * G.dims[1] + m1) * G.row + x : 0];
+      col += ok ? v : 0;
+    }
+    return __shfl_up(col, 1, 64) + col + __shfl_down(col, 1, 64);
+  };
+  int32_t sum = 0, nit = 0;
+  for (int32_t x0 = 0; x0 < d0; x0 += 62) {
+    const int32_t x = x0 - 1 + lane;
+    const int32_t own = x >= 0 && x < d0 ? count[base + x] : 0;
+    const bool mine = lane >= 1 && lane <= 62 && own > 0;
+    if (!__ballot(mine)) continue;
+    int32_t n = mine ? own : 0;
+    if constexpr (kItems) {
+      const int32_t K = block_count(x0, own);
+      if (n == 1 && K == 1) n = 0;
+      if (n > 0) {
+        const int32_t per = cell_part_size(K, batch);
+        nit += (n + per - 1) / per;
+      }
+    }
+    sum += n;
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    sum += __shfl_xor(sum, d, 64);
+    nit += __shfl_xor(nit, d, 64);
+  }
+  if (lane == 0) {
+    s_sum[wave] = sum;
+    s_items[wave] = nit;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int k = 0; k < kRowWaves; ++k) t += (unsigned long long)s_sum[k] | ((unsigned long long)s_items[k] << 32);
+    s_base = t ? atomicAdd((unsigned long long*)&counters[DPC_SORTED], t) : 0ull;
+  }
+  __syncthreads();
+  if (d0 == 0) return;
+  int32_t at = (int32_t)(uint32_t)s_base, it = (int32_t)(s_base >> 32);
+  for (int k = 0; k < wave; ++k) {
+    at += s_sum[k];
+    it += s_items[k];
+  }
+  for (int32_t x0 = 0; x0 < d0; x0 += 62) {
+    const int32_t x = x0 - 1 + lane;
+    const int32_t own = x >= 0 && x < d0 ? count[base + x] : 0;
+    const bool mine = lane >= 1 && lane <= 62 && x < d0;
+    int32_t n = mine ? own : 0;
+    int32_t parts = 0, per = 1;
+    if constexpr (kItems) {
+      if (__ballot(n > 0)) {
+        const int32_t K = block_count(x0, own);
+        if (n == 1 && K == 1) {
+          n = 0;
+          count[base + x] = -1;
+        }
+        if (n > 0) {
+          per = cell_part_size(K, batch);
+          parts = (n + per - 1) / per;
+        }
+      }
+    }
+    int32_t incl = n, iinc = parts;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t u = __shfl_up(incl, d, 64), v = __shfl_up(iinc, d, 64);
+      if (lane >= d) {
+        incl += u;
+        iinc += v;
+      }
+    }
+    const int32_t b = at + incl - n;
+    if (mine) start[base + x] = b;
+    if constexpr (kItems)
+      for (int32_t k = 0; k < parts; ++k) {
+        const int32_t g0 = k * per, m = n - g0 < per ? n - g0 : per;
+        items[it + (iinc - parts) + k] = make_int2((int32_t)((uint32_t)(base + x) | ((uint32_t)(m - 1) << 26)), b + g0);
+      }
+    at += __shfl(incl, 63, 64);
+    it += __shfl(iinc, 63, 64);
+  }
+  if (lane == 0) start[base + d0] = at;  // the end of the row's last cell
+}
+
 // ---- visited set ---------------------------------------------------------
 template <int NX>
 __global__ void k_vis_count(dp_grid_geom G, const double* __restrict__ pts, int64_t stride, int64_t n,
-                            int32_t* __restrict__ cellof, int32_t* __restrict__ counts) {
+                            int32_t* __restrict__ cellof, int32_t* __restrict__ rank, int32_t* __restrict__ counts) {
   for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = cell_of_soa<NX>(G, pts, stride, p);
     cellof[p] = (int32_t)c;
-    atomicAdd(&counts[c], 1);
+    rank[p] = atomicAdd(&counts[c], 1);
   }
 }
 
 template <int NX>
 __global__ void k_vis_scatter(const double* __restrict__ pts, int64_t stride, int64_t n,
-                              const int32_t* __restrict__ cellof, const int32_t* __restrict__ start,
-                              int32_t* __restrict__ cursor, double* __restrict__ out, int32_t* __restrict__ perm) {
+                              const int32_t* __restrict__ cellof, const int32_t* __restrict__ rank,
+                              const int32_t* __restrict__ start, double* __restrict__ out, int32_t* __restrict__ perm) {
   for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t c = cellof[p];
-    const int32_t pos = start[c] + atomicAdd(&cursor[c], 1);
+    const int32_t pos = start[cellof[p]] + rank[p];
 #pragma unroll
     for (int k = 0; k < NX; ++k) out[(int64_t)k * stride + pos] = pts[(int64_t)k * stride + p];
     perm[pos] = (int32_t)p;
@@ -116,31 +261,146 @@ __device__ __forceinline__ bool is_contender(int8_t verdict, int8_t flags) {
   return verdict == DP_V_FREE && !(flags & (DP_F_DEFER | DP_F_PRECAP)) && ((flags & 2) || !(flags & 1));
 }
 
+// The contenders counted into their cells, where the check stage has not
+// done it (limit 0, a batch resolved again).
 template <int NX>
 __global__ void k_cont_count(dp_grid_geom G, const int32_t* __restrict__ total, const int8_t* __restrict__ verdict,
                              const int8_t* __restrict__ flags, const double* __restrict__ fin, int64_t pcap,
-                             int32_t* __restrict__ counts) {
+                             int32_t* __restrict__ counts, int32_t* __restrict__ cell_of, int32_t* __restrict__ place) {
   const int64_t n = *total;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
     if (!is_contender(verdict[q], flags[q])) continue;
-    atomicAdd(&counts[cell_of_soa<NX>(G, fin, pcap, q)], 1);
+    const double x[3] = {fin[q], fin[pcap + q], fin[2 * pcap + q]};
+    dp_count_contender(G, x, q, counts, cell_of, place);
   }
 }
 
+// The contender record of pair p.
 template <int NX>
-__global__ void k_cont_scatter(dp_grid_geom G, const int32_t* __restrict__ total, const int8_t* __restrict__ verdict,
-                               const int8_t* __restrict__ flags, const double* __restrict__ fin, int64_t pcap,
-                               const int32_t* __restrict__ start, int32_t* __restrict__ cursor,
-                               int32_t* __restrict__ idx, double* __restrict__ xs) {
-  const int64_t n = *total;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-    if (!is_contender(verdict[q], flags[q])) continue;
-    const int64_t c = cell_of_soa<NX>(G, fin, pcap, q);
-    const int32_t pos = start[c] + atomicAdd(&cursor[c], 1);
-    idx[pos] = (int32_t)q;
+__device__ __forceinline__ void put_record(const double* fin, int64_t pcap, int32_t p, bool nolist, double* rec) {
+  constexpr int kRec = dp_cont_rec(NX);
+  double y[kRec];
 #pragma unroll
-    for (int k = 0; k < NX; ++k) xs[(int64_t)k * pcap + pos] = fin[(int64_t)k * pcap + q];
+  for (int k = 0; k < NX; ++k) y[k] = fin[(int64_t)k * pcap + p];
+  y[NX] = __longlong_as_double((long long)((uint32_t)p | (nolist ? DP_CONT_NOLIST : 0u)));
+  if constexpr (kRec > NX + 1) y[NX + 1] = 0.0;
+  double2* dst = reinterpret_cast<double2*>(rec);
+#pragma unroll
+  for (int k = 0; k < kRec / 2; ++k) dst[k] = make_double2(y[2 * k], y[2 * k + 1]);
+}
+
+// Contender records into cell order, and the list window (planar systems,
+// limit > 0, window > 0): the contenders of a node after its first W in
+// canonical order are flagged DP_F_NOLIST, and their list length is set to
+// -(1 + rank) (rank among the node's contenders, at most 32766).  The walk
+// reaches one of them only if more than W - limit contenders before it were
+// duplicates; it then records 1 + rank in need[0], and later batches of the
+// context use W = max(window, need + need / 4 + 16) (a fixed window leaves
+// need alone: need == null).
+//
+// One wave per node, four nodes per workgroup, four chunks of 64 pairs per
+// step with their loads issued together (indices clamped into the node).
+// The place in the cell is known from the count, so nothing is counted
+// again; a record is one 32 to 112 byte piece (state, pair index), where
+// separate arrays wrote NX + 1 scattered words.  Bound by those scattered
+// writes: 1.5M planar contenders 32 us, where the window, a separate count
+// and a scatter with cursors took 8 + 34 + 45.
+template <int NX>
+__global__ __launch_bounds__(256) void k_cont_scatter(int32_t N, const int32_t* __restrict__ app,
+                                                      const int32_t* __restrict__ total,
+                                                      const int8_t* __restrict__ verdict, int8_t* __restrict__ flags,
+                                                      const double* __restrict__ fin, int64_t pcap,
+                                                      const int32_t* __restrict__ count,
+                                                      const int32_t* __restrict__ start,
+                                                      const int32_t* __restrict__ cell_of,
+                                                      const int32_t* __restrict__ place, int32_t window,
+                                                      const int32_t* __restrict__ need, int16_t* __restrict__ conf_cnt,
+                                                      double* __restrict__ rec) {
+  const int32_t node = blockIdx.x * 4 + (int32_t)(threadIdx.x / 64);
+  if (node >= N) return;
+  const int lane = threadIdx.x % 64;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  if (window > 0 && need) {
+    const int32_t nd = need[0];
+    const int64_t w = (int64_t)nd + nd / 4 + 16;
+    if (nd > 0 && w > window) window = w < INT32_MAX ? (int32_t)w : INT32_MAX;
   }
+  const int32_t tot = *total;
+  const int32_t b = app[node] < tot ? app[node] : tot;
+  const int32_t e = app[node + 1] < tot ? app[node + 1] : tot;
+  int32_t rank = 0;
+  constexpr int kPre = 4;
+  constexpr int kRec = dp_cont_rec(NX);
+  for (int32_t c0 = b; c0 < e; c0 += 64 * kPre) {
+    int8_t v_u[kPre], f_u[kPre];
+    int32_t cell_u[kPre], pl_u[kPre];
+#pragma unroll
+    for (int u = 0; u < kPre; ++u) {
+      const int32_t p = c0 + 64 * u + lane < e ? c0 + 64 * u + lane : e - 1;
+      v_u[u] = verdict[p];
+      f_u[u] = flags[p];
+      cell_u[u] = cell_of[p];
+      pl_u[u] = place[p];
+    }
+#pragma unroll
+    for (int u = 0; u < kPre; ++u) {
+      const int32_t p = c0 + 64 * u + lane;
+      const int8_t fl = f_u[u];
+      const bool con = p < e && is_contender(v_u[u], fl);
+      const uint64_t m = __ballot(con);
+      const int32_t r = rank + __popcll(m & lt);
+      rank += __popcll(m);
+      if (!con) continue;
+      bool nolist = (fl & 2) != 0;  // goal-forced: NOVEL without a list
+      if (window > 0 && r >= window) {
+        flags[p] = (int8_t)(fl | DP_F_NOLIST);
+        conf_cnt[p] = (int16_t)(-1 - (r < 32766 ? r : 32766));
+        nolist = true;
+      }
+      const int32_t cell = cell_u[u];
+      if (count[cell] < 0) {  // alone in its 27-cell block: no earlier contender
+        if (!nolist) conf_cnt[p] = 0;
+        continue;
+      }
+      put_record<NX>(fin, pcap, p, nolist, rec + (int64_t)(start[cell] + pl_u[u]) * kRec);
+    }
+  }
+}
+
+// The same without a window, over a list of pairs that holds every contender
+// (the quadrotor's FP64 pairs: 46k of 1.13M in a batch of 2048 nodes), one
+// thread per listed pair.  Walking all pairs of the nodes to find them took
+// 22 us, this 12 (a chain of five dependent loads per pair).
+template <int NX>
+__global__ __launch_bounds__(256) void k_cont_scatter_list(const int32_t* __restrict__ list,
+                                                           const long long* __restrict__ n_list,
+                                                           const int8_t* __restrict__ verdict,
+                                                           const int8_t* __restrict__ flags,
+                                                           const double* __restrict__ fin, int64_t pcap,
+                                                           const int32_t* __restrict__ count,
+                                                           const int32_t* __restrict__ start,
+                                                           const int32_t* __restrict__ cell_of,
+                                                           const int32_t* __restrict__ place,
+                                                           int16_t* __restrict__ conf_cnt, double* __restrict__ rec) {
+  constexpr int kRec = dp_cont_rec(NX);
+  const int64_t n = *n_list;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t p = list[t];
+    const int8_t fl = flags[p];
+    if (!is_contender(verdict[p], fl)) continue;
+    const int32_t cell = cell_of[p];
+    if (count[cell] < 0) {
+      if (!(fl & 2)) conf_cnt[p] = 0;
+      continue;
+    }
+    put_record<NX>(fin, pcap, p, (fl & 2) != 0, rec + (int64_t)(start[cell] + place[p]) * kRec);
+  }
+}
+
+// Pair index of a contender record (without the no-list bit).
+template <int NX>
+__device__ __forceinline__ uint32_t rec_word(const double* rec, int64_t t) {
+  return (uint32_t)__double_as_longlong(rec[t * dp_cont_rec(NX) + NX]);
 }
 
 // Earlier contenders of pair q within r: scans the 27 cells around x.
@@ -149,8 +409,8 @@ __global__ void k_cont_scatter(dp_grid_geom G, const int32_t* __restrict__ total
 // Candidates are taken eight at a time so that their loads overlap.
 template <int NX, typename F, typename Keep>
 __device__ __forceinline__ void scan_earlier(const dp_dev_sys& S, const dp_grid_geom& G, const int32_t* cstart,
-                                             const int32_t* cidx, const double* cx, int64_t pcap, const double* x,
-                                             int64_t q, double r, F&& f, Keep&& keep) {
+                                             const double* cx, const double* x, int64_t q, double r, F&& f,
+                                             Keep&& keep) {
   int32_t c[3];
   dp_cell_coords(G, x, c);
   const double T = dp_pos_bound(S, r);
@@ -161,14 +421,16 @@ __device__ __forceinline__ void scan_earlier(const dp_dev_sys& S, const dp_grid_
     for (int32_t t0 = cstart[cell]; t0 < e; t0 += 8) {
       int32_t o[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o[k] = t0 + k < e ? cidx[t0 + k] : INT32_MAX;
+      for (int k = 0; k < 8; ++k)
+        o[k] = t0 + k < e ? (int32_t)(rec_word<NX>(cx, t0 + k) & ~DP_CONT_NOLIST) : INT32_MAX;
       uint32_t km = 0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) km |= (o[k] < q && keep(o[k]) ? 1u : 0u) << k;
       for (; km; km &= km - 1u) {
         const int32_t t = t0 + __ffs(km) - 1;
-        if (!dp_within_col_pf<NX>(S, x, cx, pcap, t, r, T)) continue;
-        if (!f(cidx[t])) return;
+        // a record's components are consecutive: stride 1 from its first
+        if (!dp_within_col_pf<NX>(S, x, cx + (int64_t)t * dp_cont_rec(NX), 1, 0, r, T)) continue;
+        if (!f((int32_t)(rec_word<NX>(cx, t) & ~DP_CONT_NOLIST))) return;
       }
     }
   }
@@ -183,113 +445,6 @@ __device__ __forceinline__ void scan_earlier(const dp_dev_sys& S, const dp_grid_
 // pool ran out), for which the resolution scans the grid.  The order of a
 // list's entries carries no meaning.
 
-// Contenders of one cell that one wave of k_conf_waves takes.  A wave's
-// serial work is its contenders times the candidate batches of the block
-// (K / batch), so the contenders of a crowded block are split over several
-// waves, about 16 contender-batches each, in at most 255 parts.
-__device__ __forceinline__ int32_t cell_part_size(int32_t m, int32_t K, int32_t batch) {
-  const int32_t nb = (K + batch - 1) / batch;
-  int32_t per = nb > 0 ? 16 / nb : 64;
-  per = per < 1 ? 1 : (per > 64 ? 64 : per);
-  const int32_t least = (m + 254) / 255;
-  return per < least ? least : per;
-}
-
-// Contenders in the 27-cell block around `cell` (the runs k_conf_waves
-// reads, with the same neighbour rules).
-__device__ __forceinline__ int32_t cell_block_count(const dp_grid_geom& G, const int32_t* __restrict__ cstart,
-                                                    int64_t cell) {
-  const int64_t d01 = (int64_t)G.dims[0] * G.dims[1];
-  const int32_t c0 = (int32_t)(cell % G.dims[0]), c1 = (int32_t)((cell / G.dims[0]) % G.dims[1]);
-  const int32_t c2 = (int32_t)(cell / d01);
-  const int32_t x0 = c0 > 0 ? c0 - 1 : 0, x1 = c0 + 1 < G.dims[0] ? c0 + 1 : G.dims[0] - 1;
-  int32_t K = 0;
-  for (int k = 0; k < 9; ++k) {
-    const int32_t n1 = c1 + k % 3 - 1;
-    const int32_t d2 = k / 3 - 1;
-    int32_t n2 = c2 + d2;
-    bool ok = n1 >= 0 && n1 < G.dims[1];
-    if (G.dims[2] == 1) {
-      ok = ok && d2 == 0;
-      n2 = 0;
-    } else if (G.periodic2) {
-      n2 = n2 < 0 ? n2 + G.dims[2] : (n2 >= G.dims[2] ? n2 - G.dims[2] : n2);
-    } else {
-      ok = ok && n2 >= 0 && n2 < G.dims[2];
-    }
-    if (ok) {
-      const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.dims[0];
-      K += cstart[row + x1 + 1] - cstart[row + x0];
-    }
-  }
-  return K;
-}
-
-// The non-empty cells of the contender grid, one thread per cell: each
-// workgroup reserves room for its listed cells with one global atomic
-// (cells are listed in no particular order).  A cell whose 27-cell
-// block holds its one contender only is settled here (no earlier
-// contender can conflict: an empty list, and NUC unless goal-forced) and is
-// not listed, when no window applies.
-__global__ __launch_bounds__(256) void k_cell_list(int64_t ncells, dp_grid_geom G, const int32_t* __restrict__ cstart,
-                                                   const int32_t* __restrict__ cidx, int32_t window, int32_t batch,
-                                                   int8_t* __restrict__ flags, int16_t* __restrict__ conf_cnt,
-                                                   int32_t* __restrict__ list, long long* __restrict__ counters) {
-  __shared__ int32_t s_cnt;
-  __shared__ long long s_base;
-  const int lane = threadIdx.x % 64;
-  // one cell per thread (the grid covers every cell)
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int kind = 0;  // 0: empty or no list needed, 1: listed, 2: settled here
-  int32_t parts = 0;
-  if (c < ncells) {
-    const int32_t b = cstart[c], e = cstart[c + 1];
-    const int32_t K = e > b ? cell_block_count(G, cstart, c) : 0;
-    if (e > b) kind = e - b != 1 || K != 1 ? 1 : 2;
-    if (kind == 1 && window > 0) {
-      // a cell whose contenders are all goal-forced or past their node's
-      // list window needs no wave; the latter are scanned when reached
-      bool any = false;
-      for (int32_t k = b; k < e && !any; ++k) {
-        const int8_t fl = flags[cidx[k]];
-        any = !(fl & 2) && !(fl & DP_F_NOLIST);
-      }
-      if (!any) kind = 0;
-    }
-    if (kind == 1) {
-      const int32_t per = cell_part_size(e - b, K, batch);
-      parts = (e - b + per - 1) / per;
-    }
-    if (kind == 2) {
-      const int32_t q = cidx[b];
-      const int8_t fl = flags[q];
-      if (!(fl & 2)) {  // goal-forced pairs are NOVEL without a list
-        conf_cnt[q] = 0;
-        flags[q] = (int8_t)(fl | DP_F_NUC);
-      }
-    }
-  }
-  if (threadIdx.x == 0) s_cnt = 0;
-  __syncthreads();
-  // items: cell | part << 24 (a grid has at most 2^24 cells)
-  int incl = parts;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int v = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += v;
-  }
-  const int wtot = __shfl(incl, 63, 64);
-  int woff = 0;
-  if (lane == 0 && wtot) woff = atomicAdd(&s_cnt, wtot);
-  __syncthreads();
-  if (threadIdx.x == 0)
-    s_base = s_cnt ? (long long)atomicAdd((unsigned long long*)&counters[DPC_CELLS], (unsigned long long)s_cnt) : 0;
-  __syncthreads();
-  woff = __shfl(woff, 0, 64);
-  for (int32_t k = 0; k < parts; ++k)
-    list[s_base + woff + (incl - parts) + k] = (int32_t)((uint32_t)c | ((uint32_t)k << 24));
-}
-
 // One wave per non-empty grid cell: the 27 cells around it
 // form 9 runs of 3 cells consecutive in memory (x is the fastest grid
 // dimension).  For each of the cell's contenders in turn, the lanes read the
@@ -298,26 +453,34 @@ __global__ __launch_bounds__(256) void k_cell_list(int64_t ncells, dp_grid_geom 
 // compaction into the list.  No LDS and no barriers, so many cells are in
 // flight per CU.
 template <int NX>
+__device__ __forceinline__ void load_rec(const double* cx, int64_t t, double* y) {
+  const double2* src = reinterpret_cast<const double2*>(cx + t * dp_cont_rec(NX));
+#pragma unroll
+  for (int k = 0; k < dp_cont_rec(NX) / 2; ++k) {
+    const double2 v = src[k];
+    y[2 * k] = v.x;
+    y[2 * k + 1] = v.y;
+  }
+}
+
+template <int NX>
 __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict__ Sp, dp_grid_geom G,
-                                                    int8_t* __restrict__ flags,
-                                                    const int32_t* __restrict__ pnode,
-                                                    const int32_t* __restrict__ app, int32_t window, int64_t pcap,
                                                     const int32_t* __restrict__ cstart,
-                                                    const int32_t* __restrict__ cidx, const double* __restrict__ cx,
-                                                    const int32_t* __restrict__ cells, double r,
+                                                    const double* __restrict__ cx, const int2* __restrict__ items,
+                                                    double r,
                                                     int16_t* __restrict__ conf_cnt, int32_t* __restrict__ conf,
                                                     int32_t* __restrict__ conf_ov, int32_t* __restrict__ pool,
                                                     int64_t pool_cap, int32_t slots, long long* __restrict__ counters) {
   const dp_dev_sys& S = *Sp;
   const int lane = threadIdx.x % 64;
   const uint64_t ltmask = (1ull << lane) - 1ull;
-  const long long ncl = counters[DPC_CELLS];
+  const long long ncl = (long long)((unsigned long long)counters[DPC_SORTED] >> 32);
   const double T = dp_pos_bound(S, r);
   // quadrotor: |q.q'| below cos(r / w1) - 1e-9 puts the attitude term alone
   // above r (acos is decreasing with slope <= -1, and the margin dwarfs the
   // series' error), so the pair is rejected without the acos
   const double cq = NX == 13 && S.w[1] > 0.0 && r / S.w[1] < DP_HALF_PI ? cos(r / S.w[1]) - 1e-9 : -1.0;
-  const int64_t d01 = (int64_t)G.dims[0] * G.dims[1];
+  constexpr int kRec = dp_cont_rec(NX);
   const long long nwaves = (long long)gridDim.x * (blockDim.x / 64);
   constexpr int kU = NX == 13 ? 2 : 4;  // candidates per lane in flight
   // Workgroups are dealt to the 8 XCDs in turn and each XCD has its own L2;
@@ -333,11 +496,13 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
     w_step = nwaves / 8;
   }
   for (long long w = w0; w < w_end; w += w_step) {
-    const uint32_t item = (uint32_t)cells[w];
-    const int64_t cell = item & 0xFFFFFFu;
-    const int32_t part = (int32_t)(item >> 24);
-    const int32_t c0 = (int32_t)(cell % G.dims[0]), c1 = (int32_t)((cell / G.dims[0]) % G.dims[1]);
-    const int32_t c2 = (int32_t)(cell / d01);
+    const int2 item = items[w];
+    const uint32_t cell = (uint32_t)item.x & 0x3ffffffu;
+    const int m = (int)((uint32_t)item.x >> 26) + 1;
+    const int32_t g0 = item.y;
+    const uint32_t line = cell / (uint32_t)G.row;
+    const int32_t c0 = (int32_t)(cell - line * (uint32_t)G.row);
+    const int32_t c2 = (int32_t)(line / (uint32_t)G.dims[1]), c1 = (int32_t)(line - (uint32_t)c2 * (uint32_t)G.dims[1]);
     // run k (lanes 0..8): rows c1 + k%3 - 1, layers c2 + k/3 - 1 (headings, or z for the
     // quadrotor; the rules of dp_cell_neighbor)
     int n = 0, st = 0;
@@ -355,7 +520,7 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
         ok = ok && n2 >= 0 && n2 < G.dims[2];
       }
       if (ok) {
-        const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.dims[0];
+        const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.row;
         const int32_t x0 = c0 > 0 ? c0 - 1 : 0, x1 = c0 + 1 < G.dims[0] ? c0 + 1 : G.dims[0] - 1;
         st = cstart[row + x0];
         n = cstart[row + x1 + 1] - st;
@@ -375,27 +540,19 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
       rp[k] = __builtin_amdgcn_readlane(incl - n, k);
     }
     const int K = __builtin_amdgcn_readlane(incl, 8);
-    const int32_t b0 = cstart[cell], e0 = cstart[cell + 1];
-    const int32_t per = cell_part_size(e0 - b0, K, 64 * kU);
-    const int32_t b = b0 + part * per, e = e0 < b + per ? e0 : b + per;
-    // the cell's contenders, 64 at a time, one per lane
-    for (int32_t g0 = b; g0 < e; g0 += 64) {
-      const int m = e - g0 < 64 ? e - g0 : 64;
+    // the item's contenders, one per lane
+    {
       int32_t q_l = INT32_MAX;
       bool list_l = false;
-      // the group's states, one per lane (broadcast by readlane below)
-      double x_l[NX];
+      // their states, one per lane (broadcast by readlane below)
+      double x_l[kRec];
 #pragma unroll
-      for (int k = 0; k < NX; ++k) x_l[k] = 0.0;
+      for (int k = 0; k < kRec; ++k) x_l[k] = 0.0;
       if (lane < m) {
-#pragma unroll
-        for (int k = 0; k < NX; ++k) x_l[k] = cx[(int64_t)k * pcap + g0 + lane];
-        q_l = cidx[g0 + lane];
-        const int8_t fl = flags[q_l];
-        list_l = !(fl & 2);  // goal-forced: NOVEL without a list
-        // past the list window: scanned when reached (k_list_window set
-        // its negative list length)
-        if (window > 0 && (fl & DP_F_NOLIST)) list_l = false;
+        load_rec<NX>(cx, (int64_t)g0 + lane, x_l);
+        const uint32_t word = (uint32_t)__double_as_longlong(x_l[NX]);
+        q_l = (int32_t)(word & ~DP_CONT_NOLIST);
+        list_l = !(word & DP_CONT_NOLIST);
       }
       const uint64_t lists = __ballot(list_l);
       int cnt_l = 0;           // list length of this lane's contender so far
@@ -408,13 +565,11 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
           // candidate index and state, every component loaded together with
           // the batch (the contender loop below then runs without loads)
           int32_t o[kU];
-          int64_t tt[kU];
-          double y[kU][NX];
+          double y[kU][kRec];
 #pragma unroll
           for (int u = 0; u < kU; ++u) {
             const int j = j0 + 64 * u + lane;
             o[u] = INT32_MAX;
-            tt[u] = 0;
             if (j < K) {
               int k = 0;
 #pragma unroll
@@ -423,10 +578,8 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
 #pragma unroll
               for (int kk = 1; kk < 9; ++kk)
                 if (k == kk) sk = rs[kk], pk = rp[kk];
-              tt[u] = (int64_t)sk + (j - pk);
-              o[u] = cidx[tt[u]];
-#pragma unroll
-              for (int d = 0; d < NX; ++d) y[u][d] = cx[(int64_t)d * pcap + tt[u]];
+              load_rec<NX>(cx, (int64_t)sk + (j - pk), y[u]);
+              o[u] = (int32_t)((uint32_t)__double_as_longlong(y[u][NX]) & ~DP_CONT_NOLIST);
             }
           }
           for (uint64_t rem = who; rem; rem &= rem - 1ull) {
@@ -444,6 +597,7 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
             const long long off = pool_pass ? (long long)__builtin_amdgcn_readlane((int)off_l, c) : 0;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
+              if (u > 0 && j0 + 64 * u >= K) break;  // uniform: no candidate left in this batch
               bool hit = false;
               if (o[u] < q) {
                 // exact rejections of dp_within_col_pf, then the metric
@@ -495,55 +649,8 @@ __global__ __launch_bounds__(256) void k_conf_waves(const dp_dev_sys* __restrict
       }
       if (list_l) {
         conf_cnt[q_l] = (int16_t)(cnt_l < DP_CONF_MAX ? cnt_l : -1);
-        // no earlier contender at all: NOVEL unless the cap falls before it
-        // (a duplicate of the visited set is not a contender)
-        if (cnt_l == 0) flags[q_l] = (int8_t)(flags[q_l] | DP_F_NUC);
       }
     }
-  }
-}
-
-// List window (planar systems, limit > 0): the contenders of a node after
-// its first W in canonical order are flagged DP_F_NOLIST, and their list
-// length is set to -(1 + rank) (rank among the node's contenders, at most
-// 32766).  The walk reaches one of them only if more than W - limit
-// contenders before it were duplicates; it then records 1 + rank in
-// need[0], and later batches of the context use W = max(window,
-// need + need / 4 + 16) (a fixed window leaves need alone: need == null).
-// One wave per node.
-__global__ __launch_bounds__(64) void k_list_window(int32_t N, const int32_t* __restrict__ app,
-                                                    const int32_t* __restrict__ total,
-                                                    const int8_t* __restrict__ verdict, int8_t* __restrict__ flags,
-                                                    int16_t* __restrict__ conf_cnt, int32_t window,
-                                                    const int32_t* __restrict__ need) {
-  const int32_t node = blockIdx.x;
-  if (node >= N) return;
-  const int lane = threadIdx.x;
-  const uint64_t lt = (1ull << lane) - 1ull;
-  if (need) {
-    const int32_t nd = need[0];
-    const int64_t w = (int64_t)nd + nd / 4 + 16;
-    if (nd > 0 && w > window) window = w < INT32_MAX ? (int32_t)w : INT32_MAX;
-  }
-  const int32_t tot = *total;
-  const int32_t b = app[node] < tot ? app[node] : tot;
-  const int32_t e = app[node + 1] < tot ? app[node + 1] : tot;
-  int32_t rank = 0;
-  for (int32_t cb = b; cb < e; cb += 64) {
-    const int32_t p = cb + lane;
-    bool con = false;
-    int8_t fl = 0;
-    if (p < e && verdict[p] == DP_V_FREE) {
-      fl = flags[p];
-      con = (fl & 2) || !(fl & 1);
-    }
-    const uint64_t m = __ballot(con);
-    const int32_t r = rank + __popcll(m & lt);
-    if (con && r >= window) {
-      flags[p] = (int8_t)(fl | DP_F_NOLIST);
-      conf_cnt[p] = (int16_t)(-1 - (r < 32766 ? r : 32766));
-    }
-    rank += __popcll(m);
   }
 }
 
@@ -576,9 +683,8 @@ __global__ __launch_bounds__(64) void k_precap_first(int32_t N, const int32_t* _
 }
 
 // ---- Pre-resolution: statuses that are certain before the walk ----------
-// A contender without any earlier contender (flag DP_F_NUC, set by
-// k_conf_waves) or goal-forced is NOVEL unless its node's cap falls before
-// it.  Each conclusion below is a certainty, so the walk reaches the same
+// A contender with an empty list of earlier contenders, or a goal-forced one,
+// is NOVEL unless its node's cap falls before it.  Each conclusion below is a certainty, so the walk reaches the same
 // statuses; waiting waves only meet fewer undecided contenders.
 //
 // One wave per node, its FREE pairs in order: after the limit-th pair that
@@ -591,7 +697,8 @@ __global__ __launch_bounds__(64) void k_precap_first(int32_t N, const int32_t* _
 __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __restrict__ app,
                                                    const int32_t* __restrict__ total,
                                                    const int8_t* __restrict__ verdict,
-                                                   const int8_t* __restrict__ flags, int8_t* __restrict__ res,
+                                                   const int8_t* __restrict__ flags,
+                                                   const int16_t* __restrict__ conf_cnt, int8_t* __restrict__ res,
                                                    int32_t limit, int32_t* __restrict__ cursor,
                                                    int32_t* __restrict__ count, int32_t* __restrict__ node_novel,
                                                    long long* __restrict__ counters) {
@@ -619,12 +726,14 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
     constexpr int kPre = 4;
     for (int32_t c0 = b; c0 < e; c0 += 64 * kPre) {
       int8_t v_u[kPre], f_u[kPre], r_u[kPre];
+      int16_t n_u[kPre];
 #pragma unroll
       for (int u = 0; u < kPre; ++u) {
         const int32_t p = c0 + 64 * u + lane < e ? c0 + 64 * u + lane : e - 1;
         v_u[u] = verdict[p];
         f_u[u] = flags[p];
         r_u[u] = res[p];
+        n_u[u] = conf_cnt[p];
       }
 #pragma unroll
       for (int u = 0; u < kPre; ++u) {
@@ -634,7 +743,8 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
         const int r = valid ? r_u[u] : DP_R_NONE;
         const bool dupv = (fl & 1) && !(fl & 2);
         const bool not_nov = valid && (dupv || r == DP_R_CAPPED);
-        const bool nuc_p = valid && (r == DP_R_NOVEL || (fl & (2 | DP_F_NUC)) != 0);
+        const bool nuc_p = valid && (r == DP_R_NOVEL || (fl & 2) != 0 ||
+                                     (!(fl & (1 | DP_F_DEFER)) && n_u[u] == 0));
         const uint64_t nuc_m = __ballot(nuc_p);
         const uint64_t pos_m = __ballot(valid && !not_nov);
         const int nuc_before = nuc + __popcll(nuc_m & lt);
@@ -722,7 +832,6 @@ struct round_args {
   int64_t pcap;
   dp_grid_geom grid;
   const int32_t* cstart;
-  const int32_t* cidx;
   const double* cx;
   double r_dup;
   int8_t* res;
@@ -873,7 +982,7 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
       double x[NX];
 #pragma unroll
       for (int k = 0; k < NX; ++k) x[k] = a.fin[(int64_t)k * a.pcap + p];
-      scan_earlier<NX>(*a.sys, a.grid, a.cstart, a.cidx, a.cx, a.pcap, x, p, a.r_dup, visit, [&](int32_t o) {
+      scan_earlier<NX>(*a.sys, a.grid, a.cstart, a.cx, x, p, a.r_dup, visit, [&](int32_t o) {
         if (o >= cb) return true;
         const int v = a.res[o];
         return v == DP_R_NOVEL || v == DP_R_UNDECIDED;
@@ -1353,7 +1462,6 @@ static round_args make_round_args(dp_ctx* c) {
   a.pcap = c->pair_cap;
   a.grid = c->grid;
   a.cstart = c->d_cont_start;
-  a.cidx = c->d_cont_idx;
   a.cx = c->d_cont_x;
   a.r_dup = c->round_r_dup;
   a.res = c->d_res;
@@ -1372,42 +1480,57 @@ static round_args make_round_args(dp_ctx* c) {
   return a;
 }
 
+static int cell_row_blocks(const dp_grid_geom& G) {
+  return (int)(((int64_t)G.dims[1] * G.dims[2] + kRowWaves - 1) / kRowWaves);
+}
+
+namespace {
+__global__ void k_vis_clear(int32_t* __restrict__ count, int64_t n, long long* __restrict__ counters) {
+  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t0 == 0) counters[DPC_SORTED] = 0;
+  for (int64_t t = t0; t < n; t += (int64_t)gridDim.x * blockDim.x) count[t] = 0;
+}
+}  // namespace
+
+int dp_ensure_cont_grid(dp_ctx* c) {
+  int rc = dp_ensure_i32(&c->d_cont_count, &c->cont_count_cap, c->grid.nslots);
+  return rc ? rc : dp_ensure_i32(&c->d_cont_start, &c->cont_start_cap, c->grid.nslots);
+}
+
 int dp_launch_visited_rebuild(dp_ctx* c, double radius, hipStream_t s) {
   c->grid = dp_make_grid(c, radius);
   c->grid_radius = radius;
-  const int64_t nc = c->grid.ncells;
-  int rc = dp_ensure_i32(&c->d_vis_start, &c->vis_cells_cap, nc + 1);
+  const int64_t nc = c->grid.nslots;
+  int rc = dp_ensure_i32(&c->d_vis_start, &c->vis_cells_cap, nc);
+  if (!rc) rc = dp_ensure_i32(&c->d_vis_count, &c->vis_count_cap, nc);
   if (rc) return rc;
-  dp_fill_i32(c->d_vis_start, nc + 1, 0, s);
-  if (c->nv > 0) {
-    rc = dp_ensure_i32(&c->d_cont_cursor, &c->cont_cursor_cap, nc + 1);
-    if (rc) return rc;
-    rc = dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
-      constexpr int NX = decltype(NXc)::value;
+  // the counters belong to the batch before; only the row kernel's use is
+  // cleared with the counts
+  k_vis_clear<<<dp_grid_blocks(nc, 256, 2048), 256, 0, s>>>(c->d_vis_count, nc, c->d_counters);
+  rc = dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
+    constexpr int NX = decltype(NXc)::value;
+    if (c->nv > 0)
       k_vis_count<NX><<<dp_grid_blocks(c->nv, 256, 8192), 256, 0, s>>>(c->grid, c->d_vis, c->nv_cap, c->nv,
-                                                                      c->d_vis_cell, c->d_vis_start);
-      (void)dp_scan_large(c, c->d_vis_start, nullptr, nc, c->d_counters, -1, s);
-      dp_fill_i32(c->d_cont_cursor, nc, 0, s);
+                                                                      c->d_vis_cell, c->d_vis_rank, c->d_vis_count);
+    k_cell_rows<false><<<cell_row_blocks(c->grid), 64 * kRowWaves, 0, s>>>(c->grid, c->d_vis_count, c->d_vis_start, 1, nullptr,
+                                                                c->d_counters);
+    if (c->nv > 0)
       k_vis_scatter<NX><<<dp_grid_blocks(c->nv, 256, 8192), 256, 0, s>>>(c->d_vis, c->nv_cap, c->nv, c->d_vis_cell,
-                                                                        c->d_vis_start, c->d_cont_cursor,
+                                                                        c->d_vis_rank, c->d_vis_start,
                                                                         c->d_vis_sorted, c->d_vis_perm);
-      return DP_OK;
-    });
-    if (rc) return rc;
-  }
+    return DP_OK;
+  });
+  if (rc) return rc;
   DP_HIP_RET(hipGetLastError());
   c->grid_dirty = false;
   dp_bump_epoch();
   return DP_OK;
 }
 
-int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, hipStream_t s) {
-  const int64_t nc = c->grid.ncells;
+int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool counted, hipStream_t s) {
+  const int64_t nc = c->grid.nslots;
   const int32_t N = c->N;
-  // the scatter cursors, then the conflict-wave items: at most one per
-  // contender
-  int rc = dp_ensure_i32(&c->d_cont_start, &c->cont_start_cap, nc + 1);
-  if (!rc) rc = dp_ensure_i32(&c->d_cont_cursor, &c->cont_cursor_cap, std::max<int64_t>(nc + 1, c->pair_cap));
+  int rc = dp_ensure_cont_grid(c);
   if (rc) return rc;
   c->round_limit = p->limit_branching_factor;
   c->round_r_dup = r_dup;
@@ -1427,28 +1550,31 @@ int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, hipStr
     constexpr int NX = decltype(NXc)::value;
     if (p->limit_branching_factor == 0 && N > 0)
       k_precap_first<<<N, 64, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_res);
-    if (window > 0 && N > 0)
-      k_list_window<<<N, 64, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_conf_cnt, window,
-                                     lneed);
-    dp_fill_i32(c->d_cont_start, nc + 1, 0, s);
-    k_cont_count<NX><<<pb, 256, 0, s>>>(c->grid, c->d_total, c->d_verdict, c->d_flags, c->d_final, c->pair_cap,
-                                        c->d_cont_start);
-    (void)dp_scan_large(c, c->d_cont_start, nullptr, nc, c->d_counters, -1, s);
-    dp_fill_i32(c->d_cont_cursor, nc, 0, s);
-    k_cont_scatter<NX><<<pb, 256, 0, s>>>(c->grid, c->d_total, c->d_verdict, c->d_flags, c->d_final, c->pair_cap,
-                                          c->d_cont_start, c->d_cont_cursor, c->d_cont_idx, c->d_cont_x);
-    // earlier-conflict lists; the scatter cursors are free again and hold
-    // the list of non-empty cells
-    k_cell_list<<<(int)((nc + 255) / 256), 256, 0, s>>>(nc, c->grid, c->d_cont_start, c->d_cont_idx, window,
-                                                                64 * (NX == 13 ? 2 : 4), c->d_flags, c->d_conf_cnt,
-                                                                c->d_cont_cursor, c->d_counters);
+    if (!counted) {
+      dp_fill_i32(c->d_cont_count, nc, 0, s);
+      k_cont_count<NX><<<pb, 256, 0, s>>>(c->grid, c->d_total, c->d_verdict, c->d_flags, c->d_final, c->pair_cap,
+                                          c->d_cont_count, c->d_cont_cell, c->d_conf_ov);
+    }
+    int2* items = reinterpret_cast<int2*>(c->d_cont_item);
+    k_cell_rows<true><<<cell_row_blocks(c->grid), 64 * kRowWaves, 0, s>>>(c->grid, c->d_cont_count, c->d_cont_start,
+                                                               64 * (NX == 13 ? 2 : 4), items, c->d_counters);
+    // after the quadrotor's FP32 pass the FP64 list holds every contender
+    if (counted && NX == 13 && p->fp32_rollout)
+      k_cont_scatter_list<NX><<<dp_grid_blocks(c->pair_cap, 256, 1024), 256, 0, s>>>(
+          c->d_q64, c->d_counters + DPC_Q64, c->d_verdict, c->d_flags, c->d_final, c->pair_cap, c->d_cont_count,
+          c->d_cont_start, c->d_cont_cell, c->d_conf_ov, c->d_conf_cnt, c->d_cont_x);
+    else
+      k_cont_scatter<NX><<<(N + 3) / 4, 256, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_final,
+                                                   c->pair_cap, c->d_cont_count, c->d_cont_start, c->d_cont_cell,
+                                                   c->d_conf_ov, window, lneed, c->d_conf_cnt, c->d_cont_x);
+    // earlier-conflict lists
     k_conf_waves<NX><<<(int)std::min<int64_t>((nc + 3) / 4, 8192), 256, 0, s>>>(
-        c->d_sys, c->grid, c->d_flags, c->d_pnode, c->d_app, window, c->pair_cap, c->d_cont_start, c->d_cont_idx, c->d_cont_x, c->d_cont_cursor,
-        r_dup, c->d_conf_cnt, c->d_conf, c->d_conf_ov, c->d_conf_pool, pool_cap, c->conf_slots, c->d_counters);
+        c->d_sys, c->grid, c->d_cont_start, c->d_cont_x, items, r_dup, c->d_conf_cnt, c->d_conf, c->d_conf_ov,
+        c->d_conf_pool, pool_cap, c->conf_slots, c->d_counters);
     if (dp_record_event(c, 7, s)) return DP_ERR_HIP;
     if (p->limit_branching_factor > 0)
-      k_pre_nodes<<<(N + 3) / 4, 256, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_res,
-                                               p->limit_branching_factor, c->d_node_cursor, c->d_node_count,
+      k_pre_nodes<<<(N + 3) / 4, 256, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_conf_cnt,
+                                               c->d_res, p->limit_branching_factor, c->d_node_cursor, c->d_node_count,
                                                c->d_node_novel, c->d_counters);
     else
       k_round_init<<<dp_grid_blocks(N, 256, 1024), 256, 0, s>>>(N, c->d_app, c->d_total, c->d_node_cursor,
@@ -1473,11 +1599,10 @@ __global__ void k_reset_resolution(const int32_t* __restrict__ total, const int8
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot; q += (int64_t)gridDim.x * blockDim.x) {
     if (verdict[q] != DP_V_FREE || (flags[q] & DP_F_PRECAP)) continue;
     res[q] = DP_R_UNDECIDED;
-    flags[q] = (int8_t)(flags[q] & ~DP_F_NUC);
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int slots[] = {DPC_NOVEL, DPC_DUPV, DPC_DUPB, DPC_CAPPED, DPC_GOAL, DPC_NODES_LEFT, DPC_CONF,
-                         DPC_TICKET, DPC_CELLS, DPC_WINDOW_OVF, DPC_ROUNDS};
+                         DPC_TICKET, DPC_SORTED, DPC_WINDOW_OVF, DPC_ROUNDS};
     for (int k : slots) counters[k] = 0;
     counters[DPC_ERRFLAG] &= ~2ll;
   }
@@ -1489,7 +1614,7 @@ int dp_launch_resolve_again(dp_ctx* c, hipStream_t s) {
                                                                            c->d_res, c->d_counters);
   DP_HIP_RET(hipGetLastError());
   const dp_expand_params p = c->round_params;
-  return dp_launch_resolve(c, &p, c->round_r_dup, s);
+  return dp_launch_resolve(c, &p, c->round_r_dup, false, s);
 }
 
 int dp_launch_more_rounds(dp_ctx* c, int rounds, hipStream_t s) {

@@ -100,6 +100,10 @@ struct dp_quad_args {
   const int32_t* rbad32;  // [P] the same in FP32
   const int32_t* rnear32; // [P] first FP32 state within the re-check margin of an attitude / rate bound
   const quad_rec* qrec;   // [P] the FP32 pass's view of each primitive
+  // contender grid (count null: contenders are not counted by this pass)
+  int32_t* cont_count;
+  int32_t* cont_cell;
+  int32_t* cont_place;
   long long* counters;
 };
 
@@ -972,6 +976,8 @@ __global__ __launch_bounds__(256) void k_quad64(dp_quad_args a) {
       for (int k = 0; k < 9 && !dupv; ++k)
         dupv = dp_grid_run_any<13>(S, a.grid, a.vstart, a.vis, a.vstride, x, k, a.r_dup, Tdup);
     a.flags[q] = (int8_t)((chosen != -1 ? 2 : 0) | (dupv ? 1 : 0));
+    if (a.cont_count && (chosen != -1 || !dupv))
+      dp_count_contender(a.grid, x, q, a.cont_count, a.cont_cell, a.cont_place);
     c_f += !a.redo;
   }
   if (c_b) atomicAdd(&s_cnt[0], (unsigned long long)c_b);
@@ -1325,8 +1331,11 @@ extern "C" int dp_debug_rollout_states(dp_ctx* c, const int32_t* pairs, int32_t 
   return DP_OK;
 }
 
-int dp_launch_quad(dp_ctx* c, const dp_expand_params* p, double goal_bound, double r_dup, hipStream_t s) {
+int dp_launch_quad(dp_ctx* c, const dp_expand_params* p, double goal_bound, double r_dup, bool count, hipStream_t s) {
   dp_quad_args a = make_quad_args(c, p, goal_bound, r_dup);
+  a.cont_count = count ? c->d_cont_count : nullptr;
+  a.cont_cell = c->d_cont_cell;
+  a.cont_place = c->d_conf_ov;
   if (p->fp32_rollout) {
     const size_t lds = sizeof(float) * kQWaves * (6 * (size_t)c->nb + 4 * (size_t)c->ns + 1);
     if (lds > 64 * 1024) {

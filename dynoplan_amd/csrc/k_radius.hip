@@ -45,7 +45,7 @@ int radius_dispatch(int nx, F&& f) {
 struct radius_args {
   const dp_dev_sys* sys;
   dp_grid_geom grid;
-  const int32_t* vstart;   // [ncells+1] visited grid cell offsets
+  const int32_t* vstart;   // [nslots] visited grid cell offsets
   const double* vis;       // [nx][vstride] visited states sorted by cell
   int64_t vstride;
   const int32_t* vperm;    // [nv] sorted position -> append index
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
         ok = ok && n2 >= 0 && n2 < G.dims[2];
       }
       if (ok) {
-        const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.dims[0];
+        const int64_t row = ((int64_t)n2 * G.dims[1] + n1) * G.row;
         const int32_t x0 = c[0] > 0 ? c[0] - 1 : 0, x1 = c[0] + 1 < G.dims[0] ? c[0] + 1 : G.dims[0] - 1;
         st = a.vstart[row + x0];
         len = a.vstart[row + x1 + 1] - st;
