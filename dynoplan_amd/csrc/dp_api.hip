@@ -197,7 +197,7 @@ dp_ctx* dp_create(const dp_system_desc* sys, int32_t device) {
   c->desc = *sys;
   c->nbox = sys->system == DP_SYS_CAR_TRAILER ? 2 : 1;
   bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
-  for (int k = 0; k < DP_EVENTS && ok; ++k) ok = hipEventCreate(&c->ev[k]) == hipSuccess;
+  for (int k = 0; k < 2 && ok; ++k) ok = hipEventCreate(&c->ev[k]) == hipSuccess;
   ok = ok && dev_alloc(&c->d_sys, 1) == DP_OK;
   ok = ok && dev_alloc(&c->d_counters, DPC_COUNT) == DP_OK;
   ok = ok && dev_alloc(&c->d_sticky, DPS_COUNT) == DP_OK;
@@ -207,6 +207,9 @@ dp_ctx* dp_create(const dp_system_desc* sys, int32_t device) {
   ok = ok && dev_alloc(&c->d_lneed, 1) == DP_OK;
   ok = ok && hipMemset(c->d_lneed, 0, sizeof(int32_t)) == hipSuccess;
   ok = ok && dev_alloc(&c->d_total, 1) == DP_OK;
+  ok = ok && dev_alloc(&c->d_marks, DP_MARKS) == DP_OK;
+  ok = ok && hipDeviceGetAttribute(&c->wall_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess &&
+       c->wall_khz > 0;
   ok = ok && hipMemset(c->d_counters, 0, sizeof(long long) * DPC_COUNT) == hipSuccess;
   ok = ok && hipMemset(c->d_total, 0, sizeof(int32_t)) == hipSuccess;
   ok = ok && upload_sys(c) == DP_OK;
@@ -258,6 +261,7 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_nodes);
   dev_free(&c->d_gpar);
   dev_free(&c->d_app);
+  dev_free(&c->d_app_cnt);
   dev_free(&c->d_app_mask);
   dev_free(&c->d_node_novel);
   dev_free(&c->d_pnode);
@@ -290,6 +294,7 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_preach);
   dev_free(&c->d_dv64);
   dev_free(&c->d_dv32);
+  dev_free(&c->d_qshort);
   dev_free(&c->d_rbad64);
   dev_free(&c->d_rbad32);
   dev_free(&c->d_rnear32);
@@ -299,7 +304,8 @@ void dp_destroy(dp_ctx* c) {
   dev_free(&c->d_counters);
   dev_free(&c->d_sticky);
   dev_free(&c->d_total);
-  for (int k = 0; k < DP_EVENTS; ++k)
+  dev_free(&c->d_marks);
+  for (int k = 0; k < 2; ++k)
     if (c->ev[k]) (void)hipEventDestroy(c->ev[k]);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -527,6 +533,7 @@ int dp_upload_primitives(dp_ctx* c, const dp_prims* pr, int32_t max_motions) {
     if ((rc = dev_alloc(&c->d_rot64, (int64_t)7 * S))) return rc;
     if ((rc = dev_alloc(&c->d_dv64, (int64_t)4 * S))) return rc;
     if ((rc = dev_alloc(&c->d_dv32, (int64_t)4 * S))) return rc;
+    if ((rc = dev_alloc(&c->d_qshort, (P + 63) / 64))) return rc;
     if ((rc = dev_alloc(&c->d_rbad64, P))) return rc;
     if ((rc = dev_alloc(&c->d_rbad32, P))) return rc;
     if ((rc = dev_alloc(&c->d_rnear32, P))) return rc;
@@ -640,6 +647,7 @@ int dp_reserve(dp_ctx* c, int32_t max_nodes, int64_t max_pairs) {
     if ((rc = dev_alloc(&c->d_nodes, (int64_t)nx * max_nodes))) return rc;
     if ((rc = dev_alloc(&c->d_gpar, max_nodes))) return rc;
     if ((rc = dev_alloc(&c->d_app, (int64_t)max_nodes + 1))) return rc;
+    if ((rc = dev_alloc(&c->d_app_cnt, (int64_t)max_nodes + 1))) return rc;
     if ((rc = dev_alloc(&c->d_node_novel, (int64_t)max_nodes + 1))) return rc;
     if ((rc = dev_alloc(&c->d_node_cursor, max_nodes))) return rc;
     if ((rc = dev_alloc(&c->d_node_count, max_nodes))) return rc;
@@ -1074,30 +1082,40 @@ int dp_visited_append_novel(dp_ctx* c) {
 }
 
 
-int dp_last_timing(dp_ctx* c, float* ms5) {
-  ARG_CHECK(c && ms5, "null argument");
+// The marks of the last expansion in ms after its start.
+static int stage_marks(dp_ctx* c, float* at) {
   if (!c->timing_valid) {
     dp_set_error("no expansion has been timed");
     return DP_ERR_STATE;
   }
-  HIP_CHECK(hipEventSynchronize(c->ev[3]));
-  HIP_CHECK(hipEventElapsedTime(&ms5[0], c->ev[0], c->ev[4]));
-  HIP_CHECK(hipEventElapsedTime(&ms5[1], c->ev[1], c->ev[2]));
-  HIP_CHECK(hipEventElapsedTime(&ms5[2], c->ev[2], c->ev[3]));
-  HIP_CHECK(hipEventElapsedTime(&ms5[3], c->ev[0], c->ev[3]));
-  HIP_CHECK(hipEventElapsedTime(&ms5[4], c->ev[4], c->ev[1]));
+  HIP_CHECK(hipEventSynchronize(c->ev[1]));
+  unsigned long long m[DP_MARKS];
+  HIP_CHECK(hipMemcpy(m, c->d_marks, sizeof(m), hipMemcpyDeviceToHost));
+  for (int k = 0; k < DP_MARKS; ++k) at[k] = (float)((double)(long long)(m[k] - m[0]) / (double)c->wall_khz);
+  HIP_CHECK(hipEventElapsedTime(&at[3], c->ev[0], c->ev[1]));
+  return DP_OK;
+}
+
+int dp_last_timing(dp_ctx* c, float* ms5) {
+  ARG_CHECK(c && ms5, "null argument");
+  float at[DP_MARKS];
+  int rc = stage_marks(c, at);
+  if (rc) return rc;
+  ms5[0] = at[4];
+  ms5[1] = at[2] - at[1];
+  ms5[2] = at[3] - at[2];
+  ms5[3] = at[3];
+  ms5[4] = at[1] - at[4];
   return DP_OK;
 }
 
 int dp_last_timing_detail(dp_ctx* c, float* ms7) {
   ARG_CHECK(c && ms7, "null argument");
-  if (!c->timing_valid) {
-    dp_set_error("no expansion has been timed");
-    return DP_ERR_STATE;
-  }
-  HIP_CHECK(hipEventSynchronize(c->ev[3]));
+  float at[DP_MARKS];
+  int rc = stage_marks(c, at);
+  if (rc) return rc;
   const int from[7] = {0, 4, 1, 5, 6, 2, 7}, to[7] = {4, 1, 5, 6, 2, 7, 3};
-  for (int k = 0; k < 7; ++k) HIP_CHECK(hipEventElapsedTime(&ms7[k], c->ev[from[k]], c->ev[to[k]]));
+  for (int k = 0; k < 7; ++k) ms7[k] = at[to[k]] - at[from[k]];
   return DP_OK;
 }
 

@@ -51,8 +51,12 @@
 // Resolution trace, per node: start and end clock of its wave, cycles
 // waiting, evaluating lists and walking chunks, chunks, waits, polls.
 #define DP_TRACE_FIELDS 8
-// HIP events of one expansion (stage and kernel timing)
-#define DP_EVENTS 8
+// Stage marks of one expansion (dp_last_timing): 0 start, 4 applicability
+// done, 1 pre-filter done, 5 before the main check kernel, 6 after it, 2 check
+// done, 7 lists done, 3 end.  Marks 0 and 3 are HIP events; between them the
+// first kernel of each stage writes the GPU's constant-rate clock (an event
+// between two kernels costs the stream about 4 us).
+#define DP_MARKS 8
 // LDS per workgroup on gfx950
 #define DP_LDS_MAX 163840
 #define DP_SPIN_LIMIT_WAITING (1 << 10)
@@ -68,7 +72,7 @@ void dp_set_error(const std::string& msg);
 enum {
   DPC_PAIRS = 0, DPC_BOUNDS, DPC_COLLIDE, DPC_FREE, DPC_SURR, DPC_NOVEL, DPC_DUPV, DPC_DUPB,
   DPC_CAPPED, DPC_GOAL, DPC_CHECKED, DPC_RECHECK, DPC_ROUNDS, DPC_ERRFLAG, DPC_OVERFLOW,
-  DPC_NODES_LEFT, DPC_CONF, DPC_TICKET, DPC_SORTED, DPC_WINDOW_OVF, DPC_DEFERRED, DPC_Q64, DPC_CONSTRAINT,
+  DPC_NODES_LEFT, DPC_CONF, DPC_TICKET, DPC_SORTED, DPC_WALK, DPC_WINDOW_OVF, DPC_DEFERRED, DPC_Q64, DPC_CONSTRAINT,
   DPC_COUNT
 };
 // DPC_SORTED: contender records in cell order (low 32 bits) and conflict-wave
@@ -167,6 +171,19 @@ struct dp_mlp {
   float* loss = nullptr;
 };
 
+// Stage marks a kernel writes as it starts (bit k of mask: mark k; at null: none).
+struct dp_marks {
+  unsigned long long* at;
+  uint32_t mask;
+};
+__device__ __forceinline__ void dp_mark(const dp_marks& m) {
+  if (m.at && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    const unsigned long long t = (unsigned long long)wall_clock64();
+    for (int k = 0; k < DP_MARKS; ++k)
+      if ((m.mask >> k) & 1u) m.at[k] = t;
+  }
+}
+
 struct dp_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -222,7 +239,8 @@ struct dp_ctx {
   int32_t N = 0, N_cap = 0;
   double* d_nodes = nullptr;  // [nx][N_cap]
   double* d_gpar = nullptr;   // [N_cap]
-  int32_t* d_app = nullptr;   // [N_cap+1] counts, then exclusive offsets
+  int32_t* d_app_cnt = nullptr;   // [N_cap+1] applicable primitives per node
+  int32_t* d_app = nullptr;       // [N_cap+1] their exclusive scan: each node's first pair
   uint64_t* d_app_mask = nullptr;  // [N][ceil(P/64)] applicable primitives per node
   int64_t app_mask_cap = 0;
 
@@ -258,7 +276,7 @@ struct dp_ctx {
   int32_t* d_node_count = nullptr;  // [N_cap] NOVEL pairs decided per node
   long long* h_pinned = nullptr;    // pinned host words for device totals
   int32_t rounds = 32;              // resolution rounds launched per batch
-  int32_t* d_chunk = nullptr;       // [N_cap+1] quadrotor: 64-pair chunks per node, scanned
+  int32_t* d_chunk = nullptr;       // [N_cap+1] quadrotor: 64-pair chunks per node, then scanned
   int32_t* d_nshort = nullptr;      // [N_cap] quadrotor: pairs whose primitive leaves the rate bounds
   int32_t* d_qperm = nullptr;       // [2][pair_cap] quadrotor: (pair, primitive) per node, rate-bound ones first
   int32_t* d_chunk_node = nullptr;  // quadrotor: node of each FP32 wave chunk
@@ -270,6 +288,7 @@ struct dp_ctx {
   double* d_rot64 = nullptr;        // [7][S]
   double* d_dv64 = nullptr;         // [S][4] (x y z, pad)
   float* d_dv32 = nullptr;          // [S][4]
+  uint64_t* d_qshort = nullptr;     // [ceil(P/64)] bit j: primitive j leaves the rate bounds (rbad32 < its length)
   int32_t *d_rbad64 = nullptr, *d_rbad32 = nullptr, *d_rnear32 = nullptr;  // [P]
   double* d_qrec = nullptr;         // [P][16] quadrotor: the FP32 pass's 128-byte record per primitive
   double prim_reach = 0.0;          // max over primitives of max_k |p_k - p_0|_inf
@@ -311,10 +330,9 @@ struct dp_ctx {
   int32_t* d_scan_tmp = nullptr;    // [1024] block partials
 
   // timing
-  // expansion stage events: 0 start, 4 applicability done, 1 pre-filter
-  // done, 5 before the main check kernel, 6 after it, 2 check done, 7 lists
-  // done, 3 end
-  hipEvent_t ev[DP_EVENTS] = {};
+  hipEvent_t ev[2] = {};            // start and end of the expansion
+  unsigned long long* d_marks = nullptr;  // [DP_MARKS] stage clocks of the last expansion
+  int wall_khz = 0;
   bool timing_valid = false;
   bool no_events = false;           // set while a multi-instance graph is captured
   bool defer_walk = false;          // set while a multi-instance batch launches: no walk (dp_walk_queue)
@@ -344,12 +362,10 @@ inline int dp_grid_blocks(int64_t work, int per_block, int max_blocks) {
 
 int dp_ensure_i32(int32_t** p, int64_t* cap, int64_t need);
 
-// Records stage event k of the expansion on s (skipped while a
-// multi-instance graph is captured).
-inline int dp_record_event(dp_ctx* c, int k, hipStream_t s) {
-  if (c->no_events) return DP_OK;
-  DP_HIP_RET(hipEventRecord(c->ev[k], s));
-  return DP_OK;
+// Marks written by a kernel of the batch being launched (none while a
+// multi-instance batch launches or is captured).
+inline dp_marks dp_stage(const dp_ctx* c, uint32_t mask) {
+  return dp_marks{c->no_events || c->defer_walk ? nullptr : c->d_marks, mask};
 }
 int dp_ensure_f64(double** p, int64_t* cap, int64_t need);
 int dp_ensure_u64(uint64_t** p, int64_t* cap, int64_t need);
@@ -357,12 +373,13 @@ int dp_ensure_u64(uint64_t** p, int64_t* cap, int64_t need);
 // ---- k_util.hip ---------------------------------------------------------
 void dp_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 // Clears the batch counters, a[0..na) and b[0..nb) in one launch.
-void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t nb, hipStream_t s);
-// Exclusive scan of data[0..n-1] into data[0..n]; data[n] = total.  Small n
-// (one workgroup).  total (optional) receives min(total, cap); counters[slot]
-// receives the total when slot >= 0.
-void dp_scan_small(int32_t* data, int64_t n, int32_t* total, int64_t cap, long long* counters, int slot,
-                   hipStream_t s);
+void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t nb, dp_marks marks, hipStream_t s);
+// Exclusive scan of src[0..n-1] into dst[0..n] (dst may be src); dst[n] =
+// total.  One workgroup.  total (optional) receives min(total, cap);
+// counters[slot] receives the total when slot >= 0.
+void dp_scan_small(const int32_t* src, int32_t* dst, int64_t n, int32_t* total, int64_t cap, long long* counters,
+                   int slot, hipStream_t s);
+
 // ---- k_grid.hip ---------------------------------------------------------
 dp_grid_geom dp_make_grid(const dp_ctx* c, double r);
 int dp_launch_visited_rebuild(dp_ctx* c, double radius, hipStream_t s);

@@ -292,42 +292,124 @@ __global__ __launch_bounds__(64) void k_app_blk(const dp_dev_sys* __restrict__ S
 // words at a time: each lane expands its own word's set bits into LDS at the
 // word's offset (an exclusive scan of the counts across the lanes), then the
 // wave copies the batch out with full-width stores.
+//
+// Up to kFillScan nodes the wave sums the counts of the nodes before its own
+// itself (at most 16 loads per lane) and writes the node's offset: no scan
+// launch.  The quadrotor's FP32 pass also gets the node's pairs reordered
+// from here (qperm: (pair, primitive)), those whose primitive leaves the
+// attitude / rate bounds first (BOUNDS whatever the translation: short
+// rollouts, no collision tests), each group in canonical order: with one bit
+// per primitive the two groups' places are bit counts of the masks, where a
+// kernel that looked every pair's primitive up took 16 us (1.13M pairs).
+constexpr int32_t kFillScan = 1024;
+
+struct fill_args {
+  int32_t N, P;
+  const int32_t* cnt;      // pairs per node
+  int32_t* app;            // offsets: read, or written when scan is set
+  int32_t scan;
+  const uint64_t* mask;
+  const int32_t* order;
+  int32_t rows;
+  int32_t* pnode;
+  int32_t* pprim;
+  int64_t pair_cap;
+  int32_t* total;
+  long long* counters;
+  const uint64_t* qshort;  // quadrotor FP32 pass (else null): bit j: the primitive's rates leave the bounds
+  int2* qperm;
+  int32_t* nshort;
+  int32_t* chunks;         // 64-pair chunks of the two groups
+};
+
 template <bool kRow>
-__global__ __launch_bounds__(64) void k_app_fill(int32_t N, int32_t P, const int32_t* __restrict__ app,
-                                                 const uint64_t* __restrict__ mask, const int32_t* __restrict__ order,
-                                                 int32_t rows, int32_t* __restrict__ pnode,
-                                                 int32_t* __restrict__ pprim, int64_t pair_cap) {
+__global__ __launch_bounds__(64) void k_app_fill(fill_args a) {
   __shared__ int32_t s_p[64 * 64];
   const int32_t i = blockIdx.x;
-  if (i >= N) return;
+  if (i >= a.N) return;
   const int lane = threadIdx.x;
-  const int32_t words = (P + 63) / 64;
-  const int32_t* row = kRow ? order + (int64_t)(i % rows) * P : nullptr;
-  int64_t q0 = app[i];
+  const int32_t words = (a.P + 63) / 64;
+  const int32_t* row = kRow ? a.order + (int64_t)(i % a.rows) * a.P : nullptr;
+  int64_t q0;
+  if (a.scan) {
+    long long sum = 0;
+    for (int32_t k = lane; k < i; k += 64) sum += a.cnt[k];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    q0 = sum;
+    if (lane == 0) {
+      a.app[i] = (int32_t)sum;
+      if (i == a.N - 1) {
+        const long long tot = sum + a.cnt[i];
+        a.app[a.N] = (int32_t)tot;
+        *a.total = (int32_t)(tot < a.pair_cap ? tot : a.pair_cap);
+        a.counters[DPC_PAIRS] = tot;
+        if (tot > a.pair_cap) a.counters[DPC_OVERFLOW] = 1;
+      }
+    }
+  } else {
+    q0 = a.app[i];
+  }
+  // first places of the short and the long group
+  int64_t ws = q0, wl = q0;
+  if (a.qshort) {
+    int32_t ns = 0;
+    for (int32_t w = lane; w < words; w += 64) ns += __popcll(a.mask[(int64_t)i * words + w] & a.qshort[w]);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) ns += __shfl_xor(ns, d, 64);
+    wl = q0 + ns;
+    if (lane == 0) {
+      // pairs past the capacity are dropped at the end of the list
+      const int64_t end = q0 + a.cnt[i] < a.pair_cap ? q0 + a.cnt[i] : a.pair_cap;
+      const int32_t n = end > q0 ? (int32_t)(end - q0) : 0;
+      a.nshort[i] = n < a.cnt[i] ? 0 : ns;
+      a.chunks[i] = n < a.cnt[i] ? 0 : (ns + 63) / 64 + (n - ns + 63) / 64;
+    }
+  }
   for (int32_t wb = 0; wb < words; wb += 64) {
-    const int32_t wl = wb + lane;
-    uint64_t m = wl < words ? mask[(int64_t)i * words + wl] : 0ull;
-    int32_t incl = __popcll(m);
+    const int32_t wl_ = wb + lane;
+    uint64_t m = wl_ < words ? a.mask[(int64_t)i * words + wl_] : 0ull;
+    const uint64_t sh = a.qshort && wl_ < words ? a.qshort[wl_] : 0ull;
+    int32_t incl = __popcll(m), sinc = __popcll(m & sh);
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const int32_t v = __shfl_up(incl, o);
-      if (lane >= o) incl += v;
+      const int32_t v = __shfl_up(incl, o), u = __shfl_up(sinc, o);
+      if (lane >= o) {
+        incl += v;
+        sinc += u;
+      }
     }
     int32_t pos = incl - __popcll(m);
+    int32_t sp = sinc - __popcll(m & sh), lp = pos - sp;
+    const uint64_t m0 = m;
     while (m) {
-      s_p[pos++] = wl * 64 + (__ffsll((long long)m) - 1);
+      s_p[pos++] = wl_ * 64 + (__ffsll((long long)m) - 1);
       m &= m - 1ull;
     }
     wave_lds_sync();
     const int32_t total = __builtin_amdgcn_readlane(incl, 63);
     for (int32_t k = lane; k < total; k += 64) {
       const int64_t q = q0 + k;
-      if (q < pair_cap) {
+      if (q < a.pair_cap) {
         const int32_t r = s_p[k];
-        pnode[q] = i;
-        if constexpr (kRow) pprim[q] = row[r];
-        else pprim[q] = r;
+        a.pnode[q] = i;
+        if constexpr (kRow) a.pprim[q] = row[r];
+        else a.pprim[q] = r;
       }
+    }
+    if (a.qshort) {
+      // the same bits again into the two groups
+      const int64_t first = q0 + incl - __popcll(m0);
+      int32_t k = 0;
+      for (m = m0; m; m &= m - 1ull, ++k) {
+        const int bit = __ffsll((long long)m) - 1;
+        const bool is_short = (sh >> bit) & 1ull;
+        const int64_t at = is_short ? ws + sp++ : wl + lp++;
+        if (at < a.pair_cap) a.qperm[at] = make_int2((int32_t)(first + k), wl_ * 64 + bit);
+      }
+      const int32_t st = __builtin_amdgcn_readlane(sinc, 63);
+      ws += st;
+      wl += total - st;
     }
     q0 += total;
     wave_lds_sync();
@@ -389,6 +471,7 @@ struct dp_check_args {
   int32_t* cont_count;
   int32_t* cont_cell;
   int32_t* cont_place;
+  dp_marks marks;
 };
 
 namespace {
@@ -493,6 +576,7 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
   __shared__ check_wave<NX> s_wave[kWaves];
   const dp_dev_sys& S = s_sys;
   const int nobs = a.nobs;
+  dp_mark(a.marks);
   // a.ppw 0: about 9 waves per CU over the batch's pairs, 4 to 64 pairs each
   int ppw = a.ppw;
   if (ppw == 0) {
@@ -873,6 +957,7 @@ __global__ __launch_bounds__(64) void k_select(dp_check_args a, const int32_t* _
                                                const double* __restrict__ targets, const double* __restrict__ cost,
                                                double cost_jump, int32_t choose_first, int32_t* __restrict__ sel_q,
                                                int32_t* __restrict__ sel_prim, double* __restrict__ sel) {
+  dp_mark(a.marks);
   const dp_dev_sys& S = *a.sys;
   const int32_t i = blockIdx.x;
   if (i >= N) return;
@@ -1032,31 +1117,31 @@ static void launch_app(dp_ctx* c, const app_bounds& B, double r_app, hipStream_t
   const double* keys = c->forward ? c->d_start : c->d_last;
   if (app_per_node_order(c)) {  // a pair order per node: one wave per node part
     k_app_count<NX><<<N * kAppParts, 64, 0, s>>>(c->d_sys, B, c->d_nodes, c->N_cap, N, keys, c->P, r_app, c->d_order,
-                                                 c->order_rows, c->d_app, c->d_app_mask);
+                                                 c->order_rows, c->d_app_cnt, c->d_app_mask);
     return;
   }
   const int32_t groups = (N + kAppNodes - 1) / kAppNodes;
   const int32_t parts = app_parts(c);
   const float* keys32 = c->forward ? c->d_start32 : c->d_last32;
   k_app_blk<NX><<<groups * parts, 64, 0, s>>>(c->d_sys, make_app_bounds32(c, r_app), c->d_nodes, c->N_cap, N, keys,
-                                              keys32, c->P, r_app, c->d_order, parts, c->d_app, c->d_app_mask);
+                                              keys32, c->P, r_app, c->d_order, parts, c->d_app_cnt, c->d_app_mask);
 }
 
 int dp_launch_count(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   const double r_app = app_radius(c, p);
   const int32_t N = c->N;
   const app_bounds B = make_app_bounds(c, r_app);
-  dp_fill_i32(c->d_app, N, 0, s);
+  dp_fill_i32(c->d_app_cnt, N, 0, s);
   return dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     launch_app<NX>(c, B, r_app, s);
-    dp_scan_small(c->d_app, N, c->d_total, c->pair_cap, c->d_counters, DPC_PAIRS, s);
+    dp_scan_small(c->d_app_cnt, c->d_app, N, c->d_total, c->pair_cap, c->d_counters, DPC_PAIRS, s);
     DP_HIP_RET(hipGetLastError());
     return DP_OK;
   });
 }
 
-// Stage events are skipped while a multi-instance graph is being captured.
+// Start and end events are skipped while a multi-instance graph is captured.
 #define DP_EV(ev_, s_) \
   do { \
     if (!c->no_events) DP_HIP_RET(hipEventRecord(ev_, s_)); \
@@ -1086,22 +1171,39 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   int rc = c->select_mode ? DP_OK : dp_ensure_cont_grid(c);
   if (rc) return rc;
   DP_EV(c->ev[0], s);
-  dp_begin(c->d_counters, c->d_app, N, c->d_cont_count, count ? c->grid.nslots : 0, s);
+  dp_begin(c->d_counters, c->d_app_cnt, N, c->d_cont_count, count ? c->grid.nslots : 0, dp_stage(c, 1u << 0), s);
   const app_bounds B = make_app_bounds(c, r_app);
   rc = dispatch_nx(nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     launch_app<NX>(c, B, r_app, s);
-    dp_scan_small(c->d_app, N, c->d_total, c->pair_cap, c->d_counters, DPC_PAIRS, s);
-    if (c->d_order)
-      k_app_fill<true><<<N, 64, 0, s>>>(N, c->P, c->d_app, c->d_app_mask, c->d_order, c->order_rows, c->d_pnode,
-                                        c->d_pprim, c->pair_cap);
-    else
-      k_app_fill<false><<<N, 64, 0, s>>>(N, c->P, c->d_app, c->d_app_mask, nullptr, 1, c->d_pnode, c->d_pprim,
-                                         c->pair_cap);
+    fill_args f{};
+    f.N = N;
+    f.P = c->P;
+    f.cnt = c->d_app_cnt;
+    f.app = c->d_app;
+    f.scan = N <= kFillScan ? 1 : 0;
+    f.mask = c->d_app_mask;
+    f.order = c->d_order;
+    f.rows = c->order_rows;
+    f.pnode = c->d_pnode;
+    f.pprim = c->d_pprim;
+    f.pair_cap = c->pair_cap;
+    f.total = c->d_total;
+    f.counters = c->d_counters;
+    // the FP32 pass's order needs the primitive of a mask bit: with a caller's
+    // order the pairs are split afterwards
+    if (NX == 13 && p->fp32_rollout && !c->d_order) {
+      f.qshort = c->d_qshort;
+      f.qperm = reinterpret_cast<int2*>(c->d_qperm);
+      f.nshort = c->d_nshort;
+      f.chunks = c->d_chunk;
+    }
+    if (!f.scan) dp_scan_small(c->d_app_cnt, c->d_app, N, c->d_total, c->pair_cap, c->d_counters, DPC_PAIRS, s);
+    if (c->d_order) k_app_fill<true><<<N, 64, 0, s>>>(f);
+    else k_app_fill<false><<<N, 64, 0, s>>>(f);
     return DP_OK;
   });
   if (rc) return rc;
-  DP_EV(c->ev[4], s);
   if (p->use_surrogate) {
     if (!c->mlp.w || (p->use_surrogate == 1 && !c->mlp.ready)) {
       dp_set_error("use_surrogate needs a trained and calibrated surrogate");
@@ -1114,8 +1216,6 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     rc = dp_launch_surrogate(c, p->use_surrogate == 1, s);
     if (rc) return rc;
   }
-  DP_EV(c->ev[1], s);
-
   dp_check_args a{};
   a.sys = c->d_sys;
   a.nodes = c->d_nodes;
@@ -1169,21 +1269,20 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   if (c->desc.system == DP_SYS_QUADROTOR) {
     rc = dp_launch_quad(c, p, goal_bound, r_dup, count, s);
     if (rc) return rc;
-    DP_EV(c->ev[2], s);
     rc = dp_launch_resolve(c, p, r_dup, count, s);
     if (rc) return rc;
-    DP_EV(c->ev[3], s);
+    DP_EV(c->ev[1], s);
     c->timing_valid = !c->no_events && !c->defer_walk;
     return DP_OK;
   }
   a.ppw = planar_pairs_per_wave(c);
+  a.marks = dp_stage(c, p->use_surrogate ? (1u << 1) | (1u << 5) : (1u << 4) | (1u << 1) | (1u << 5));
   // LDS: the obstacles plus one list of obstacles near a node per wave
   const size_t lds = (sizeof(double) * 4 + sizeof(int16_t) * kWaves) * (size_t)c->nb;
   // The pair count is on the device; size the grid from the bound N*P.
   const int32_t least = a.ppw > 0 ? a.ppw : 4;
   const int64_t groups = ((int64_t)N * c->P + least - 1) / least;
   const int blocks = dp_grid_blocks(groups, kWaves, c->tiles.check_blocks);
-  if ((rc = dp_record_event(c, 5, s))) return rc;
   rc = dispatch_nx(nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     if constexpr (NX == 13) {
@@ -1195,8 +1294,6 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   });
   if (rc) return rc;
   DP_HIP_RET(hipGetLastError());
-  DP_EV(c->ev[6], s);
-  DP_EV(c->ev[2], s);
 
   if (c->select_mode) {
     rc = dispatch_nx(nx, [&](auto NXc) -> int {
@@ -1204,6 +1301,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
       if constexpr (NX == 13) {
         return DP_ERR_ARG;
       } else {
+        a.marks = dp_stage(c, (1u << 6) | (1u << 2) | (1u << 7));
         k_select<NX><<<N, 64, 0, s>>>(a, c->d_app, N, c->d_targets, c->d_cost, c->select_cost_jump,
                                       c->select_first, c->d_sel_q, c->d_sel_q + c->sel_cap, c->d_sel);
         return DP_OK;
@@ -1211,14 +1309,13 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     });
     if (rc) return rc;
     DP_HIP_RET(hipGetLastError());
-    DP_EV(c->ev[7], s);
-    DP_EV(c->ev[3], s);
+    DP_EV(c->ev[1], s);
     c->timing_valid = !c->no_events && !c->defer_walk;
     return DP_OK;
   }
   rc = dp_launch_resolve(c, p, r_dup, count, s);
   if (rc) return rc;
-  DP_EV(c->ev[3], s);
+  DP_EV(c->ev[1], s);
   c->timing_valid = !c->no_events && !c->defer_walk;
   return DP_OK;
 }

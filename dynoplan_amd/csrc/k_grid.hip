@@ -120,7 +120,8 @@ constexpr int kRowWaves = 16;  // rows per workgroup
 template <bool kItems>
 __global__ __launch_bounds__(64 * kRowWaves) void k_cell_rows(dp_grid_geom G, int32_t* __restrict__ count,
                                                    int32_t* __restrict__ start, int32_t batch, int2* __restrict__ items,
-                                                   long long* __restrict__ counters) {
+                                                   long long* __restrict__ counters, dp_marks marks) {
+  dp_mark(marks);
   __shared__ int32_t s_sum[kRowWaves], s_items[kRowWaves];
   __shared__ unsigned long long s_base;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -701,7 +702,8 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
                                                    const int16_t* __restrict__ conf_cnt, int8_t* __restrict__ res,
                                                    int32_t limit, int32_t* __restrict__ cursor,
                                                    int32_t* __restrict__ count, int32_t* __restrict__ node_novel,
-                                                   long long* __restrict__ counters) {
+                                                   long long* __restrict__ counters, dp_marks marks) {
+  dp_mark(marks);
   // four nodes per workgroup, one per wave; the counts are summed in LDS and
   // added with one atomic per counter and workgroup (one per node, all at
   // the same moment, queued on the same few addresses)
@@ -784,7 +786,7 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
       cursor[node] = finished ? e : b;
       count[node] = finished ? c_nov : 0;
       if (node_novel) node_novel[node] = finished ? c_nov : 0;
-      if (b < e && !finished) atomicAdd((unsigned long long*)&s_add[0], 1ull);
+      if (b < e && !finished) atomicAdd((unsigned long long*)&s_add[0], 1ull);  // left to walk
       if (finished) {
         atomicAdd((unsigned long long*)&s_add[1], (unsigned long long)c_nov);
         atomicAdd((unsigned long long*)&s_add[2], (unsigned long long)c_cap);
@@ -794,7 +796,10 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    if (s_add[0]) atomicAdd((unsigned long long*)&counters[DPC_NODES_LEFT], (unsigned long long)s_add[0]);
+    if (s_add[0]) {
+      atomicAdd((unsigned long long*)&counters[DPC_NODES_LEFT], (unsigned long long)s_add[0]);
+      atomicAdd((unsigned long long*)&counters[DPC_WALK], (unsigned long long)s_add[0]);
+    }
     if (s_add[1]) atomicAdd((unsigned long long*)&counters[DPC_NOVEL], (unsigned long long)s_add[1]);
     if (s_add[2]) atomicAdd((unsigned long long*)&counters[DPC_CAPPED], (unsigned long long)s_add[2]);
     if (s_add[3]) atomicAdd((unsigned long long*)&counters[DPC_GOAL], (unsigned long long)s_add[3]);
@@ -805,7 +810,8 @@ __global__ __launch_bounds__(256) void k_pre_nodes(int32_t N, const int32_t* __r
 // are counted into DPC_NODES_LEFT, empty nodes are finished here.
 __global__ void k_round_init(int32_t N, const int32_t* __restrict__ app, const int32_t* __restrict__ total,
                              int32_t* __restrict__ cursor, int32_t* __restrict__ count,
-                             int32_t* __restrict__ node_novel, long long* counters) {
+                             int32_t* __restrict__ node_novel, long long* counters, dp_marks marks) {
+  dp_mark(marks);
   const int32_t tot = *total;
   for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
     const int32_t b = app[i] < tot ? app[i] : tot;
@@ -813,7 +819,10 @@ __global__ void k_round_init(int32_t N, const int32_t* __restrict__ app, const i
     cursor[i] = b;
     count[i] = 0;
     node_novel[i] = 0;
-    if (b < e) atomicAdd((unsigned long long*)&counters[DPC_NODES_LEFT], 1ull);
+    if (b < e) {
+      atomicAdd((unsigned long long*)&counters[DPC_NODES_LEFT], 1ull);
+      atomicAdd((unsigned long long*)&counters[DPC_WALK], 1ull);
+    }
   }
 }
 
@@ -1356,14 +1365,32 @@ __device__ void walk_node(const round_args& a, int32_t node) {
   if (a.trace && threadIdx.x == 0) a.trace[(int64_t)DP_TRACE_FIELDS * node + 1] = (unsigned long long)wall_clock64();
 }
 
+// A ticket covers a group of consecutive nodes, walked in order by its wave
+// (the nodes before them in the group are finished by then, those before the
+// group have smaller tickets): 1 node when most are left to walk, up to 16
+// where k_pre_nodes has finished nearly all.  Each ticket is an atomic on one
+// address (about 15 ns), and a wave that finds its node finished has still
+// paid a launch and two dependent loads: 2048 tickets of which 1% had a node
+// to walk took 55 us.
 template <int NX>
 __global__ __launch_bounds__(64) void k_resolve_ticketed(round_args a) {
-  __shared__ int32_t s_node;
-  if (threadIdx.x == 0) s_node = (int32_t)atomicAdd((unsigned long long*)&a.counters[DPC_TICKET], 1ull);
+  const int lane = threadIdx.x;
+  const long long left = a.counters[DPC_WALK];  // not changed by the walk
+  int32_t group = 1;
+  while (group < 16 && (long long)group * 4 * (left + 1) <= a.N) group *= 2;
+  if ((int64_t)blockIdx.x * group >= a.N) return;  // one workgroup per group takes a ticket
+  __shared__ int32_t s_t;
+  if (lane == 0) s_t = (int32_t)atomicAdd((unsigned long long*)&a.counters[DPC_TICKET], 1ull);
   __syncthreads();
-  const int32_t node = s_node;
-  if (node >= a.N) return;
-  walk_node<NX>(a, node);
+  const int32_t n0 = __builtin_amdgcn_readfirstlane(s_t) * group;
+  if (n0 >= a.N) return;
+  bool todo = false;
+  if (lane < group && n0 + lane < a.N) {
+    const int32_t tot = *a.total;
+    const int32_t end = a.app[n0 + lane + 1] < tot ? a.app[n0 + lane + 1] : tot;
+    todo = a.cursor[n0 + lane] < end;
+  }
+  for (uint64_t m = __ballot(todo); m; m &= m - 1ull) walk_node<NX>(a, n0 + __ffsll((long long)m) - 1);
 }
 
 // The ordered walks of many instances of one system in one launch.  Waves
@@ -1513,7 +1540,7 @@ int dp_launch_visited_rebuild(dp_ctx* c, double radius, hipStream_t s) {
       k_vis_count<NX><<<dp_grid_blocks(c->nv, 256, 8192), 256, 0, s>>>(c->grid, c->d_vis, c->nv_cap, c->nv,
                                                                       c->d_vis_cell, c->d_vis_rank, c->d_vis_count);
     k_cell_rows<false><<<cell_row_blocks(c->grid), 64 * kRowWaves, 0, s>>>(c->grid, c->d_vis_count, c->d_vis_start, 1, nullptr,
-                                                                c->d_counters);
+                                                                c->d_counters, dp_marks{nullptr, 0});
     if (c->nv > 0)
       k_vis_scatter<NX><<<dp_grid_blocks(c->nv, 256, 8192), 256, 0, s>>>(c->d_vis, c->nv_cap, c->nv, c->d_vis_cell,
                                                                         c->d_vis_rank, c->d_vis_start,
@@ -1557,7 +1584,8 @@ int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool c
     }
     int2* items = reinterpret_cast<int2*>(c->d_cont_item);
     k_cell_rows<true><<<cell_row_blocks(c->grid), 64 * kRowWaves, 0, s>>>(c->grid, c->d_cont_count, c->d_cont_start,
-                                                               64 * (NX == 13 ? 2 : 4), items, c->d_counters);
+                                                               64 * (NX == 13 ? 2 : 4), items, c->d_counters,
+                                                               dp_stage(c, NX == 13 ? 1u << 2 : (1u << 2) | (1u << 6)));
     // after the quadrotor's FP32 pass the FP64 list holds every contender
     if (counted && NX == 13 && p->fp32_rollout)
       k_cont_scatter_list<NX><<<dp_grid_blocks(c->pair_cap, 256, 1024), 256, 0, s>>>(
@@ -1571,14 +1599,14 @@ int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool c
     k_conf_waves<NX><<<(int)std::min<int64_t>((nc + 3) / 4, 8192), 256, 0, s>>>(
         c->d_sys, c->grid, c->d_cont_start, c->d_cont_x, items, r_dup, c->d_conf_cnt, c->d_conf, c->d_conf_ov,
         c->d_conf_pool, pool_cap, c->conf_slots, c->d_counters);
-    if (dp_record_event(c, 7, s)) return DP_ERR_HIP;
     if (p->limit_branching_factor > 0)
       k_pre_nodes<<<(N + 3) / 4, 256, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_conf_cnt,
                                                c->d_res, p->limit_branching_factor, c->d_node_cursor, c->d_node_count,
-                                               c->d_node_novel, c->d_counters);
+                                               c->d_node_novel, c->d_counters, dp_stage(c, 1u << 7));
     else
       k_round_init<<<dp_grid_blocks(N, 256, 1024), 256, 0, s>>>(N, c->d_app, c->d_total, c->d_node_cursor,
-                                                                c->d_node_count, c->d_node_novel, c->d_counters);
+                                                                c->d_node_count, c->d_node_novel, c->d_counters,
+                                                                dp_stage(c, 1u << 7));
     if (c->defer_walk) return DP_OK;  // a multi-instance batch walks every instance in one queue
     round_args ra = make_round_args(c);
     ra.wait = DP_WAIT_POLLS;
@@ -1602,7 +1630,7 @@ __global__ void k_reset_resolution(const int32_t* __restrict__ total, const int8
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int slots[] = {DPC_NOVEL, DPC_DUPV, DPC_DUPB, DPC_CAPPED, DPC_GOAL, DPC_NODES_LEFT, DPC_CONF,
-                         DPC_TICKET, DPC_SORTED, DPC_WINDOW_OVF, DPC_ROUNDS};
+                         DPC_TICKET, DPC_SORTED, DPC_WALK, DPC_WINDOW_OVF, DPC_ROUNDS};
     for (int k : slots) counters[k] = 0;
     counters[DPC_ERRFLAG] &= ~2ll;
   }
@@ -1751,7 +1779,7 @@ int dp_launch_visited_append_novel(dp_ctx* c, int64_t novel_total, hipStream_t s
   // Caller guarantees visited capacity >= nv + novel_total.
   const int32_t N = c->N;
   if (N <= 0 || novel_total <= 0) return DP_OK;
-  dp_scan_small(c->d_node_novel, N, nullptr, INT64_MAX, c->d_counters, -1, s);
+  dp_scan_small(c->d_node_novel, c->d_node_novel, N, nullptr, INT64_MAX, c->d_counters, -1, s);
   int rc = dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
     k_gather_novel<NX><<<N, 64, 0, s>>>(N, c->d_app, c->d_total, c->d_res, c->d_node_novel, c->d_final,

@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void k_gemm(gemm_args g) {
 // in an obstacle box (planar AABBs), else 0.  One workgroup per node.
 __global__ __launch_bounds__(256) void k_patch(const double* __restrict__ nodes, int32_t Ncap, int32_t N,
                                                const double* __restrict__ obs, int32_t nobs, double cell,
-                                               uint16_t* __restrict__ patch) {
+                                               uint16_t* __restrict__ patch, dp_marks marks) {
+  dp_mark(marks);
   // Obstacles that can contain a cell centre of this patch go to LDS first
   // (a superset: the exact per-cell test below decides).
   __shared__ double cand[4 * DP_MAX_OBS];
@@ -550,7 +551,7 @@ static int patches_and_node_terms(dp_ctx* c, hipStream_t s) {
   int rc;
   if ((rc = ensure_u16(&m.patch, &m.patch_cap, (int64_t)c->N_cap * 1024))) return rc;
   if ((rc = ensure_f32(&m.An, &m.An_cap, (int64_t)c->N_cap * 256))) return rc;
-  k_patch<<<c->N, 256, 0, s>>>(c->d_nodes, c->N_cap, c->N, c->d_obs, c->nb, 0.1, m.patch);
+  k_patch<<<c->N, 256, 0, s>>>(c->d_nodes, c->N_cap, c->N, c->d_obs, c->nb, 0.1, m.patch, dp_stage(c, 1u << 4));
   // A_i = W1[:, :1024] patch_i
   gemm(s, m.patch, 1024, 1, m.wb + L.W1, 1, 1088, m.An, 256, nullptr, nullptr, c->N, 256, 1024, false, false);
   DP_HIP_RET(hipGetLastError());
@@ -679,7 +680,7 @@ int dp_surrogate_train(dp_ctx* c, const double* nodes, int32_t N, const dp_expan
   }
   // occupancy patches of the training nodes
   if ((rc = ensure_u16(&m.patch, &m.patch_cap, (int64_t)c->N_cap * 1024))) return rc;
-  k_patch<<<c->N, 256, 0, s>>>(c->d_nodes, c->N_cap, c->N, c->d_obs, c->nb, 0.1, m.patch);
+  k_patch<<<c->N, 256, 0, s>>>(c->d_nodes, c->N_cap, c->N, c->d_obs, c->nb, 0.1, m.patch, dp_marks{nullptr, 0});
   if ((rc = ensure_u16(&m.xb, &m.xb_cap, (int64_t)batch * 1088))) return rc;
   if ((rc = dp_ensure_i32(&m.sid, &m.sid_cap, batch))) return rc;
   if (!m.loss) {

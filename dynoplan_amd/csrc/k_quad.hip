@@ -105,6 +105,7 @@ struct dp_quad_args {
   int32_t* cont_cell;
   int32_t* cont_place;
   long long* counters;
+  dp_marks marks;
 };
 
 namespace {
@@ -334,6 +335,7 @@ __device__ __forceinline__ void quad32_start(const dp_quad_args& a, int32_t j, c
 }
 
 __global__ __launch_bounds__(256) void k_quad32(dp_quad_args a) {
+  dp_mark(a.marks);
   extern __shared__ float qsm[];
   const dp_dev_sys& S = *a.sys;
   // the wave index is uniform: in a scalar register, every per-chunk value
@@ -744,6 +746,7 @@ __global__ __launch_bounds__(256) void k_quad64(dp_quad_args a) {
   // per-lane candidate lists [blockDim.x][kQ64Cand]
   extern __shared__ double q64_lds[];
   const dp_dev_sys& S = *a.sys;
+  dp_mark(a.marks);
   const int64_t n64 = quad64_count(a);
   if ((int64_t)blockIdx.x * blockDim.x >= n64) return;  // uniform per block
   const int nobs_d = 6 * a.nb + 4 * a.ns;
@@ -993,15 +996,14 @@ __global__ __launch_bounds__(256) void k_quad64(dp_quad_args a) {
   }
 }
 
-// Per node: its pairs reordered for the FP32 pass, those whose primitive
-// leaves the attitude / rate bounds within its length first (their verdict
-// is BOUNDS whatever the translation, so their rollouts are short and need
-// no collision test), then the rest, each group in canonical order (the
-// results are written nearly in order); and the node's wave chunks (64
-// pairs, one group per chunk).  One wave per node.
+// The FP32 pass's order for a batch with a caller's pair order (without one,
+// k_app_fill writes it): per node, its pairs whose primitive leaves the
+// attitude / rate bounds first, then the rest, each group in the batch's
+// order, and the node's wave chunks (64 pairs, one group per chunk).  One
+// wave per node.
 __global__ __launch_bounds__(64) void k_quad_split(int32_t N, const int32_t* __restrict__ app,
                                                    const int32_t* __restrict__ total, const int32_t* __restrict__ pprim,
-                                                   const int32_t* __restrict__ off, const int32_t* __restrict__ rbad32,
+                                                   const uint64_t* __restrict__ qshort,
                                                    int2* __restrict__ qperm, int32_t* __restrict__ nshort,
                                                    int32_t* __restrict__ chunks) {
   const int32_t node = blockIdx.x;
@@ -1011,25 +1013,17 @@ __global__ __launch_bounds__(64) void k_quad_split(int32_t N, const int32_t* __r
   const int32_t tot = *total;
   const int32_t b = app[node] < tot ? app[node] : tot;
   const int32_t e = app[node + 1] < tot ? app[node + 1] : tot;
+  auto is_short = [&](int32_t j) { return ((qshort[j >> 6] >> (j & 63)) & 1ull) != 0; };
   int32_t ns = 0;
   for (int32_t cb = b; cb < e; cb += 64) {
     const int32_t p = cb + lane;
-    bool sh = false;
-    if (p < e) {
-      const int32_t j = pprim[p];
-      sh = rbad32[j] < off[j + 1] - off[j];
-    }
-    ns += __popcll(__ballot(sh));
+    ns += __popcll(__ballot(p < e && is_short(pprim[p])));
   }
   int32_t ws = b, wl = b + ns;
   for (int32_t cb = b; cb < e; cb += 64) {
     const int32_t p = cb + lane;
-    bool sh = false;
-    int32_t j = 0;
-    if (p < e) {
-      j = pprim[p];
-      sh = rbad32[j] < off[j + 1] - off[j];
-    }
+    const int32_t j = p < e ? pprim[p] : 0;
+    const bool sh = p < e && is_short(j);
     const uint64_t ms = __ballot(sh), ml = __ballot(p < e && !sh);
     if (p < e) qperm[sh ? ws + __popcll(ms & lt) : wl + __popcll(ml & lt)] = make_int2(p, j);
     ws += __popcll(ms);
@@ -1041,10 +1035,45 @@ __global__ __launch_bounds__(64) void k_quad_split(int32_t N, const int32_t* __r
   }
 }
 
-// Node of every wave chunk (after the scan of the chunk counts).
-__global__ void k_quad_chunk_nodes(int32_t N, const int32_t* __restrict__ chunk_off, int32_t* __restrict__ chunk_node) {
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x)
-    for (int32_t w = chunk_off[i]; w < chunk_off[i + 1]; ++w) chunk_node[w] = i;
+// Chunk counts per node to offsets, and the node of every wave chunk: one
+// workgroup, 1024 nodes at a time, each thread writing its node's chunks
+// (two launches, a scan and this, took 9 us with the gap between them).
+__global__ __launch_bounds__(1024) void k_quad_chunks(int32_t N, int32_t* __restrict__ chunk,
+                                                      int32_t* __restrict__ chunk_node, dp_marks marks) {
+  dp_mark(marks);
+  __shared__ int32_t s[16];
+  const int t = threadIdx.x, lane = t % 64;
+  int32_t base = 0;
+  for (int32_t n0 = 0; n0 < N; n0 += 1024) {
+    const int32_t i = n0 + t;
+    const int32_t v = i < N ? chunk[i] : 0;
+    int32_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t u = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += u;
+    }
+    if (lane == 63) s[t / 64] = incl;
+    __syncthreads();
+    int32_t off = base + incl - v;
+    for (int k = 0; k < t / 64; ++k) off += s[k];
+    for (int k = 0; k < 16; ++k) base += s[k];
+    if (i < N) {
+      chunk[i] = off;
+      for (int32_t k = 0; k < v; ++k) chunk_node[off + k] = i;
+    }
+    __syncthreads();
+  }
+  if (t == 0) chunk[N] = base;
+}
+
+// One bit per primitive: its attitude / rate leaves the bounds (FP32 rollout).
+__global__ void k_quad_short(int32_t P, const int32_t* __restrict__ off, const int32_t* __restrict__ rbad32,
+                             uint64_t* __restrict__ qshort) {
+  for (int32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < (P + 63) / 64 * 64; j += gridDim.x * blockDim.x) {
+    const uint64_t m = __ballot(j < P && rbad32[j < P ? j : 0] < off[j < P ? j + 1 : 1] - off[j < P ? j : 0]);
+    if (threadIdx.x % 64 == 0) qshort[j / 64] = m;
+  }
 }
 
 // FP64 window of each node: the pairs the FP32 pass found FREE are ranked in
@@ -1065,7 +1094,9 @@ __global__ __launch_bounds__(256) void k_quad_window(int32_t N, const int32_t* _
                                                      int32_t* __restrict__ firstk, int32_t* __restrict__ goal_out,
                                                      int8_t* __restrict__ res, int8_t* __restrict__ flags,
                                                      int32_t window, int32_t fixed, int32_t* __restrict__ wshift,
-                                                     int32_t* __restrict__ q64, long long* __restrict__ counters) {
+                                                     int32_t* __restrict__ q64, long long* __restrict__ counters,
+                                                     dp_marks marks) {
+  dp_mark(marks);
   // four nodes per workgroup, one per wave: their places in the compact list
   // are reserved with one atomic per workgroup (one per node, all issued
   // together on one address, queue behind each other)
@@ -1274,6 +1305,7 @@ int dp_launch_quad_rot(dp_ctx* c, hipStream_t s) {
                                                            c->d_act32, c->d_rot64, c->d_dv64, c->d_dv32, c->d_rbad64,
                                                            c->d_rbad32, c->d_rnear32, c->d_preach,
                                                            reinterpret_cast<quad_rec*>(c->d_qrec));
+  k_quad_short<<<dp_grid_blocks(c->P, 256, 1024), 256, 0, s>>>(c->P, c->d_off, c->d_rbad32, c->d_qshort);
   DP_HIP_RET(hipGetLastError());
   return DP_OK;
 }
@@ -1342,25 +1374,22 @@ int dp_launch_quad(dp_ctx* c, const dp_expand_params* p, double goal_bound, doub
       dp_set_error("too many obstacles for the FP32 quadrotor staging (max 64 KiB LDS per workgroup)");
       return DP_ERR_ARG;
     }
-    k_quad_split<<<c->N, 64, 0, s>>>(c->N, c->d_app, c->d_total, c->d_pprim, c->d_off, c->d_rbad32,
-                                     reinterpret_cast<int2*>(c->d_qperm),
-                                     c->d_nshort, c->d_chunk);
-    dp_scan_small(c->d_chunk, c->N, nullptr, INT64_MAX, c->d_counters, -1, s);
-    k_quad_chunk_nodes<<<dp_grid_blocks(c->N, 256, 1024), 256, 0, s>>>(c->N, c->d_chunk, c->d_chunk_node);
+    if (c->d_order)  // else k_app_fill has written the order
+      k_quad_split<<<c->N, 64, 0, s>>>(c->N, c->d_app, c->d_total, c->d_pprim, c->d_qshort,
+                                       reinterpret_cast<int2*>(c->d_qperm), c->d_nshort, c->d_chunk);
+    k_quad_chunks<<<1, 1024, 0, s>>>(c->N, c->d_chunk, c->d_chunk_node, dp_stage(c, (1u << 4) | (1u << 1)));
     const int64_t max_chunks = (int64_t)c->N * ((c->P + 63) / 64);
-    int rc = dp_record_event(c, 5, s);
-    if (rc) return rc;
+    a.marks = dp_stage(c, 1u << 5);
     k_quad32<<<dp_grid_blocks(max_chunks, kQWaves, c->tiles.quad32_blocks), 256, lds, s>>>(a);
-    if ((rc = dp_record_event(c, 6, s))) return rc;
+    a.marks = dp_marks{nullptr, 0};
     const int32_t window = dp_fp64_window(c, p->limit_branching_factor);
     const int32_t fixed = c->fp64_window > 0 || p->limit_branching_factor < 0 ? 1 : 0;
     if (c->N > 0)
       k_quad_window<<<(c->N + 3) / 4, 256, 0, s>>>(c->N, c->d_app, c->d_total, c->d_verdict, c->d_firstk, c->d_goal, c->d_res,
-                                        c->d_flags, window, fixed, c->d_wshift, c->d_q64, c->d_counters);
+                                        c->d_flags, window, fixed, c->d_wshift, c->d_q64, c->d_counters,
+                                        dp_stage(c, 1u << 6));
   } else {
-    int rc = dp_record_event(c, 5, s);
-    if (!rc) rc = dp_record_event(c, 6, s);
-    if (rc) return rc;
+    a.marks = dp_stage(c, (1u << 4) | (1u << 1) | (1u << 5) | (1u << 6));
   }
   const int t64 = c->tiles.quad64_threads;
   k_quad64<<<dp_grid_blocks(c->pair_cap, t64, c->tiles.quad64_blocks), t64, quad64_lds(c, t64), s>>>(a);

@@ -13,7 +13,8 @@ __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
 }
 
 __global__ void k_begin(long long* __restrict__ counters, int n, int32_t* __restrict__ a, int64_t na,
-                        int32_t* __restrict__ b, int64_t nb) {
+                        int32_t* __restrict__ b, int64_t nb, dp_marks marks) {
+  dp_mark(marks);
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
   if (t0 < n) counters[t0] = 0;
   for (int64_t t = t0; t < na; t += step) a[t] = 0;
@@ -23,15 +24,15 @@ __global__ void k_begin(long long* __restrict__ counters, int n, int32_t* __rest
 // One workgroup, each thread a contiguous chunk: the chunk sums scanned with
 // wave shuffles and one exchange of the 16 wave sums (a step-by-step scan
 // of 1024 sums in LDS paid 20 barriers, 4.7 us at 4096 elements against 3.0).
-__global__ __launch_bounds__(1024) void k_scan_small(int32_t* data, int64_t n, int32_t* total, int64_t cap,
-                                                     long long* counters, int slot) {
+__global__ __launch_bounds__(1024) void k_scan_small(const int32_t* src, int32_t* dst, int64_t n,
+                                                     int32_t* total, int64_t cap, long long* counters, int slot) {
   __shared__ long long s[16];
   const int t = threadIdx.x, lane = t % 64;
   const int64_t chunk = (n + 1023) / 1024;
   const int64_t b = t * chunk;
   const int64_t e = b + chunk < n ? b + chunk : n;
   long long sum = 0;
-  for (int64_t k = b; k < e; ++k) sum += data[k];
+  for (int64_t k = b; k < e; ++k) sum += src[k];
   long long incl = sum;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -43,13 +44,13 @@ __global__ __launch_bounds__(1024) void k_scan_small(int32_t* data, int64_t n, i
   long long run = incl - sum;
   for (int k = 0; k < t / 64; ++k) run += s[k];
   for (int64_t k = b; k < e; ++k) {
-    int32_t v = data[k];
-    data[k] = (int32_t)run;
+    int32_t v = src[k];
+    dst[k] = (int32_t)run;
     run += v;
   }
   if (t == 1023) {
     long long tot = run;  // thread 1023 owns the last chunk
-    data[n] = (int32_t)tot;
+    dst[n] = (int32_t)tot;
     if (total) *total = (int32_t)(tot < cap ? tot : cap);
     if (slot >= 0) counters[slot] = tot;
     if (tot > cap) counters[DPC_OVERFLOW] = 1;
@@ -63,13 +64,13 @@ void dp_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s) {
   k_fill_i32<<<dp_grid_blocks(n, 256, 4096), 256, 0, s>>>(p, n, v);
 }
 
-void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t nb, hipStream_t s) {
-  k_begin<<<dp_grid_blocks(na + nb, 256, 2048), 256, 0, s>>>(counters, DPC_COUNT, a, na, b, nb);
+void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t nb, dp_marks marks, hipStream_t s) {
+  k_begin<<<dp_grid_blocks(na + nb, 256, 2048), 256, 0, s>>>(counters, DPC_COUNT, a, na, b, nb, marks);
 }
 
-void dp_scan_small(int32_t* data, int64_t n, int32_t* total, int64_t cap, long long* counters, int slot,
-                   hipStream_t s) {
-  k_scan_small<<<1, 1024, 0, s>>>(data, n, total, cap, counters, slot);
+void dp_scan_small(const int32_t* src, int32_t* dst, int64_t n, int32_t* total, int64_t cap, long long* counters,
+                   int slot, hipStream_t s) {
+  k_scan_small<<<1, 1024, 0, s>>>(src, dst, n, total, cap, counters, slot);
 }
 
 // Growth frees a buffer earlier kernels of the batch may still read, so the
