@@ -848,6 +848,7 @@ struct round_args {
   int32_t* count;
   int32_t* node_novel;
   int32_t limit;
+  int32_t precap;    // limit 0: FREE pairs after a node's first were CAPPED before the walk
   int32_t slots;     // inline conflict slots in use (<= DP_CONF_SLOTS)
   int32_t wait;      // polls a lane may spend on one undecided earlier contender
   int32_t poll_cap;  // longest pause between polls, in 64-cycle sleeps
@@ -871,15 +872,31 @@ __device__ __forceinline__ void poll_pause(int32_t w, int32_t cap) {
 // true when the node is finished.  Executed by one whole wave.
 // cur / count are wave-uniform registers carried across retries; they are
 // also stored for the round kernel, which reloads them in a later launch.
+//
+// Planar systems (most pairs FREE) walk 64 consecutive pairs at a time, the
+// next chunk's inputs loaded while a chunk is decided: the critical path of a
+// batch is a chain through nodes that walk all their chunks, so a chunk's
+// latency counts (4.7 us; from the queue below 8.3, and 1.25 -> 1.6 ms for the
+// walk of 4096 unicycle1 nodes).
+//
+// The quadrotor's pairs are mostly not FREE (4% of 550 per node): there the
+// FREE pairs are taken from a queue in LDS, filled from 256 pairs per step, so
+// a node is one chunk instead of nine (walk of 2048 nodes 55 -> 24 us).
+constexpr int kWalkQueue = 64 + 256;
+
 template <int NX>
-__device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, int32_t& count) {
+__device__ __forceinline__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, int32_t& count) {
   // per chunk: same-chunk contender masks, undecided-entry masks, flags
   // (1: an earlier contender is NOVEL, 2: an entry past the 64th is
   // undecided), exclusive scan of list lengths, overflow offsets
   __shared__ unsigned long long s_same[64], s_undec[64];
   __shared__ int32_t s_pre[64], s_ov[64], s_flag[64];
+  // FREE pairs not yet walked, ascending, and their flags
+  __shared__ int32_t s_q[kWalkQueue];
+  __shared__ int8_t s_qf[kWalkQueue];
   constexpr int kCoop = 16;  // list entries per lane in flight
   const int lane = threadIdx.x & 63;
+  const uint64_t lt = (1ull << lane) - 1ull, lane_bit = 1ull << lane;
   const int32_t tot = *a.total;
   const int32_t end = a.app[node + 1] < tot ? a.app[node + 1] : tot;
   if (cur >= end) return true;
@@ -889,59 +906,187 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
   // in-chunk walk, cycles waiting, chunks, waits, polls
   unsigned long long tr_eval = 0, tr_walk = 0, tr_wait = 0, tr_chunks = 0, tr_waits = 0, tr_polls = 0;
   bool stopped = false;
-  // per-pair inputs of a chunk (verdict, flags, list length, overflow
-  // offset) are loaded together, and those of the next chunk while this one
-  // is decided; the values of pairs that are not contenders go unused
+  constexpr bool kSparse = NX == 13;
+  int32_t pos = cur;  // first pair not yet walked
+  int qn = 0;
+  int32_t scan = cur;  // next pair to look at for the queue
+  // dense: inputs of the next chunk (the values of pairs that are not
+  // contenders go unused)
   int8_t m_vd = -1, m_fl = 0;
   int16_t m_cc = 0;
   int32_t m_ov = 0;
-  if (cur + lane < end) {
-    m_vd = a.verdict[cur + lane];
-    m_fl = a.flags[cur + lane];
-    m_cc = a.conf_cnt[cur + lane];
-    m_ov = a.conf_ov[cur + lane];
-  }
-  for (int32_t cb = cur; cb < end; cb += 64) {
-    const int32_t p = cb + lane;
-    const int8_t vd_p = m_vd, fl_p = m_fl;
-    const int16_t cc_p = m_cc;
-    const int32_t ov_p = m_ov;
+  auto fetch = [&](int32_t p) {
     m_vd = -1;
-    if (p + 64 < end) {
-      m_vd = a.verdict[p + 64];
-      m_fl = a.flags[p + 64];
-      m_cc = a.conf_cnt[p + 64];
-      m_ov = a.conf_ov[p + 64];
+    if (p < end) {
+      m_vd = a.verdict[p];
+      m_fl = a.flags[p];
+      m_cc = a.conf_cnt[p];
+      m_ov = a.conf_ov[p];
     }
-    // FREE pairs capped before the walk (limit 0) are not walked
-    const bool pre = p < end && vd_p == DP_V_FREE && (fl_p & DP_F_PRECAP);
-    const bool fr = p < end && vd_p == DP_V_FREE && !pre;
-    n_cap += __popcll(__ballot(pre));
-    if (a.limit > 0 && count >= a.limit) {
-      // The reference has left this node's loop: every later FREE pair is
-      // capped.  Other nodes may be waiting for any of them, so the whole
-      // tail is published in one pass with its verdict loads in flight
-      // together, not chunk by chunk.
-      if (fr) __hip_atomic_store(&a.res[p], (int8_t)DP_R_CAPPED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      n_cap += __popcll(__ballot(fr));
-      for (int32_t t0 = cb + 64; t0 < end; t0 += 64 * 8) {
-        bool f8[8];
+  };
+  if constexpr (!kSparse) fetch(cur + lane);
+  auto put = [&](int32_t p, int r) {
+    __hip_atomic_store(&a.res[p], (int8_t)r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  [[maybe_unused]] auto refill = [&](int want) {
+    while (qn < want && scan < end) {
+      int8_t v4[4], f4[4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int32_t t = t0 + 64 * k + lane;
-          f8[k] = t < end && a.verdict[t] == DP_V_FREE && !(a.flags[t] & DP_F_PRECAP);
+      for (int u = 0; u < 4; ++u) {
+        const int32_t p = scan + 64 * u + lane < end ? scan + 64 * u + lane : end - 1;
+        v4[u] = a.verdict[p];
+        f4[u] = a.flags[p];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int32_t p = scan + 64 * u + lane;
+        // FREE pairs capped before the walk (limit 0) are not walked
+        const bool fr = p < end && v4[u] == DP_V_FREE && !(f4[u] & DP_F_PRECAP);
+        const uint64_t m = __ballot(fr);
+        if (fr) {
+          s_q[qn + __popcll(m & lt)] = p;
+          s_qf[qn + __popcll(m & lt)] = f4[u];
         }
+        qn += __popcll(m);
+      }
+      scan += 256;
+    }
+    __syncthreads();
+  };
+  // The reference has left this node's loop: every FREE pair from `from` on is
+  // capped.  Other nodes may be waiting for any of them, so all are published
+  // in one pass with their verdict loads in flight together.
+  auto cap_tail = [&](int32_t from) -> long long {
+    long long n = 0;
+    for (int32_t t0 = from; t0 < end; t0 += 64 * 8) {
+      bool f8[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          if (f8[k])
-            __hip_atomic_store(&a.res[t0 + 64 * k + lane], (int8_t)DP_R_CAPPED, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-          n_cap += __popcll(__ballot(f8[k]));
+      for (int k = 0; k < 8; ++k) {
+        const int32_t t = t0 + 64 * k + lane < end ? t0 + 64 * k + lane : end - 1;
+        f8[k] = a.verdict[t] == DP_V_FREE && !(a.flags[t] & DP_F_PRECAP);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const bool f = f8[k] && t0 + 64 * k + lane < end;
+        if (f) put(t0 + 64 * k + lane, DP_R_CAPPED);
+        n += __popcll(__ballot(f));
+      }
+    }
+    return n;
+  };
+  // Place in the chunk of the n pairs from `first` on of its pair o.
+  auto place = [&](int32_t o, int32_t first, int n) -> int {
+    if constexpr (!kSparse) return o - first;
+    int l = 0;
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1)
+      if (l + st < n && s_q[l + st] <= o) l += st;
+    return l;
+  };
+  // Stored lists of the chunk's n pairs, evaluated by the whole wave:
+  // the entries are numbered consecutively over the pairs (exclusive scan of
+  // the counts) and lane l takes entries l, l+64, ..., so a long list costs
+  // no more than its share.  Plain (cached) loads suffice: a decided verdict
+  // never changes, and a stale "undecided" is polled coherently later.
+  auto eval_lists = [&](int32_t first, int n, int cnt, int32_t ov, uint64_t& same, uint64_t& undec, bool& dup,
+                        bool& more) {
+    const int n_l = cnt > 0 ? cnt : 0;
+    int incl = n_l;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    const int total_e = __shfl(incl, 63, 64);
+    s_pre[lane] = incl - n_l;
+    s_ov[lane] = n_l > a.slots ? ov : 0;
+    s_same[lane] = 0;
+    s_undec[lane] = 0;
+    s_flag[lane] = 0;
+    __syncthreads();
+    for (int f0 = 0; f0 < total_e; f0 += 64 * kCoop) {
+      int32_t os[kCoop];
+      int rs[kCoop], oe[kCoop];  // oe: owner lane << 16 | entry index, or -1
+#pragma unroll
+      for (int k = 0; k < kCoop; ++k) {
+        const int f = f0 + 64 * k + lane;
+        oe[k] = -1;
+        os[k] = INT32_MAX;
+        if (f < total_e) {
+          int lo = 0;
+#pragma unroll
+          for (int st = 32; st > 0; st >>= 1)  // lo + st <= 63
+            if (s_pre[lo + st] <= f) lo += st;
+          const int e = f - s_pre[lo];  // < DP_CONF_MAX
+          oe[k] = (lo << 16) | e;
+          const int32_t q = kSparse ? s_q[lo] : first + lo;
+          os[k] = e < a.slots ? a.conf[(int64_t)q * DP_CONF_SLOTS + e] : a.pool[(int64_t)s_ov[lo] + (e - a.slots)];
         }
       }
+#pragma unroll
+      for (int k = 0; k < kCoop; ++k) rs[k] = os[k] < first ? a.res[os[k]] : (int)DP_R_NONE;
+#pragma unroll
+      for (int k = 0; k < kCoop; ++k) {
+        if (oe[k] < 0) continue;
+        const int own = oe[k] >> 16, ee = oe[k] & 0xffff;
+        if (os[k] >= first) {  // a pair of this chunk: its place in it
+          atomicOr(&s_same[own], 1ull << place(os[k], first, n));
+        } else if (rs[k] == DP_R_NOVEL) {
+          atomicOr(&s_flag[own], 1);
+        } else if (rs[k] == DP_R_UNDECIDED) {
+          if (ee < 64) atomicOr(&s_undec[own], 1ull << ee);
+          else atomicOr(&s_flag[own], 2);
+        }
+      }
+    }
+    __syncthreads();
+    if (cnt > 0) {
+      same = s_same[lane];
+      undec = s_undec[lane];
+      dup = (s_flag[lane] & 1) != 0;
+      more = (s_flag[lane] & 2) != 0;
+    }
+    __syncthreads();  // the arrays are rewritten by the next chunk
+  };
+  // lanes up to and including the k-th set bit of m (m has at least k)
+  auto upto_kth = [&](uint64_t m, int k) -> uint64_t {
+    for (int t = 1; t < k; ++t) m &= m - 1ull;
+    const int c = __ffsll((long long)m) - 1;
+    return c >= 63 ? ~0ull : ((2ull << c) - 1ull);
+  };
+  for (;;) {
+    if (a.limit > 0 && count >= a.limit) {
+      n_cap += cap_tail(pos);
       break;
     }
-    const int8_t fl = fr ? fl_p : 0;
+    int n = 64;
+    bool fr;
+    int32_t p, first, ov_p;
+    int8_t fl;
+    int16_t cc_p;
+    if constexpr (kSparse) {
+      refill(64);
+      if (qn == 0) break;
+      n = qn < 64 ? qn : 64;
+      fr = lane < n;
+      first = s_q[0];
+      p = s_q[fr ? lane : 0];
+      fl = fr ? s_qf[lane] : (int8_t)0;
+      cc_p = a.conf_cnt[p];
+      ov_p = a.conf_ov[p];
+      pos = s_q[n - 1] + 1;
+    } else {
+      if (pos >= end) break;
+      first = pos;
+      p = first + lane;
+      // FREE pairs capped before the walk (limit 0) are not walked
+      fr = p < end && m_vd == DP_V_FREE && !(m_fl & DP_F_PRECAP);
+      fl = fr ? m_fl : (int8_t)0;
+      cc_p = m_cc;
+      ov_p = m_ov;
+      pos += 64;
+      fetch(p + 64);
+    }
     const bool forced = (fl & 2) != 0;
     const bool dupv = (fl & 1) != 0;
     // past the node's FP64 window: no final state, so it blocks the walk for
@@ -967,8 +1112,8 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
     // earlier node, whose wave is resident in persistent mode).
     auto eval = [&](int32_t p, int32_t polls) {
       auto visit = [&](int32_t o) {
-        if (o >= cb) {
-          same |= 1ull << (o - cb);
+        if (o >= first) {
+          same |= 1ull << place(o, first, n);
           return true;
         }
         int r = polls == 0 ? a.res[o] : __hip_atomic_load(&a.res[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -992,79 +1137,15 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
 #pragma unroll
       for (int k = 0; k < NX; ++k) x[k] = a.fin[(int64_t)k * a.pcap + p];
       scan_earlier<NX>(*a.sys, a.grid, a.cstart, a.cx, x, p, a.r_dup, visit, [&](int32_t o) {
-        if (o >= cb) return true;
+        if (o >= first) return true;
         const int v = a.res[o];
         return v == DP_R_NOVEL || v == DP_R_UNDECIDED;
       });
     };
     const unsigned long long t_eval = a.trace ? (unsigned long long)wall_clock64() : 0ull;
     const int cnt = fr && !forced && !dupv && !deferred ? cc_p : 0;
-    {
-      // Stored lists of the chunk's 64 pairs, evaluated by the whole wave:
-      // the entries are numbered consecutively over the pairs (exclusive
-      // scan of the counts) and lane l takes entries l, l+64, ..., so a long
-      // list costs no more than its share.  Plain (cached) loads suffice: a
-      // decided verdict never changes, and a stale "undecided" is polled
-      // coherently later.
-      const int n_l = cnt > 0 ? cnt : 0;
-      int incl = n_l;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += v;
-      }
-      const int total_e = __shfl(incl, 63, 64);
-      s_pre[lane] = incl - n_l;
-      s_ov[lane] = n_l > a.slots ? ov_p : 0;
-      s_same[lane] = 0;
-      s_undec[lane] = 0;
-      s_flag[lane] = 0;
-      __syncthreads();
-      for (int f0 = 0; f0 < total_e; f0 += 64 * kCoop) {
-        int32_t os[kCoop];
-        int rs[kCoop], oe[kCoop];  // oe: owner lane << 16 | entry index, or -1
-#pragma unroll
-        for (int k = 0; k < kCoop; ++k) {
-          const int f = f0 + 64 * k + lane;
-          oe[k] = -1;
-          os[k] = INT32_MAX;
-          if (f < total_e) {
-            int lo = 0;
-#pragma unroll
-            for (int st = 32; st > 0; st >>= 1)  // lo + st <= 63
-              if (s_pre[lo + st] <= f) lo += st;
-            const int e = f - s_pre[lo];  // < DP_CONF_MAX
-            oe[k] = (lo << 16) | e;
-            const int32_t q = cb + lo;
-            os[k] = e < a.slots ? a.conf[(int64_t)q * DP_CONF_SLOTS + e] : a.pool[(int64_t)s_ov[lo] + (e - a.slots)];
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < kCoop; ++k) rs[k] = os[k] < cb ? a.res[os[k]] : (int)DP_R_NONE;
-#pragma unroll
-        for (int k = 0; k < kCoop; ++k) {
-          if (oe[k] < 0) continue;
-          const int own = oe[k] >> 16, ee = oe[k] & 0xffff;
-          if (os[k] >= cb) {
-            atomicOr(&s_same[own], 1ull << (os[k] - cb));
-          } else if (rs[k] == DP_R_NOVEL) {
-            atomicOr(&s_flag[own], 1);
-          } else if (rs[k] == DP_R_UNDECIDED) {
-            if (ee < 64) atomicOr(&s_undec[own], 1ull << ee);
-            else atomicOr(&s_flag[own], 2);
-          }
-        }
-      }
-      __syncthreads();
-      if (cnt > 0) {
-        same = s_same[lane];
-        undec = s_undec[lane];
-        ext_dup = (s_flag[lane] & 1) != 0;
-        more = (s_flag[lane] & 2) != 0;
-        ext_block = !ext_dup && (undec != 0 || more);
-      }
-      __syncthreads();  // the arrays are rewritten by the next chunk
-    }
+    eval_lists(first, n, cnt, ov_p, same, undec, ext_dup, more);
+    if (cnt > 0) ext_block = !ext_dup && (undec != 0 || more);
     if (a.lneed && __ballot(cnt < 0)) {
       // a contender past the list window was reached before the cap: later
       // batches list at least this many contenders per node
@@ -1090,7 +1171,6 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
     int stop_lane = 64;
     // Store the verdicts decided since the last call: other nodes' waves may
     // be waiting for them, so they go out before this wave waits itself.
-    const uint64_t lane_bit = 1ull << lane;
     auto publish = [&]() {
       const uint64_t dec = (novel_m | capped_m | dupb_m | dupvr_m) & ~pub_m;
       if (fr && (dec & lane_bit)) {
@@ -1098,7 +1178,7 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
                       : (novel_m & lane_bit) ? DP_R_NOVEL
                       : (dupvr_m & lane_bit) ? DP_R_DUP_VISITED
                                              : DP_R_DUP_BATCH;
-        __hip_atomic_store(&a.res[p], (int8_t)r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        put(p, r);
       }
       pub_m |= dec;
     };
@@ -1126,10 +1206,7 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
       }
       if (a.limit > 0 && count + __popcll(nov) >= a.limit) {
         // lanes up to the (limit - count)-th NOVEL keep their status
-        uint64_t m = nov;
-        for (int t = count + 1; t < a.limit; ++t) m &= m - 1ull;
-        const int c = __ffsll((long long)m) - 1;
-        const uint64_t upto = c >= 63 ? ~0ull : ((2ull << c) - 1ull);
+        const uint64_t upto = upto_kth(nov, a.limit - count);
         novel_m = nov & upto;
         dupvr_m = dupv_m & upto;
         dupb_m = free_m & upto & ~novel_m & ~dupvr_m;
@@ -1179,11 +1256,8 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
         still = still || (def_m & lane_bit) != 0;
         dup_m |= __ballot(nov_found);
         const uint64_t nb = __ballot(still);
-        if (!(nb & (1ull << fb))) {
-          block_m = nb;
-          continue;  // fb is decided now: walk on
-        }
         block_m = nb;
+        if (!(nb & (1ull << fb))) continue;  // fb is decided now: walk on
       }
       int32_t polled = 0;
       const unsigned long long t_wait = a.trace ? (unsigned long long)wall_clock64() : 0ull;
@@ -1219,7 +1293,7 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
                 for (int k = 0; k < 8; ++k) oo[k] = g + k < cnt ? entry(g + k) : INT32_MAX;
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
-                  if (oo[k] >= cb) continue;  // past the list, or in this chunk
+                  if (oo[k] >= first) continue;  // past the list, or in this chunk
                   const int r = __hip_atomic_load(&a.res[oo[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                   if (r == DP_R_NOVEL) d = true;
                   else if (r == DP_R_UNDECIDED) mo = true;
@@ -1281,9 +1355,24 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
     n_dv += __popcll(dupvr_m);
     n_db += __popcll(dupb_m);
     if (stop_lane < 64) {
-      cur = cb + stop_lane;
+      cur = kSparse ? s_q[stop_lane] : first + stop_lane;
       stopped = true;
       break;
+    }
+    // the queue moves up by the chunk (64 when anything is left)
+    if constexpr (kSparse) {
+      for (int e0 = n; e0 < qn; e0 += 64) {
+        const bool mv = e0 + lane < qn;
+        const int32_t q = mv ? s_q[e0 + lane] : 0;
+        const int8_t f = mv ? s_qf[e0 + lane] : (int8_t)0;
+        __syncthreads();
+        if (mv) {
+          s_q[e0 - n + lane] = q;
+          s_qf[e0 - n + lane] = f;
+        }
+      }
+      qn -= n;
+      __syncthreads();
     }
     if (overflow) {
       // the rest of the node's FREE pairs go out CAPPED, as at the cap
@@ -1297,7 +1386,15 @@ __device__ bool advance_node(const round_args& a, int32_t node, int32_t& cur, in
       overflow = false;
     }
   }
-  if (!stopped) cur = end;
+  if (!stopped) {
+    cur = end;
+    // pairs capped before the walk (limit 0)
+    if (a.precap)
+      for (int32_t t0 = a.app[node]; t0 < end; t0 += 64) {
+        const int32_t t = t0 + lane;
+        n_cap += __popcll(__ballot(t < end && a.verdict[t] == DP_V_FREE && (a.flags[t] & DP_F_PRECAP)));
+      }
+  }
   if (a.trace && lane == 0) {
     unsigned long long* t = a.trace + (int64_t)DP_TRACE_FIELDS * node;
     t[2] += tr_wait;
@@ -1341,7 +1438,7 @@ __global__ __launch_bounds__(64) void k_round(round_args a) {
 // a wave that exhausts it leaves its node to the round kernel and raises a
 // flag the host checks.
 template <int NX>
-__device__ void walk_node(const round_args& a, int32_t node) {
+__device__ __forceinline__ void walk_node(const round_args& a, int32_t node) {
   if (a.trace && threadIdx.x == 0) {
     unsigned long long* t = a.trace + (int64_t)DP_TRACE_FIELDS * node;
     t[0] = (unsigned long long)wall_clock64();
@@ -1496,6 +1593,7 @@ static round_args make_round_args(dp_ctx* c) {
   a.count = c->d_node_count;
   a.node_novel = c->d_node_novel;
   a.limit = c->round_limit > 0 ? c->round_limit : 0;  // 0 (no cap here) also for limit 0: k_precap_first
+  a.precap = c->round_limit == 0 ? 1 : 0;
   a.slots = c->conf_slots;
   a.wait = 0;
   a.poll_cap = c->poll_cap;
