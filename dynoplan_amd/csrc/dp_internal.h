@@ -37,7 +37,10 @@
 #define DP_F_NOLIST 0x08
 // FP64 window of a quadrotor node, in FREE pairs: enough for the
 // cap of limit NOVEL pairs with a wide margin for duplicates.
-#define DP_FP64_WINDOW(limit) (3 * (limit) + 32)
+#define DP_FP64_WINDOW(limit) ((limit) < (1 << 28) ? 3 * (limit) + 32 : INT32_MAX)
+// Contenders of a planar node that get a conflict list before the context's
+// walks have shown how many they go through.
+#define DP_LIST_WINDOW(limit) ((limit) < (1 << 26) ? 20 * (limit) + 32 : INT32_MAX)
 // Pad added to swept boxes of the broad phase (m): bounds the rounding of
 // "canonical sweep + offset" versus per-state "state + offset" by 1e6x.
 #define DP_SWEEP_PAD 1e-9
@@ -318,7 +321,7 @@ struct dp_ctx {
   long long* d_counters = nullptr;  // [DPC_COUNT]
   long long* d_sticky = nullptr;    // [DPS_COUNT] never reset
   int32_t* d_wshift = nullptr;      // [2] quadrotor FP64 window growth (k_quad_window)
-  int32_t* d_lneed = nullptr;       // [1] planar list window need (k_list_window)
+  int32_t* d_lneed = nullptr;       // [1] planar: most contenders a walk went through (list window)
   int64_t n_batches = 0;            // dp_expand calls
   int64_t host_completions = 0;     // batches finished by host-launched work in dp_get_counts
   // test-only limits (dp_debug_set_limits): inline conflict slots used

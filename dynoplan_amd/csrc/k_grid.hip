@@ -293,11 +293,14 @@ __device__ __forceinline__ void put_record(const double* fin, int64_t pcap, int3
 // Contender records into cell order, and the list window (planar systems,
 // limit > 0, window > 0): the contenders of a node after its first W in
 // canonical order are flagged DP_F_NOLIST, and their list length is set to
-// -(1 + rank) (rank among the node's contenders, at most 32766).  The walk
-// reaches one of them only if more than W - limit contenders before it were
-// duplicates; it then records 1 + rank in need[0], and later batches of the
-// context use W = max(window, need + need / 4 + 16) (a fixed window leaves
-// need alone: need == null).
+// -(1 + rank) (rank among the node's contenders, at most 32766); the walk
+// scans the grid if it reaches one before the cap, which is slow (per lane,
+// and again on every retry).  The walks of the context's batches record in
+// need[0] the most contenders one of them went through; W is need + need / 4
+// + 16 (at least `least`), or `window` before the first batch: generous (20 * limit + 32, where
+// walks of 4096 unicycle1 nodes reach 79 contenders at the median and 342 at
+// most), since a first batch with W = 92 spent 13 to 17 ms scanning.  A fixed
+// window (need == null) is used as given.
 //
 // One wave per node, four nodes per workgroup, four chunks of 64 pairs per
 // step with their loads issued together (indices clamped into the node).
@@ -315,7 +318,7 @@ __global__ __launch_bounds__(256) void k_cont_scatter(int32_t N, const int32_t* 
                                                       const int32_t* __restrict__ start,
                                                       const int32_t* __restrict__ cell_of,
                                                       const int32_t* __restrict__ place, int32_t window,
-                                                      const int32_t* __restrict__ need, int16_t* __restrict__ conf_cnt,
+                                                      int32_t least, const int32_t* __restrict__ need, int16_t* __restrict__ conf_cnt,
                                                       double* __restrict__ rec) {
   const int32_t node = blockIdx.x * 4 + (int32_t)(threadIdx.x / 64);
   if (node >= N) return;
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(256) void k_cont_scatter(int32_t N, const int32_t* 
   if (window > 0 && need) {
     const int32_t nd = need[0];
     const int64_t w = (int64_t)nd + nd / 4 + 16;
-    if (nd > 0 && w > window) window = w < INT32_MAX ? (int32_t)w : INT32_MAX;
+    if (nd > 0) window = w < least ? least : (w < INT32_MAX ? (int32_t)w : INT32_MAX);
   }
   const int32_t tot = *total;
   const int32_t b = app[node] < tot ? app[node] : tot;
@@ -856,7 +859,7 @@ struct round_args {
   long long* counters;
   long long* sticky;  // [DPS_COUNT] never reset
   int32_t* wshift;    // quadrotor FP64 window: [0] growth for later batches, [1] the growth this batch used
-  int32_t* lneed;     // planar list window: [0] largest 1 + rank of a listless contender a walk reached
+  int32_t* lneed;     // planar list window: [0] most contenders a walk went through
 };
 
 // Pause between two polls of a contender's verdict: grows with the number of
@@ -901,6 +904,7 @@ __device__ __forceinline__ bool advance_node(const round_args& a, int32_t node, 
   const int32_t end = a.app[node + 1] < tot ? a.app[node + 1] : tot;
   if (cur >= end) return true;
   long long n_nov = 0, n_cap = 0, n_dv = 0, n_db = 0, n_goal = 0;
+  int32_t seen = 0;  // contenders gone through
   bool overflow = false;  // a deferred pair (past the FP64 window) was reached before the cap
   // diagnostics (trace only): cycles evaluating lists, cycles in the
   // in-chunk walk, cycles waiting, chunks, waits, polls
@@ -1146,14 +1150,6 @@ __device__ __forceinline__ bool advance_node(const round_args& a, int32_t node, 
     const int cnt = fr && !forced && !dupv && !deferred ? cc_p : 0;
     eval_lists(first, n, cnt, ov_p, same, undec, ext_dup, more);
     if (cnt > 0) ext_block = !ext_dup && (undec != 0 || more);
-    if (a.lneed && __ballot(cnt < 0)) {
-      // a contender past the list window was reached before the cap: later
-      // batches list at least this many contenders per node
-      int need = cnt < 0 && (fl & DP_F_NOLIST) ? -cnt : 0;
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) need = max(need, __shfl_xor(need, d, 64));
-      if (lane == 0 && need > 0) atomicMax(a.lneed, need);
-    }
     if (cnt < 0) eval(p, 0);
     unsigned long long t_walk = 0;
     if (a.trace) {
@@ -1354,6 +1350,7 @@ __device__ __forceinline__ bool advance_node(const round_args& a, int32_t node, 
     n_cap += __popcll(capped_m);
     n_dv += __popcll(dupvr_m);
     n_db += __popcll(dupb_m);
+    seen += __popcll(novel_m | dupb_m);
     if (stop_lane < 64) {
       cur = kSparse ? s_q[stop_lane] : first + stop_lane;
       stopped = true;
@@ -1405,6 +1402,8 @@ __device__ __forceinline__ bool advance_node(const round_args& a, int32_t node, 
     t[7] += tr_polls;
   }
   if (lane == 0) {
+    // the plain load filters: few nodes raise the maximum
+    if (a.lneed && seen > *a.lneed) atomicMax(a.lneed, seen);
     a.cursor[node] = cur;
     a.count[node] = count;
     if (!stopped) {
@@ -1660,13 +1659,13 @@ int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool c
   c->round_limit = p->limit_branching_factor;
   c->round_r_dup = r_dup;
   c->round_params = *p;
-  // Planar systems with a cap: only the first DP_FP64_WINDOW(limit) FREE
-  // pairs of each node get a stored list (or the test limit).  Quadrotor
+  // Planar systems with a cap: only the first contenders of each node get a
+  // stored list (k_cont_scatter; or the test limit).  Quadrotor
   // pairs past their node's FP64 window are not contenders at all
   // (k_quad_window), so every quadrotor contender gets a list.
   const int32_t lim = p->limit_branching_factor;
   const int32_t window = lim > 0 && c->desc.system != DP_SYS_QUADROTOR && !c->select_mode
-                             ? (c->fp64_window > 0 ? c->fp64_window : DP_FP64_WINDOW(lim))
+                             ? (c->fp64_window > 0 ? c->fp64_window : DP_LIST_WINDOW(lim))
                              : 0;
   const int32_t* lneed = c->fp64_window > 0 ? nullptr : c->d_lneed;
   const int pb = dp_grid_blocks(c->pair_cap, 256, 8192);
@@ -1692,7 +1691,7 @@ int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool c
     else
       k_cont_scatter<NX><<<(N + 3) / 4, 256, 0, s>>>(N, c->d_app, c->d_total, c->d_verdict, c->d_flags, c->d_final,
                                                    c->pair_cap, c->d_cont_count, c->d_cont_start, c->d_cont_cell,
-                                                   c->d_conf_ov, window, lneed, c->d_conf_cnt, c->d_cont_x);
+                                                   c->d_conf_ov, window, DP_FP64_WINDOW(lim), lneed, c->d_conf_cnt, c->d_cont_x);
     // earlier-conflict lists
     k_conf_waves<NX><<<(int)std::min<int64_t>((nc + 3) / 4, 8192), 256, 0, s>>>(
         c->d_sys, c->grid, c->d_cont_start, c->d_cont_x, items, r_dup, c->d_conf_cnt, c->d_conf, c->d_conf_ov,

@@ -260,8 +260,9 @@ int dp_health(dp_ctx* ctx, dp_health_info* out);
  * FREE pairs per node: the quadrotor's FP64 window (0: 3 * limit + 32,
  * doubled for a context's later batches each time one of its batches
  * overflowed it, up to 2^10 times) and, for planar systems, the pairs that
- * get stored conflict lists (0: 3 * limit + 32; a pair past it is scanned
- * from the grid when reached).  Results do not depend on them. */
+ * get stored conflict lists (0: 20 * limit + 32, then from the pairs that
+ * the context's batches went through; a pair past it is scanned from the
+ * grid when reached).  Results do not depend on them. */
 int dp_debug_set_limits(dp_ctx* ctx, int32_t conf_slots, int64_t pool_entries, int32_t fp64_window);
 
 /* Copy the per-pair results of the last dp_expand into caller buffers, in
