@@ -597,6 +597,7 @@ static int ensure_visited_cap(dp_ctx* c, int64_t need) {
   }
   dev_free(&c->d_vis);
   c->d_vis = nv_;
+  c->nv_sorted = 0;  // the sorted copy is allocated anew: the grid is dirty
   int rc;
   if ((rc = dev_alloc(&c->d_vis_sorted, (int64_t)nx * cap))) return rc;
   if ((rc = dev_alloc(&c->d_vis_cell, cap))) return rc;
@@ -610,6 +611,7 @@ static int ensure_visited_cap(dp_ctx* c, int64_t need) {
 int dp_visited_reset(dp_ctx* c) {
   ARG_CHECK(c, "null context");
   c->nv = 0;
+  c->nv_sorted = 0;
   c->grid_dirty = true;
   dp_bump_epoch();
   return DP_OK;

@@ -225,6 +225,8 @@ struct dp_ctx {
 
   // visited set (T_n)
   int64_t nv = 0, nv_cap = 0;
+  int64_t nv_sorted = 0;           // states the grid holds; [nv_sorted, nv) lie behind them, unsorted, and every
+                                   // duplicate test reads them as one more run
   double* d_vis = nullptr;         // [nx][nv_cap] append order
   double* d_vis_sorted = nullptr;  // [nx][nv_cap] sorted by cell
   int32_t* d_vis_cell = nullptr;   // scratch [nv_cap]
@@ -390,6 +392,10 @@ int dp_launch_visited_append_novel(dp_ctx* c, int64_t novel_total, hipStream_t s
 // counted: the check stage has counted the contenders into their cells (else
 // they are counted here).
 int dp_launch_resolve(dp_ctx* c, const dp_expand_params* p, double r_dup, bool counted, hipStream_t s);
+// Few nodes with a cap: the batch is resolved by one workgroup, without a
+// contender grid (and without the test limits of the general path).
+bool dp_small_batch(const dp_ctx* c, const dp_expand_params* p);
+int dp_launch_resolve_small(dp_ctx* c, const dp_expand_params* p, double r_dup, hipStream_t s);
 // Contender grid buffers for the current geometry (before the check stage).
 int dp_ensure_cont_grid(dp_ctx* c);
 // Doubles of a contender record: the state, its pair index (int32, bit 31:
@@ -465,6 +471,14 @@ int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s);
 // block is 9 runs of 3 cells adjacent in memory (x is the fastest grid axis):
 // run k covers rows c1 + k%3 - 1 and layers c2 + k/3 - 1 (the rules of
 // dp_cell_neighbor), x from c0 - 1 to c0 + 1 clipped to the grid.
+// Visited states an expansion may leave unsorted: the tail costs every FREE
+// pair one test per state, a rebuild of the grid four launches (20 us).  At
+// 1000 combinations and 20 new states per batch, 524 states at most cost 7 us
+// a batch on average and 262 cost 3.5, against 1 and 2 us of rebuilding.
+inline bool dp_tail_fits(const dp_ctx* c) {
+  return (c->nv - c->nv_sorted) * (int64_t)c->N * c->P <= (1ll << 18);
+}
+
 template <int NX>
 __device__ __forceinline__ bool dp_grid_run_any(const dp_dev_sys& S, const dp_grid_geom& G, const int32_t* start,
                                              const double* pts, int64_t stride, const double* x, int k, double r,

@@ -438,7 +438,7 @@ struct dp_check_args {
   int32_t nobs;
   const double* vis;
   int64_t vstride;
-  int64_t nv;
+  int64_t nv, nv_sorted;
   const int32_t* vstart;
   dp_grid_geom grid;
   const int32_t* pnode;
@@ -506,7 +506,7 @@ struct check_wave {
     } con;                   // constraints: per pair to test
     struct {
       double x[NX][64];      // state of the new node, per lane
-      int2 run[9 * 64];      // per non-empty run: the pair's lane, sorted position minus first item
+      int2 run[10 * 64];      // per non-empty run: the pair's lane, sorted position minus first item
     } vis;
   };
 };
@@ -841,11 +841,11 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
     bool dupv = false;
     if (a.nv > 0 && !a.select && __ballot(fr)) {
       // the 9 runs of each final state's 27-cell block (dp_grid_run_any's
-      // rules), their bounds loaded together
-      int32_t rb[9], rn[9];
+      // rules), their bounds loaded together, and the unsorted tail
+      int32_t rb[10], rn[10];
       int K = 0, nr = 0;
 #pragma unroll
-      for (int k = 0; k < 9; ++k) rb[k] = rn[k] = 0;
+      for (int k = 0; k < 10; ++k) rb[k] = rn[k] = 0;
       if (fr) {
         const dp_grid_geom& G = a.grid;
         int32_t c[3];
@@ -868,8 +868,10 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
           rb[k] = a.vstart[ok ? row + x0 : 0];
           rn[k] = a.vstart[ok ? row + x1 + 1 : 0];
         }
+        rb[9] = (int32_t)a.nv_sorted;
+        rn[9] = (int32_t)a.nv;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) {
+        for (int k = 0; k < 10; ++k) {
           rn[k] -= rb[k];
           K += rn[k];
           nr += rn[k] > 0 ? 1 : 0;
@@ -880,7 +882,7 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
       {
         int f = incl - K, at = run0;
 #pragma unroll
-        for (int k = 0; k < 9; ++k)
+        for (int k = 0; k < 10; ++k)
           if (rn[k] > 0) {
             W.vis.run[at++] = make_int2(lane, rb[k] - f);
             f += rn[k];
@@ -894,7 +896,7 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
           [&](int w0) {
             int f = incl - K;
 #pragma unroll
-            for (int k = 0; k < 9; ++k)
+            for (int k = 0; k < 10; ++k)
               if (rn[k] > 0) {
                 mark_item(W.head, f, w0);
                 f += rn[k];
@@ -1159,7 +1161,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   const double r_dup = (1. - (double)p->alpha) * (double)p->delta;      // dbastar.cpp:852
   const double goal_bound = p->delta_factor_goal * (double)p->delta;    // dbastar.cpp:827
 
-  if (!c->select_mode && (c->grid_dirty || c->grid_radius != r_dup)) {
+  if (!c->select_mode && (c->grid_dirty || c->grid_radius != r_dup || !dp_tail_fits(c))) {
     int rc = dp_launch_visited_rebuild(c, r_dup, s);
     if (rc) return rc;
   }
@@ -1167,8 +1169,9 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   // The check stage counts the contenders into their grid cells as it finds
   // them; limit 0 takes pairs out again after it (k_precap_first), so there
   // they are counted later.
-  const bool count = !c->select_mode && p->limit_branching_factor != 0;
-  int rc = c->select_mode ? DP_OK : dp_ensure_cont_grid(c);
+  const bool small = dp_small_batch(c, p);
+  const bool count = !c->select_mode && p->limit_branching_factor != 0 && !small;
+  int rc = c->select_mode || small ? DP_OK : dp_ensure_cont_grid(c);
   if (rc) return rc;
   DP_EV(c->ev[0], s);
   dp_begin(c->d_counters, c->d_app_cnt, N, c->d_cont_count, count ? c->grid.nslots : 0, dp_stage(c, 1u << 0), s);
@@ -1236,6 +1239,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   a.vis = c->d_vis_sorted;
   a.vstride = c->nv_cap;
   a.nv = c->nv;
+  a.nv_sorted = c->nv_sorted;
   a.vstart = c->d_vis_start;
   a.grid = c->grid;
   a.pnode = c->d_pnode;
@@ -1261,7 +1265,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   a.con = c->d_con;
   a.con_delta = (double)p->delta;
   a.select = c->select_mode ? 1 : 0;
-  if (c->select_mode) a.nv = 0;
+  if (c->select_mode) a.nv = a.nv_sorted = 0;
   a.cont_count = count ? c->d_cont_count : nullptr;
   a.cont_cell = c->d_cont_cell;
   a.cont_place = c->d_conf_ov;
@@ -1269,7 +1273,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   if (c->desc.system == DP_SYS_QUADROTOR) {
     rc = dp_launch_quad(c, p, goal_bound, r_dup, count, s);
     if (rc) return rc;
-    rc = dp_launch_resolve(c, p, r_dup, count, s);
+    rc = small ? dp_launch_resolve_small(c, p, r_dup, s) : dp_launch_resolve(c, p, r_dup, count, s);
     if (rc) return rc;
     DP_EV(c->ev[1], s);
     c->timing_valid = !c->no_events && !c->defer_walk;
@@ -1313,7 +1317,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     c->timing_valid = !c->no_events && !c->defer_walk;
     return DP_OK;
   }
-  rc = dp_launch_resolve(c, p, r_dup, count, s);
+  rc = small ? dp_launch_resolve_small(c, p, r_dup, s) : dp_launch_resolve(c, p, r_dup, count, s);
   if (rc) return rc;
   DP_EV(c->ev[1], s);
   c->timing_valid = !c->no_events && !c->defer_walk;

@@ -1430,6 +1430,218 @@ __global__ __launch_bounds__(64) void k_round(round_args a) {
   (void)advance_node<NX>(a, node, cur, count);
 }
 
+// Whole resolution of a batch of few nodes (the reference's loop expands one)
+// in one workgroup: the sequential rule itself, 64 pairs at a time, against
+// the NOVEL states so far, which fit LDS (at most kSmallNovel, limit per
+// node).  Per chunk the waves test the chunk's contenders against those
+// states and against each other (one ballot per earlier contender), then one
+// wave takes the lowest undecided lane as NOVEL, strikes its conflicts out
+// and so on: at most `limit` steps per node.  The grid, lists, pre-pass and
+// walk of a large batch are six launches and about 45 us at any size; this
+// takes 6 us for one node of 100 pairs, 4 us more per further node.
+constexpr int kSmallNodes = 4, kSmallNovel = 160;
+
+struct small_args {
+  const dp_dev_sys* sys;
+  int32_t N;
+  const int32_t* app;
+  const int32_t* total;
+  const int8_t* verdict;
+  const int8_t* flags;
+  const double* fin;
+  int64_t pcap;
+  double r_dup;
+  int32_t limit;  // > 0
+  int8_t* res;
+  int32_t* node_novel;
+  long long* counters;
+  long long* sticky;
+  int32_t* wshift;
+  dp_marks marks;
+};
+
+// Waves of the workgroup (the quadrotor's 13 components need the registers).
+constexpr int small_waves(int nx) { return nx == 13 ? 8 : 16; }
+
+template <int NX>
+__global__ __launch_bounds__(64 * small_waves(NX)) void k_resolve_small(small_args a) {
+  constexpr int kW = small_waves(NX);
+  dp_mark(a.marks);
+  __shared__ dp_dev_sys s_sys;
+  __shared__ double s_nov[NX][kSmallNovel], s_x[NX][64];
+  __shared__ unsigned long long s_hit[64], s_dup, s_con, s_forced, s_free, s_dupv, s_def;
+  __shared__ int32_t s_count, s_nnov, s_stop, s_tail, s_n, s_base[kW], s_list[64 * kW];
+  __shared__ int8_t s_flag[64 * kW];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  for (int t = threadIdx.x; t < (int)(sizeof(dp_dev_sys) / sizeof(double)); t += blockDim.x)
+    reinterpret_cast<double*>(&s_sys)[t] = reinterpret_cast<const double*>(a.sys)[t];
+  if (threadIdx.x == 0) {
+    s_nnov = 0;
+    s_tail = 0;
+  }
+  __syncthreads();
+  const dp_dev_sys& S = s_sys;
+  const double T = dp_pos_bound(S, a.r_dup);
+  auto within = [&](const double* x, const double* y) {
+    if constexpr (NX == 13) return dp_within_quad_fast(S, x, y, a.r_dup);
+    else return dp_within_planar_fast<NX>(S, x, y, a.r_dup, T);
+  };
+  const uint64_t lt = (1ull << lane) - 1ull, lane_bit = 1ull << lane;
+  const int32_t tot = *a.total;
+  long long n_nov = 0, n_cap = 0, n_dv = 0, n_db = 0, n_goal = 0;
+  for (int32_t node = 0; node < a.N; ++node) {
+    const int32_t b = a.app[node] < tot ? a.app[node] : tot;
+    const int32_t e = a.app[node + 1] < tot ? a.app[node + 1] : tot;
+    if (threadIdx.x == 0) {
+      s_count = 0;
+      s_stop = 0;
+    }
+    __syncthreads();
+    int32_t from = e;  // first pair after the node's loop ended
+    for (int32_t sb = b; sb < e && from == e; sb += 64 * kW) {
+      // the FREE pairs of the next 64 * kW, in order (a quadrotor node's are
+      // 4% of its pairs: one chunk instead of nine)
+      {
+        const int32_t t = sb + 64 * wave + lane;
+        const int8_t v = a.verdict[t < e ? t : e - 1], f = a.flags[t < e ? t : e - 1];
+        const bool fr = t < e && v == DP_V_FREE;
+        const uint64_t m = __ballot(fr);
+        if (lane == 0) s_base[wave] = __popcll(m);
+        __syncthreads();
+        int32_t at = __popcll(m & lt);
+        for (int k = 0; k < wave; ++k) at += s_base[k];
+        if (fr) {
+          s_list[at] = t;
+          s_flag[at] = f;
+        }
+        if (threadIdx.x == 0) {
+          int32_t n = 0;
+          for (int k = 0; k < kW; ++k) n += s_base[k];
+          s_n = n;
+        }
+        __syncthreads();
+      }
+      const int32_t n_free = s_n;
+      for (int32_t cb = 0; cb < n_free; cb += 64) {
+        const bool fr = cb + lane < n_free;
+        const int32_t p = s_list[fr ? cb + lane : 0];
+        if (wave == 0) {
+          const int8_t fl = fr ? s_flag[cb + lane] : (int8_t)0;
+          const bool df = fr && (fl & DP_F_DEFER), fo = fr && !df && (fl & 2), dv = fr && !df && !fo && (fl & 1);
+          const bool con = fr && !df && !dv;
+          if (con)
+#pragma unroll
+            for (int k = 0; k < NX; ++k) s_x[k][lane] = a.fin[(int64_t)k * a.pcap + p];
+          const uint64_t m0 = __ballot(fr), m1 = __ballot(con), m2 = __ballot(fo), m3 = __ballot(dv), m4 = __ballot(df);
+          if (lane == 0) {
+            s_free = m0;
+            s_con = m1;
+            s_forced = m2;
+            s_dupv = m3;
+            s_def = m4;
+            s_dup = 0;
+          }
+        }
+        __syncthreads();
+        {
+          const uint64_t cm = s_con;
+          const bool con = (cm & lane_bit) != 0;
+          double x[NX], y[NX];
+#pragma unroll
+          for (int k = 0; k < NX; ++k) x[k] = con ? s_x[k][lane] : 0.0;
+          bool hit = false;
+          for (int t = wave; t < s_nnov; t += kW) {
+#pragma unroll
+            for (int k = 0; k < NX; ++k) y[k] = s_nov[k][t];
+            if (con && !hit) hit = within(x, y);
+          }
+          const uint64_t d = __ballot(hit);
+          if (lane == 0 && d) atomicOr(&s_dup, d);
+          for (int j = wave; j < 64; j += kW) {
+            if (!((cm >> j) & 1ull)) continue;
+#pragma unroll
+            for (int k = 0; k < NX; ++k) y[k] = s_x[k][j];
+            const uint64_t m = __ballot(con && lane > j && within(x, y));
+            if (lane == 0) s_hit[j] = m;
+          }
+        }
+        __syncthreads();
+        if (wave == 0) {
+          const uint64_t con = s_con, forced = s_forced, fm = s_free, dv = s_dupv, def = s_def;
+          // a deferred pair (past the FP64 window) reached before the cap is a
+          // window overflow, as in advance_node
+          const int fd = def ? __ffsll((long long)def) - 1 : 64;
+          const uint64_t below = fd >= 64 ? ~0ull : ((1ull << fd) - 1ull);
+          uint64_t rem = ((con & ~s_dup) | forced) & below, nov = 0;
+          int count = s_count, cap = -1;
+          while (rem) {
+            const int j = __ffsll((long long)rem) - 1;
+            nov |= 1ull << j;
+            rem &= ~(1ull << j);
+            rem &= ~(s_hit[j] & ~forced);
+            if (++count >= a.limit) {
+              cap = j;
+              break;
+            }
+          }
+          const bool over = cap < 0 && fd < 64;
+          const uint64_t upto = cap >= 0 ? (cap >= 63 ? ~0ull : (2ull << cap) - 1ull) : below;
+          const uint64_t capped = fm & ~upto, dupv = dv & upto, dupb = fm & upto & ~nov & ~dupv;
+          if (fm & lane_bit)
+            a.res[p] = (int8_t)((capped & lane_bit) ? DP_R_CAPPED
+                                : (nov & lane_bit)  ? DP_R_NOVEL
+                                : (dupv & lane_bit) ? DP_R_DUP_VISITED
+                                                    : DP_R_DUP_BATCH);
+          const int at = s_nnov + __popcll(nov & lt);
+          if ((nov & lane_bit) && at < kSmallNovel)
+#pragma unroll
+            for (int k = 0; k < NX; ++k) s_nov[k][at] = s_x[k][lane];
+          n_nov += __popcll(nov);
+          n_goal += __popcll(nov & forced);
+          n_cap += __popcll(capped);
+          n_dv += __popcll(dupv);
+          n_db += __popcll(dupb);
+          if (lane == 0) {
+            s_count = count;
+            s_nnov += __popcll(nov);
+            s_stop = cap >= 0 || over;
+            if (over) {
+              atomicAdd((unsigned long long*)&a.counters[DPC_WINDOW_OVF], 1ull);
+              atomicAdd((unsigned long long*)&a.sticky[DPS_WINDOW], 1ull);
+              atomicMax(&a.wshift[0], a.wshift[1] + 1);
+            }
+          }
+        }
+        __syncthreads();
+        if (s_stop) {
+          from = s_list[cb + 64 < n_free ? cb + 63 : n_free - 1] + 1;
+          break;
+        }
+      }
+      __syncthreads();  // the list is written again
+    }
+    // the node's loop has ended: every later FREE pair is CAPPED
+    if (from < e) {
+      int n = 0;
+      for (int32_t t = from + (int32_t)threadIdx.x; t < e; t += 64 * kW)
+        if (a.verdict[t] == DP_V_FREE) {
+          a.res[t] = DP_R_CAPPED;
+          ++n;
+        }
+      if (n) atomicAdd(&s_tail, n);
+    }
+    if (threadIdx.x == 0) a.node_novel[node] = s_count;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    a.counters[DPC_NOVEL] = n_nov;
+    a.counters[DPC_CAPPED] = n_cap + s_tail;
+    a.counters[DPC_DUPV] = n_dv;
+    a.counters[DPC_DUPB] = n_db;
+    a.counters[DPC_GOAL] = n_goal;
+  }
+}
+
 // Persistent resolution: waves claim nodes in ascending order through a
 // ticket and advance them until finished, backing off while blocked.  A
 // wave only waits for nodes with smaller tickets, all held by resident
@@ -1528,20 +1740,32 @@ __global__ void k_queue_reset(unsigned long long* __restrict__ queues, int32_t n
 }
 
 // Append the NOVEL final states of the batch to the visited set in canonical
-// order; dst holds the exclusive scan of NOVEL pairs per node.
+// order, one wave per node; novel: NOVEL pairs per node, or (scanned) their
+// exclusive scan.  The states also go behind the sorted ones, where queries
+// read them as one more run until the grid is built again.
 template <int NX>
 __global__ __launch_bounds__(64) void k_gather_novel(int32_t N, const int32_t* __restrict__ app,
                                                      const int32_t* __restrict__ total,
-                                                     const int8_t* __restrict__ res, const int32_t* __restrict__ dst,
-                                                     const double* __restrict__ fin, int64_t pcap,
-                                                     double* __restrict__ vis, int64_t vstride, int64_t vbase) {
+                                                     const int8_t* __restrict__ res, const int32_t* __restrict__ novel,
+                                                     int32_t scanned, const double* __restrict__ fin, int64_t pcap,
+                                                     double* __restrict__ vis, double* __restrict__ sorted,
+                                                     int64_t vstride, int64_t vbase) {
   const int32_t node = blockIdx.x;
   if (node >= N) return;
   const int lane = threadIdx.x;
   const int32_t tot = *total;
   const int32_t begin = app[node] < tot ? app[node] : tot;
   const int32_t end = app[node + 1] < tot ? app[node + 1] : tot;
-  int64_t w = vbase + dst[node];
+  int64_t w = vbase;
+  if (scanned) {
+    w += novel[node];
+  } else {
+    int32_t sum = 0;
+    for (int32_t k = lane; k < node; k += 64) sum += novel[k];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    w += sum;
+  }
   for (int32_t cb = begin; cb < end; cb += 64) {
     const int32_t p = cb + lane;
     const bool nov = p < end && res[p] == DP_R_NOVEL;
@@ -1549,7 +1773,11 @@ __global__ __launch_bounds__(64) void k_gather_novel(int32_t N, const int32_t* _
     if (nov) {
       const int64_t pos = w + __popcll(m & ((1ull << lane) - 1ull));
 #pragma unroll
-      for (int c = 0; c < NX; ++c) vis[(int64_t)c * vstride + pos] = fin[(int64_t)c * pcap + p];
+      for (int c = 0; c < NX; ++c) {
+        const double v = fin[(int64_t)c * pcap + p];
+        vis[(int64_t)c * vstride + pos] = v;
+        sorted[(int64_t)c * vstride + pos] = v;
+      }
     }
     w += __popcll(m);
   }
@@ -1647,7 +1875,45 @@ int dp_launch_visited_rebuild(dp_ctx* c, double radius, hipStream_t s) {
   if (rc) return rc;
   DP_HIP_RET(hipGetLastError());
   c->grid_dirty = false;
+  c->nv_sorted = c->nv;
   dp_bump_epoch();
+  return DP_OK;
+}
+
+bool dp_small_batch(const dp_ctx* c, const dp_expand_params* p) {
+  const int64_t lim = p->limit_branching_factor;
+  return c->N <= kSmallNodes && lim > 0 && lim * c->N <= kSmallNovel && !c->select_mode && !c->defer_walk &&
+         !c->d_trace && c->conf_slots == DP_CONF_SLOTS && c->pool_limit == 0 && c->fp64_window == 0;
+}
+
+int dp_launch_resolve_small(dp_ctx* c, const dp_expand_params* p, double r_dup, hipStream_t s) {
+  c->round_limit = p->limit_branching_factor;
+  c->round_r_dup = r_dup;
+  c->round_params = *p;
+  small_args a{};
+  a.sys = c->d_sys;
+  a.N = c->N;
+  a.app = c->d_app;
+  a.total = c->d_total;
+  a.verdict = c->d_verdict;
+  a.flags = c->d_flags;
+  a.fin = c->d_final;
+  a.pcap = c->pair_cap;
+  a.r_dup = r_dup;
+  a.limit = p->limit_branching_factor;
+  a.res = c->d_res;
+  a.node_novel = c->d_node_novel;
+  a.counters = c->d_counters;
+  a.sticky = c->d_sticky;
+  a.wshift = c->d_wshift;
+  a.marks = dp_stage(c, c->desc.system == DP_SYS_QUADROTOR ? (1u << 2) | (1u << 7) : (1u << 2) | (1u << 6) | (1u << 7));
+  int rc = dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
+    constexpr int NX = decltype(NXc)::value;
+    k_resolve_small<NX><<<1, 64 * small_waves(NX), 0, s>>>(a);
+    return DP_OK;
+  });
+  if (rc) return rc;
+  DP_HIP_RET(hipGetLastError());
   return DP_OK;
 }
 
@@ -1876,17 +2142,17 @@ int dp_launch_visited_append_novel(dp_ctx* c, int64_t novel_total, hipStream_t s
   // Caller guarantees visited capacity >= nv + novel_total.
   const int32_t N = c->N;
   if (N <= 0 || novel_total <= 0) return DP_OK;
-  dp_scan_small(c->d_node_novel, c->d_node_novel, N, nullptr, INT64_MAX, c->d_counters, -1, s);
+  const bool scan = N > 1024;  // below, each wave sums the nodes before its own
+  if (scan) dp_scan_small(c->d_node_novel, c->d_node_novel, N, nullptr, INT64_MAX, c->d_counters, -1, s);
   int rc = dispatch_nx(c->desc.nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
-    k_gather_novel<NX><<<N, 64, 0, s>>>(N, c->d_app, c->d_total, c->d_res, c->d_node_novel, c->d_final,
-                                        c->pair_cap, c->d_vis, c->nv_cap, c->nv);
+    k_gather_novel<NX><<<N, 64, 0, s>>>(N, c->d_app, c->d_total, c->d_res, c->d_node_novel, scan ? 1 : 0, c->d_final,
+                                        c->pair_cap, c->d_vis, c->d_vis_sorted, c->nv_cap, c->nv);
     return DP_OK;
   });
   if (rc) return rc;
   DP_HIP_RET(hipGetLastError());
-  c->nv += novel_total;
-  c->grid_dirty = true;
+  c->nv += novel_total;  // past nv_sorted: the unsorted tail
   dp_bump_epoch();
   return DP_OK;
 }

@@ -66,7 +66,7 @@ struct dp_quad_args {
   double tmax;            // longest primitive duration
   const float* preach;    // [P] per primitive: max_k |p_k - p_0|_inf + (L - 1) dt, the reach at unit speed offset
   const double* vis;
-  int64_t vstride, nv;
+  int64_t vstride, nv, nv_sorted;
   const int32_t* vstart;
   dp_grid_geom grid;
   const int32_t* app;     // pair offsets per node [N+1]
@@ -978,6 +978,8 @@ __global__ __launch_bounds__(256) void k_quad64(dp_quad_args a) {
     if (a.nv > 0)
       for (int k = 0; k < 9 && !dupv; ++k)
         dupv = dp_grid_run_any<13>(S, a.grid, a.vstart, a.vis, a.vstride, x, k, a.r_dup, Tdup);
+    for (int64_t t = a.nv_sorted; t < a.nv && !dupv; ++t)  // the unsorted tail
+      dupv = dp_within_col_pf<13>(S, x, a.vis, a.vstride, t, a.r_dup, Tdup);
     a.flags[q] = (int8_t)((chosen != -1 ? 2 : 0) | (dupv ? 1 : 0));
     if (a.cont_count && (chosen != -1 || !dupv))
       dp_count_contender(a.grid, x, q, a.cont_count, a.cont_cell, a.cont_place);
@@ -1260,6 +1262,7 @@ dp_quad_args make_quad_args(dp_ctx* c, const dp_expand_params* p, double goal_bo
   a.vis = c->d_vis_sorted;
   a.vstride = c->nv_cap;
   a.nv = c->nv;
+  a.nv_sorted = c->nv_sorted;
   a.vstart = c->d_vis_start;
   a.grid = c->grid;
   a.app = c->d_app;

@@ -340,7 +340,7 @@ int dp_visited_radius(dp_ctx* c, const double* queries, int64_t n, double radius
   if (n == 0) return DP_OK;
   hipStream_t s = c->stream;
   // A grid built for a radius R >= radius has cells wide enough for it.
-  if (c->grid_dirty || !(c->grid_radius >= radius)) {
+  if (c->grid_dirty || c->nv != c->nv_sorted || !(c->grid_radius >= radius)) {
     int rc = dp_launch_visited_rebuild(c, radius, s);
     if (rc) return rc;
   }
@@ -398,7 +398,7 @@ int dp_visited_radius_noalloc(dp_ctx* c, const double* d_queries, int64_t n, dou
     dp_set_error("radius must be finite and >= 0");
     return DP_ERR_ARG;
   }
-  if (c->nv > 0 && (c->grid_dirty || !(c->grid_radius >= radius))) {
+  if (c->nv > 0 && (c->grid_dirty || c->nv != c->nv_sorted || !(c->grid_radius >= radius))) {
     dp_set_error("the visited grid is not built for this radius: call dp_visited_radius or dp_expand once "
                  "after the last change of the visited set");
     return DP_ERR_STATE;
