@@ -228,6 +228,10 @@ int dp_batch_expand(dp_batch* b, const dp_expand_params* params, void* stream) {
     B_HIP(hipGraphLaunch(b->exec, s));
     b->last = s;
   }
+  for (dp_ctx* c : b->ctx) {
+    c->counts_fresh = false;
+    c->outside = true;
+  }
   ++b->launches;
   b->stamped = true;
   return DP_OK;

@@ -60,6 +60,9 @@
 // first kernel of each stage writes the GPU's constant-rate clock (an event
 // between two kernels costs the stream about 4 us).
 #define DP_MARKS 8
+// Largest pinned staging buffer: three of them per context at most, and large
+// enough that a piece takes far longer on the host link than its launch.
+#define DP_STAGE_MAX (8ll << 20)
 // LDS per workgroup on gfx950
 #define DP_LDS_MAX 163840
 #define DP_SPIN_LIMIT_WAITING (1 << 10)
@@ -279,7 +282,20 @@ struct dp_ctx {
   double round_r_dup = 0.0;         // duplicate radius of the batch in flight
   int32_t* d_node_cursor = nullptr; // [N_cap] first undecided pair per node
   int32_t* d_node_count = nullptr;  // [N_cap] NOVEL pairs decided per node
-  long long* h_pinned = nullptr;    // pinned host words for device totals
+  long long* h_pinned = nullptr;    // [DPC_COUNT + 4] pinned host words: the batch counters as last read, then device totals
+  bool counts_fresh = false;        // h_pinned holds the counters of the last expansion, its work finished
+  // Pinned staging of uploads and read-back, grown on demand to at most
+  // DP_STAGE_MAX bytes each (larger results go through in pieces).
+  char* h_up = nullptr;             // nodes and g, or dbrrt targets
+  int64_t h_up_cap = 0;
+  char* h_down[2] = {nullptr, nullptr};
+  int64_t h_down_cap[2] = {0, 0};
+  hipEvent_t down_ev[2] = {};
+  bool up_busy = false;             // a kernel may still be reading h_up
+  // The context has been given to work that its own stream does not order (a
+  // caller's stream, a batch's graph, its stream handed out): from then on
+  // uploads and reads wait for the whole device and counters are read anew.
+  bool outside = false;
   int32_t rounds = 32;              // resolution rounds launched per batch
   int32_t* d_chunk = nullptr;       // [N_cap+1] quadrotor: 64-pair chunks per node, then scanned
   int32_t* d_nshort = nullptr;      // [N_cap] quadrotor: pairs whose primitive leaves the rate bounds
@@ -308,8 +324,8 @@ struct dp_ctx {
   double* d_con = nullptr;          // [con_cap] times, then [con_cap][nx] states
   double* d_targets = nullptr;      // [nx][N_cap] dbrrt targets of dp_expand_select
   int32_t targets_cap = 0;
-  int32_t* d_sel_q = nullptr;       // [N_cap] chosen pair per node (-1: none)
-  double* d_sel = nullptr;          // [N_cap][2 nx + 3] last state, first state, distance, g, h
+  double* d_sel = nullptr;          // [sel_cap][2 nx + 3] last state, first state, distance, g, h; then as int32
+                                    // [sel_cap] chosen pair per node (-1: none), [sel_cap] its primitive
   int32_t sel_cap = 0;
   bool sel_valid = false;           // the last expansion was a dp_expand_select
   bool select_mode = false;         // set while dp_expand_select enqueues its kernels
@@ -384,6 +400,28 @@ void dp_begin(long long* counters, int32_t* a, int64_t na, int32_t* b, int64_t n
 // counters[slot] receives the total when slot >= 0.
 void dp_scan_small(const int32_t* src, int32_t* dst, int64_t n, int32_t* total, int64_t cap, long long* counters,
                    int slot, hipStream_t s);
+
+// dp_visited_append_novel without its wait
+int dp_append_novel_async(dp_ctx* c);
+
+// Read-back: pair results packed into (pinned host) output arrays; null ones
+// are left out.
+struct dp_pack {
+  int64_t q0, n, pcap;
+  int nx;
+  const int32_t *node, *prim, *firstk, *goal;
+  const int8_t *verdict, *res;
+  const double *fin, *g, *h;
+  int32_t *o_node, *o_prim, *o_firstk, *o_goal;
+  int8_t *o_verdict, *o_res;
+  double *o_final, *o_g, *o_h;
+};
+void dp_pack_pairs(const dp_pack& a, hipStream_t s);
+// Row-major [n][nx] (and n values behind them for g, if not null) into
+// component arrays of `cap`.
+void dp_upload_rows(const double* src, int32_t n, int nx, int32_t cap, double* rows, double* g, hipStream_t s);
+// The batch counters into c->h_pinned.
+void dp_put_counters(dp_ctx* c, hipStream_t s);
 
 // ---- k_grid.hip ---------------------------------------------------------
 dp_grid_geom dp_make_grid(const dp_ctx* c, double r);

@@ -1173,6 +1173,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   const bool count = !c->select_mode && p->limit_branching_factor != 0 && !small;
   int rc = c->select_mode || small ? DP_OK : dp_ensure_cont_grid(c);
   if (rc) return rc;
+  c->counts_fresh = false;
   DP_EV(c->ev[0], s);
   dp_begin(c->d_counters, c->d_app_cnt, N, c->d_cont_count, count ? c->grid.nslots : 0, dp_stage(c, 1u << 0), s);
   const app_bounds B = make_app_bounds(c, r_app);
@@ -1306,8 +1307,9 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
         return DP_ERR_ARG;
       } else {
         a.marks = dp_stage(c, (1u << 6) | (1u << 2) | (1u << 7));
+        int32_t* sel_q = reinterpret_cast<int32_t*>(c->d_sel + (int64_t)(2 * nx + 3) * c->sel_cap);
         k_select<NX><<<N, 64, 0, s>>>(a, c->d_app, N, c->d_targets, c->d_cost, c->select_cost_jump,
-                                      c->select_first, c->d_sel_q, c->d_sel_q + c->sel_cap, c->d_sel);
+                                      c->select_first, sel_q, sel_q + c->sel_cap, c->d_sel);
         return DP_OK;
       }
     });

@@ -422,9 +422,9 @@ int dp_visited_radius_noalloc(dp_ctx* c, const double* d_queries, int64_t n, dou
   if (rc) return rc;
   rc = launch_radius(c, d_queries, n, radius, counts, d_offsets, d_idx, idx_cap, status, true, s);
   if (rc) return rc;
-  DP_HIP_RET(hipMemcpyAsync(c->h_pinned, status, sizeof(long long) * 2, hipMemcpyDeviceToHost, s));
+  DP_HIP_RET(hipMemcpyAsync(c->h_pinned + DPC_COUNT, status, sizeof(long long) * 2, hipMemcpyDeviceToHost, s));
   DP_HIP_RET(hipStreamSynchronize(s));
-  const long long total = c->h_pinned[0], longest = c->h_pinned[1];
+  const long long total = c->h_pinned[DPC_COUNT], longest = c->h_pinned[DPC_COUNT + 1];
   if (total > idx_cap) {
     dp_set_error("radius query output capacity exceeded (entries beyond idx_cap not written)");
     return DP_ERR_CAPACITY;

@@ -57,7 +57,63 @@ __global__ __launch_bounds__(1024) void k_scan_small(const int32_t* src, int32_t
   }
 }
 
+// Row-major pinned host memory ([n][nx], then n values of g) into component
+// arrays: one launch of a few us, read over the host link.
+__global__ void k_upload_rows(const double* __restrict__ src, int32_t n, int nx, int32_t ncap,
+                              double* __restrict__ nodes, double* __restrict__ g) {
+  const int64_t total = (int64_t)n * (nx + (g ? 1 : 0));
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
+    const double v = src[t];
+    if (t < (int64_t)n * nx) nodes[(t % nx) * (int64_t)ncap + t / nx] = v;
+    else g[t - (int64_t)n * nx] = v;
+  }
+}
+
+__global__ void k_put_counters(const long long* __restrict__ c, int n, long long* __restrict__ host) {
+  if ((int)threadIdx.x < n) host[threadIdx.x] = c[threadIdx.x];
+}
+
+// The results of pairs [q0, q0 + n) as the caller's arrays hold them, written
+// straight into pinned host memory: no final state, g or h but of a FREE pair
+// before its node's cap (NaN otherwise), no goal index past the cap.
+__global__ __launch_bounds__(256) void k_pack_pairs(dp_pack a) {
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < a.n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t q = a.q0 + t;
+    const int8_t v = a.verdict[q], r = a.res[q];
+    const bool capped = r == DP_R_CAPPED, has = v == DP_V_FREE && !capped;
+    if (a.o_node) a.o_node[t] = a.node[q];
+    if (a.o_prim) a.o_prim[t] = a.prim[q];
+    if (a.o_verdict) a.o_verdict[t] = v;
+    if (a.o_firstk) a.o_firstk[t] = a.firstk[q];
+    if (a.o_goal) a.o_goal[t] = capped ? -1 : a.goal[q];
+    if (a.o_res) a.o_res[t] = r;
+    if (a.o_g) a.o_g[t] = has ? a.g[q] : __longlong_as_double(0x7ff8000000000000ll);
+    if (a.o_h) a.o_h[t] = has ? a.h[q] : __longlong_as_double(0x7ff8000000000000ll);
+  }
+  if (a.o_final) {
+    const int nx = a.nx;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < a.n * nx;
+         t += (int64_t)gridDim.x * blockDim.x) {
+      const int64_t i = t / nx, q = a.q0 + i;
+      const int k = (int)(t - i * nx);
+      const bool has = a.verdict[q] == DP_V_FREE && a.res[q] != DP_R_CAPPED;
+      a.o_final[t] = has ? a.fin[(int64_t)k * a.pcap + q] : __longlong_as_double(0x7ff8000000000000ll);
+    }
+  }
+}
+
 }  // namespace
+
+void dp_upload_rows(const double* src, int32_t n, int nx, int32_t cap, double* rows, double* g, hipStream_t s) {
+  k_upload_rows<<<dp_grid_blocks((int64_t)n * (nx + 1), 256, 1024), 256, 0, s>>>(src, n, nx, cap, rows, g);
+}
+void dp_put_counters(dp_ctx* c, hipStream_t s) {
+  static_assert(DPC_COUNT <= 64, "one wave copies the counters");
+  k_put_counters<<<1, 64, 0, s>>>(c->d_counters, DPC_COUNT, c->h_pinned);
+}
+void dp_pack_pairs(const dp_pack& a, hipStream_t s) {
+  k_pack_pairs<<<dp_grid_blocks(a.n * (a.o_final ? a.nx : 1), 256, 2048), 256, 0, s>>>(a);
+}
 
 void dp_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s) {
   if (n <= 0) return;

@@ -315,7 +315,7 @@ int dp_search(dp_ctx* c, const double* start, const double* goal, const dp_searc
     po.g = pg.data();
     po.h = ph.data();
     if (n > 0 && (rc = dp_fetch_pairs(c, &po))) return rc;
-    if ((rc = dp_visited_append_novel(c))) return rc;
+    if ((rc = dp_append_novel_async(c))) return rc;
     t_gpu += now_ms() - tg;
     ++info->gpu_batches;
     info->pairs += n;
@@ -371,6 +371,10 @@ int dp_search(dp_ctx* c, const double* start, const double* goal, const dp_searc
     }
   }
 
+  if (hipStreamSynchronize(c->stream) != hipSuccess) {  // the last append
+    dp_set_error("hipStreamSynchronize failed");
+    return DP_ERR_HIP;
+  }
   if (status != DP_SEARCH_SOLVED) {  // closest node to the goal (dbastar.cpp:944-952)
     double best = INFINITY;
     for (size_t i = 0; i < nodes.size(); ++i) {
