@@ -9,12 +9,14 @@
 //                        the query's 27-cell block: the hit count
 //   k_radius_offsets     one workgroup: exclusive scan of the counts into
 //                        the CSR offsets, plus total and longest list
-//   k_radius<NX, true>   the same scan again, hits written at their offsets
-//   k_radius_sort        one workgroup per query: its list sorted in LDS
+//   k_radius<NX, true>   the same scan again, hits written at their offsets;
+//                        lists of up to 64 are sorted by their wave first
+//   k_radius_sort        one workgroup per query: longer lists sorted in LDS,
+//                        launched when there is one
 //
 // Two entry points share the kernels: dp_visited_radius (host buffers;
 // device buffers grown on demand) and dp_visited_radius_noalloc (device
-// buffers; no allocation: its per-query counts and status words live in the
+// buffers; no allocation: its per-query counts live in the
 // file-scope array `scratch` below, one copy per device).
 #include <hip/hip_runtime.h>
 
@@ -69,6 +71,7 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
   const int lane = threadIdx.x % 64;
   const uint64_t lt = (1ull << lane) - 1ull;
   const double T = dp_pos_bound(S, a.r);
+  __shared__ int32_t hits[4][64];
   const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
   for (int64_t q = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; q < a.n; q += nwaves) {
     double x[NX];
@@ -111,6 +114,11 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
     }
     const int K = __builtin_amdgcn_readlane(incl, 8);
     const int64_t base = FILL ? a.offsets[q] : 0;
+    const int64_t total = FILL ? a.offsets[q + 1] - base : 0;
+    // a list that fits a lane per entry is gathered in LDS and sorted here: a
+    // kernel for the lists of 8192 queries of a few neighbours took 5 us
+    const bool own = FILL && total <= 64 && base + total <= a.idx_cap;
+    int32_t* const list = hits[threadIdx.x / 64];
     int64_t cnt = 0;
     for (int j0 = 0; j0 < K; j0 += 64) {
       const int j = j0 + lane;
@@ -129,54 +137,88 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       }
       const uint64_t m = __ballot(hit);
       if (FILL && hit) {
-        const int64_t pos = base + cnt + __popcll(m & lt);
-        if (pos < a.idx_cap) a.idx[pos] = a.vperm[t];
+        const int64_t at = cnt + __popcll(m & lt);
+        if (own) list[at] = a.vperm[t];
+        else if (base + at < a.idx_cap) a.idx[base + at] = a.vperm[t];
       }
       cnt += __popcll(m);
+    }
+    if (own && total > 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      int32_t v = lane < total ? list[lane] : INT32_MAX;
+      // ascending bitonic network over the power of two that holds the list
+      for (int k = 2; k < 2 * total; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          const int32_t u = __shfl_xor(v, j);
+          const bool low = ((lane & j) == 0) == ((lane & k) == 0);
+          v = (u < v) == low ? u : v;
+        }
+      if (lane < total) a.idx[base + lane] = v;
     }
     if (!FILL && lane == 0) a.counts[q] = (int32_t)cnt;
   }
 }
 
 // Exclusive scan of counts[0..n) into offsets[0..n], one workgroup of 1024
-// threads, each over a contiguous chunk.  status[0] = total, status[1] =
-// longest list.
+// threads, four neighbouring counts each and 4096 at a time, the next on their
+// way (a run of n / 1024 counts per thread, one after another, took 14.5 us for
+// 8192 queries; this 6.4).  status[0] = total, status[1] = longest list; it may be
+// pinned host memory.
 __global__ __launch_bounds__(1024) void k_radius_offsets(const int32_t* __restrict__ counts, int64_t n,
                                                          int64_t* __restrict__ offsets, long long* __restrict__ status) {
-  __shared__ long long s[1024];
-  __shared__ int smax[1024];
-  const int t = threadIdx.x;
-  const int64_t chunk = (n + 1023) / 1024;
-  const int64_t b = t * chunk < n ? t * chunk : n;
-  const int64_t e = b + chunk < n ? b + chunk : n;
-  long long sum = 0;
+  __shared__ long long wsum[2][16];
+  __shared__ int wmax[16];
+  const int t = threadIdx.x, lane = t % 64, wave = t / 64;
+  auto load = [&](int64_t b, int32_t* v) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = b + k < n ? counts[b + k] : 0;
+  };
+  long long carry = 0;
   int mx = 0;
-  for (int64_t k = b; k < e; ++k) {
-    sum += counts[k];
-    mx = counts[k] > mx ? counts[k] : mx;
+  int32_t v[4], next[4];
+  load(4 * t, v);
+  int parity = 0;
+  for (int64_t b0 = 0; b0 < n; b0 += 4096, parity ^= 1) {
+    const int64_t b = b0 + 4 * t;
+    load(b + 4096, next);
+    const long long sum = (long long)v[0] + v[1] + v[2] + v[3];
+    long long incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const long long u = __shfl_up(incl, d);
+      if (lane >= d) incl += u;
+    }
+    if (lane == 63) wsum[parity][wave] = incl;
+    __syncthreads();
+    long long run = carry + incl - sum;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const long long u = wsum[parity][k];
+      if (k < wave) run += u;
+      carry += u;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (b + k < n) offsets[b + k] = run;
+      run += v[k];
+      mx = v[k] > mx ? v[k] : mx;
+      v[k] = next[k];
+    }
   }
-  s[t] = sum;
-  smax[t] = mx;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const int u = __shfl_xor(mx, d);
+    mx = u > mx ? u : mx;
+  }
+  if (lane == 0) wmax[wave] = mx;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const long long u = t >= off ? s[t - off] : 0;
-    __syncthreads();
-    s[t] += u;
-    __syncthreads();
-  }
-  for (int off = 512; off > 0; off >>= 1) {
-    if (t < off) smax[t] = smax[t + off] > smax[t] ? smax[t + off] : smax[t];
-    __syncthreads();
-  }
-  long long run = s[t] - sum;
-  for (int64_t k = b; k < e; ++k) {
-    offsets[k] = run;
-    run += counts[k];
-  }
-  if (t == 1023) {
-    offsets[n] = s[1023];
-    status[0] = s[1023];
-    status[1] = smax[0];
+  if (t == 0) {
+    for (int k = 1; k < 16; ++k) mx = wmax[k] > mx ? wmax[k] : mx;
+    offsets[n] = carry;
+    status[0] = carry;
+    status[1] = mx;
   }
 }
 
@@ -189,7 +231,7 @@ __global__ __launch_bounds__(256) void k_radius_sort(const int64_t* __restrict__
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
     const int64_t b = offsets[q], e = offsets[q + 1];
     const int64_t len = e - b;
-    if (len < 2 || len > DP_RADIUS_SORT_MAX || e > idx_cap) continue;
+    if (len <= 64 || len > DP_RADIUS_SORT_MAX || e > idx_cap) continue;  // up to 64: sorted by k_radius
     int p2 = 2;
     while (p2 < len) p2 <<= 1;
     for (int i = threadIdx.x; i < p2; i += blockDim.x) s[i] = i < len ? (int32_t)idx[b + i] : INT32_MAX;
@@ -240,11 +282,15 @@ int launch_radius(const dp_ctx* c, const double* d_queries, int64_t n, double ra
       k_radius_offsets<<<1, 1024, 0, s>>>(d_counts, n, d_offsets, d_status);
     } else {
       k_radius<NX, true><<<blocks, 256, 0, s>>>(a);
-      k_radius_sort<<<dp_grid_blocks(n, 1, 8192), 256, 0, s>>>(d_offsets, n, d_idx, idx_cap);
     }
     DP_HIP_RET(hipGetLastError());
     return DP_OK;
   });
+}
+
+// The lists past 64 entries, when the longest (known once the counts are) is one.
+void launch_sort(int64_t longest, const int64_t* d_offsets, int64_t n, int64_t* d_idx, int64_t idx_cap, hipStream_t s) {
+  if (longest > 64) k_radius_sort<<<dp_grid_blocks(n, 1, 8192), 256, 0, s>>>(d_offsets, n, d_idx, idx_cap);
 }
 
 // ---- device buffers of the allocating entry point ---------------------------
@@ -257,7 +303,6 @@ struct radius_bufs {
   int64_t off_cap = 0;
   int64_t* idx = nullptr;
   int64_t idx_cap = 0;
-  long long* status = nullptr;
 };
 
 template <typename T>
@@ -275,11 +320,9 @@ int grow(T** p, int64_t* cap, int64_t need) {
 }  // namespace
 
 // ---- the scratch of the allocation-free entry point -------------------------
-// Per-query hit counts (int32, DP_NOALLOC_MAX_QUERIES) followed by two status
-// words (total hits, longest list).  One copy per device, for the life of
-// the process; every call on a device reuses it.
-#define DP_NOALLOC_COUNTS_BYTES ((size_t)DP_NOALLOC_MAX_QUERIES * sizeof(int32_t))
-#define DP_NOALLOC_SCRATCH_BYTES (DP_NOALLOC_COUNTS_BYTES + 256)
+// Per-query hit counts (int32, DP_NOALLOC_MAX_QUERIES).  One copy per device,
+// for the life of the process; every call on a device reuses it.
+#define DP_NOALLOC_SCRATCH_BYTES ((size_t)DP_NOALLOC_MAX_QUERIES * sizeof(int32_t))
 static __device__ __align__(256) unsigned char scratch[DP_NOALLOC_SCRATCH_BYTES];
 
 namespace {
@@ -314,7 +357,6 @@ void dp_radius_free(dp_ctx* c) {
   (void)hipFree(b->cnt);
   (void)hipFree(b->off);
   (void)hipFree(b->idx);
-  (void)hipFree(b->status);
   delete b;
   c->radius = nullptr;
 }
@@ -350,22 +392,23 @@ int dp_visited_radius(dp_ctx* c, const double* queries, int64_t n, double radius
   }
   if (!c->radius) c->radius = new radius_bufs();
   radius_bufs* B = (radius_bufs*)c->radius;
+  long long* status = c->h_pinned + DPC_COUNT;
   const int nx = c->desc.nx;
   int rc;
   DP_HIP_RET(hipStreamSynchronize(s));  // buffers may grow below
   if ((rc = grow(&B->q, &B->q_cap, n * nx))) return rc;
   if ((rc = grow(&B->cnt, &B->cnt_cap, n))) return rc;
   if ((rc = grow(&B->off, &B->off_cap, n + 1))) return rc;
-  if (!B->status) DP_HIP_RET(hipMalloc((void**)&B->status, sizeof(long long) * 2));
   DP_HIP_RET(hipMemcpyAsync(B->q, queries, sizeof(double) * n * nx, hipMemcpyHostToDevice, s));
-  if ((rc = launch_radius(c, B->q, n, radius, B->cnt, B->off, nullptr, 0, B->status, false, s))) return rc;
-  long long st[2];
-  DP_HIP_RET(hipMemcpyAsync(st, B->status, sizeof(st), hipMemcpyDeviceToHost, s));
+  if ((rc = launch_radius(c, B->q, n, radius, B->cnt, B->off, nullptr, 0, status, false, s))) return rc;
   DP_HIP_RET(hipStreamSynchronize(s));
+  const long long st[2] = {status[0], status[1]};
   const int64_t keep = std::min<int64_t>(st[0], idx_cap);
   if (keep > 0) {
     if ((rc = grow(&B->idx, &B->idx_cap, keep))) return rc;
-    if ((rc = launch_radius(c, B->q, n, radius, B->cnt, B->off, B->idx, keep, B->status, true, s))) return rc;
+    if ((rc = launch_radius(c, B->q, n, radius, B->cnt, B->off, B->idx, keep, status, true, s))) return rc;
+    launch_sort(st[1], B->off, n, B->idx, keep, s);
+    DP_HIP_RET(hipGetLastError());
   }
   DP_HIP_RET(hipMemcpyAsync(out_offsets, B->off, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost, s));
   if (keep > 0) DP_HIP_RET(hipMemcpyAsync(out_idx, B->idx, sizeof(int64_t) * keep, hipMemcpyDeviceToHost, s));
@@ -411,7 +454,7 @@ int dp_visited_radius_noalloc(dp_ctx* c, const double* d_queries, int64_t n, dou
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   unsigned char* base = (unsigned char*)g_scratch_ptr[c->device];
   int32_t* counts = (int32_t*)base;
-  long long* status = (long long*)(base + DP_NOALLOC_COUNTS_BYTES);
+  long long* status = c->h_pinned + DPC_COUNT;  // written by the device
   if (n == 0 || c->nv == 0) {
     // every list is empty: offsets of zero counts
     DP_HIP_RET(hipMemsetAsync(d_offsets, 0, sizeof(int64_t) * (n + 1), s));
@@ -422,9 +465,13 @@ int dp_visited_radius_noalloc(dp_ctx* c, const double* d_queries, int64_t n, dou
   if (rc) return rc;
   rc = launch_radius(c, d_queries, n, radius, counts, d_offsets, d_idx, idx_cap, status, true, s);
   if (rc) return rc;
-  DP_HIP_RET(hipMemcpyAsync(c->h_pinned + DPC_COUNT, status, sizeof(long long) * 2, hipMemcpyDeviceToHost, s));
   DP_HIP_RET(hipStreamSynchronize(s));
-  const long long total = c->h_pinned[DPC_COUNT], longest = c->h_pinned[DPC_COUNT + 1];
+  const long long total = status[0], longest = status[1];
+  if (longest > 64) {
+    launch_sort(longest, d_offsets, n, d_idx, idx_cap, s);
+    DP_HIP_RET(hipGetLastError());
+    DP_HIP_RET(hipStreamSynchronize(s));
+  }
   if (total > idx_cap) {
     dp_set_error("radius query output capacity exceeded (entries beyond idx_cap not written)");
     return DP_ERR_CAPACITY;
