@@ -811,7 +811,7 @@ int dp_prepare_goal_index(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
 // capacity nothing is synchronised; otherwise the applicable pairs are counted
 // exactly first (one small device-to-host read) and the buffers grow to that
 // count plus 1/8 headroom.  Small batches reserve N * P outright.
-int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
+int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s, bool* counted) {
   const int64_t worst = (int64_t)c->N * c->P;
   const int64_t kOutright = 1ll << 22;
   int rc = dp_reserve(c, c->N, std::min(worst, kOutright));
@@ -822,10 +822,12 @@ int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     return rc;
   if (worst <= c->pair_cap) return DP_OK;
   if ((rc = dp_launch_count(c, p, s))) return rc;
-  long long total = 0;
-  HIP_CHECK(hipMemcpyAsync(c->h_pinned + DPC_COUNT, c->d_counters + DPC_PAIRS, sizeof(long long), hipMemcpyDeviceToHost, s));
+  if (counted) *counted = true;
+  c->counts_fresh = false;
+  dp_put_counters(c, s);
+  HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(s));
-  std::memcpy(&total, c->h_pinned + DPC_COUNT, sizeof(long long));
+  const long long total = c->h_pinned[DPC_PAIRS];
   if (total > c->pair_cap) {
     ARG_CHECK(total < (long long)INT32_MAX / 2, "more than 2^30 applicable pairs in one batch");
     rc = dp_reserve(c, c->N, std::min<int64_t>(worst, total + total / 8 + 1024));
@@ -851,9 +853,12 @@ int dp_expand(dp_ctx* c, const dp_expand_params* p, void* stream) {
   if (s != c->stream) c->outside = true;
   int rc = dp_prepare_goal_index(c, p, s);
   if (rc) return rc;
-  rc = dp_size_pairs(c, p, s);
+  bool counted = false;
+  rc = dp_size_pairs(c, p, s, &counted);
   if (rc) return rc;
+  c->app_ready = counted;
   rc = dp_launch_expand(c, p, s);
+  c->app_ready = false;
   c->last_pairs = -1;
   c->sel_valid = false;
   if (!rc) ++c->n_batches;
@@ -969,8 +974,11 @@ int dp_expand_select(dp_ctx* c, const double* targets, const dp_select_params* s
   c->select_radius = sp->radius;
   c->select_cost_jump = sp->cost_jump;
   c->select_first = sp->choose_first ? 1 : 0;
-  rc = dp_size_pairs(c, &p, s);
+  bool counted = false;
+  rc = dp_size_pairs(c, &p, s, &counted);
+  c->app_ready = counted;
   if (!rc) rc = dp_launch_expand(c, &p, s);
+  c->app_ready = false;
   c->select_mode = false;
   c->last_pairs = -1;
   c->sel_valid = rc == DP_OK;

@@ -283,6 +283,7 @@ struct dp_ctx {
   int32_t* d_node_cursor = nullptr; // [N_cap] first undecided pair per node
   int32_t* d_node_count = nullptr;  // [N_cap] NOVEL pairs decided per node
   long long* h_pinned = nullptr;    // [DPC_COUNT + 4] pinned host words: the batch counters as last read, then device totals
+  bool app_ready = false;           // dp_size_pairs just computed this batch's applicability
   bool counts_fresh = false;        // h_pinned holds the counters of the last expansion, its work finished
   // Pinned staging of uploads and read-back, grown on demand to at most
   // DP_STAGE_MAX bytes each (larger results go through in pieces).
@@ -503,7 +504,11 @@ int dp_launch_count(dp_ctx* c, const dp_expand_params* p, hipStream_t s);
 void dp_bump_epoch();
 uint64_t dp_epoch();
 int dp_prepare_goal_index(dp_ctx* c, const dp_expand_params* p, hipStream_t s);
-int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s);
+// `counted` (or null): set when the applicability masks and counts of the
+// uploaded nodes were computed on the way, so that dp_launch_expand of the same
+// parameters on the same stream, next, can be told (dp_ctx::app_ready) not to
+// compute them again.  A launch that is captured must not be told.
+int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s, bool* counted = nullptr);
 
 // Any visited state within r of x in run k (0..8) of x's 27-cell block?  The
 // block is 9 runs of 3 cells adjacent in memory (x is the fastest grid axis):

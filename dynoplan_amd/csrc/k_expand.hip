@@ -1,21 +1,24 @@
 // k_expand.hip -- gfx950 kernels of the batched db-A* expansion.
 //
 // Pipeline of one dp_expand (all on one stream, no host round trip):
-//   k_app_count       one wave per node: applicability query nearestR(c, alpha*delta)
-//                     over primitive start states (Expander::expand_lazy,
-//                     dbastar.hpp:270-312), brute force with exact early
-//                     rejections, one bit mask per 64 primitives, counted
-//   k_scan            exclusive scan -> canonical pair offsets per node
-//   k_app_fill        the masks as the (node, primitive) pair list
-//   k_check_planar    LPP lanes per pair, one lane per primitive state:
-//                     translate (transform_primitive), is_state_valid on every
-//                     state, swept-box cull of LDS-staged obstacles, SAT
-//                     per state, first offending index by ballot
-//                     (check_lazy_trajectory, dbastar.cpp:391-490), check_goal
-//                     (:492-512), g/h (:833-847), duplicate test against the
-//                     visited grid (:850-854)
-//   k_grid.hip        contender grid, earlier-conflict lists and the round-
-//                     based duplicate / branching-cap resolution (:856-918)
+//   k_begin           counters, counts and grid cells cleared, one launch
+//   k_app_blk         applicability query nearestR(c, alpha*delta) over primitive
+//                     start states (Expander::expand_lazy, dbastar.hpp:270-312),
+//                     brute force with exact early rejections, one bit mask per
+//                     64 primitives, counted (k_app_count with a pair order per
+//                     node)
+//   k_app_fill        the masks as the (node, primitive) pair list; up to 1024
+//                     nodes it scans the counts itself
+//   k_check_planar    one lane per pair, then one lane per (state, obstacle) or
+//                     visited candidate: translate (transform_primitive),
+//                     is_state_valid on every state, swept-box cull of the
+//                     node's obstacles in LDS, SAT per state, first offending
+//                     index (check_lazy_trajectory, dbastar.cpp:391-490),
+//                     check_goal (:492-512), g/h (:833-847), duplicate test
+//                     against the visited grid (:850-854), contenders counted
+//                     into their grid cells
+//   k_grid.hip        contender grid, earlier-conflict lists and the ordered
+//                     duplicate / branching-cap resolution (:856-918)
 #include <hip/hip_runtime.h>
 #include <float.h>
 #include <limits.h>
@@ -952,10 +955,13 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
 // in pair order, the first with the smallest distance(last placed state,
 // target) below DBL_MAX (the reference starts from
 // numeric_limits<double>::max() and keeps a candidate only when d < min), or
-// the first FREE one with choose_first.  One wave per node.  Writes the pair
-// index (-1: none) and [last state, first state, distance, g, h].
+// the first FREE one with choose_first.  Writes the pair index (-1: none) and
+// [last state, first state, distance, g, h].  Bounded by four dependent loads
+// per chunk of pairs, so a node's chunks go to four waves at once (one wave per
+// node, chunk after chunk: 30 us for 1000 nodes of 175 pairs; this 20).
+constexpr int kSelectWaves = 4;
 template <int NX>
-__global__ __launch_bounds__(64) void k_select(dp_check_args a, const int32_t* __restrict__ app, int32_t N,
+__global__ __launch_bounds__(64 * kSelectWaves) void k_select(dp_check_args a, const int32_t* __restrict__ app, int32_t N,
                                                const double* __restrict__ targets, const double* __restrict__ cost,
                                                double cost_jump, int32_t choose_first, int32_t* __restrict__ sel_q,
                                                int32_t* __restrict__ sel_prim, double* __restrict__ sel) {
@@ -963,7 +969,9 @@ __global__ __launch_bounds__(64) void k_select(dp_check_args a, const int32_t* _
   const dp_dev_sys& S = *a.sys;
   const int32_t i = blockIdx.x;
   if (i >= N) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  __shared__ double wave_d[kSelectWaves];
+  __shared__ int32_t wave_q[kSelectWaves];
   const int32_t tot = *a.total;
   const int32_t b = app[i] < tot ? app[i] : tot;
   const int32_t e = app[i + 1] < tot ? app[i + 1] : tot;
@@ -973,7 +981,7 @@ __global__ __launch_bounds__(64) void k_select(dp_check_args a, const int32_t* _
   const double ox = a.nodes[i], oy = a.nodes[(int64_t)a.Ncap + i];
   double best_d = DBL_MAX;
   int32_t best_q = -1;
-  for (int32_t cb = b; cb < e; cb += 64) {
+  for (int32_t cb = b + 64 * wave; cb < e; cb += 64 * kSelectWaves) {
     const int32_t q = cb + lane;
     double d = DBL_MAX;
     bool ok = false;
@@ -1009,6 +1017,26 @@ __global__ __launch_bounds__(64) void k_select(dp_check_args a, const int32_t* _
     if (mq != INT_MAX && md < best_d) {  // strictly below every earlier chunk's minimum
       best_d = md;
       best_q = mq;
+    }
+  }
+  // the waves' choices: the smallest distance, then the lowest pair (with
+  // choose_first the lowest pair)
+  if (lane == 0) {
+    wave_d[wave] = best_d;
+    wave_q[wave] = best_q;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  best_q = -1;
+#pragma unroll
+  for (int w = 0; w < kSelectWaves; ++w) {
+    const double d = wave_d[w];
+    const int32_t q = wave_q[w];
+    if (q < 0) continue;
+    const bool better = best_q < 0 || (choose_first ? q < best_q : d < best_d || (d == best_d && q < best_q));
+    if (better) {
+      best_d = d;
+      best_q = q;
     }
   }
   if (lane == 0) {
@@ -1175,11 +1203,13 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
   if (rc) return rc;
   c->counts_fresh = false;
   DP_EV(c->ev[0], s);
-  dp_begin(c->d_counters, c->d_app_cnt, N, c->d_cont_count, count ? c->grid.nslots : 0, dp_stage(c, 1u << 0), s);
+  dp_begin(c->d_counters, c->d_app_cnt, c->app_ready ? 0 : N, c->d_cont_count, count ? c->grid.nslots : 0, dp_stage(c, 1u << 0), s);
   const app_bounds B = make_app_bounds(c, r_app);
   rc = dispatch_nx(nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
-    launch_app<NX>(c, B, r_app, s);
+    // counted already when the batch did not fit its pair arrays outright
+    // (1000 nodes x 5000 primitives: 15 us of a steering selection's 234)
+    if (!c->app_ready) launch_app<NX>(c, B, r_app, s);
     fill_args f{};
     f.N = N;
     f.P = c->P;
@@ -1308,7 +1338,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
       } else {
         a.marks = dp_stage(c, (1u << 6) | (1u << 2) | (1u << 7));
         int32_t* sel_q = reinterpret_cast<int32_t*>(c->d_sel + (int64_t)(2 * nx + 3) * c->sel_cap);
-        k_select<NX><<<N, 64, 0, s>>>(a, c->d_app, N, c->d_targets, c->d_cost, c->select_cost_jump,
+        k_select<NX><<<N, 64 * kSelectWaves, 0, s>>>(a, c->d_app, N, c->d_targets, c->d_cost, c->select_cost_jump,
                                       c->select_first, sel_q, sel_q + c->sel_cap, c->d_sel);
         return DP_OK;
       }

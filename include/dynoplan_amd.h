@@ -274,7 +274,7 @@ int dp_fetch_pairs(dp_ctx* ctx, dp_pairs_out* out);
 void* dp_stream(dp_ctx* ctx);
 
 /* Device time (ms) of the kernels of the last dp_expand, split by stage
- * (HIP events on the expansion stream), ms5[5]: 0 applicability, 1 check,
+ * (the device clock at the first kernel of a stage), ms5[5]: 0 applicability, 1 check,
  * 2 duplicate resolution, 3 total, 4 learned pre-filter (0 without it). */
 int dp_last_timing(dp_ctx* ctx, float* ms5);
 /* The same split per kernel group, ms7[7]: 0 applicability, 1 learned
