@@ -8,7 +8,7 @@ set and the ordered in-batch duplicate / branching-cap resolution.  The unit
 is one (frontier node, applicable primitive) pair that received a verdict.
 
 Printed: ONE JSON line with the batched throughput (``value``), the roofline
-of the dominant kernel (HIP events on the expansion stream), the plain GPU
+of the dominant kernel (device clock at the first kernel of each stage), the plain GPU
 path (one node per call, as the reference's loop pops one node at a time)
 and the CPU FP64 oracle timed on a bounded sample of the same workload.
 """
@@ -49,13 +49,13 @@ def workloads():
     }
 
 
-# Kernel groups timed by dp_last_timing_detail (HIP events on the expansion
-# stream), per system family.
+# Kernel groups timed by dp_last_timing_detail (device clock at the stages'
+# first kernels), per system family.
 KERNEL_GROUPS = {
     "check_main": {"quad": "k_quad32", "planar": "k_check_planar"},
     "check_post": {"quad": "k_quad_window + k_quad64 (with the visited duplicate test)", "planar": "(none)"},
-    "lists": {"quad": "k_cont_count + k_cont_scatter + k_cell_list + k_conf_waves (+ fills, scans)",
-              "planar": "k_cont_count + k_cont_scatter + k_cell_list + k_conf_waves (+ fills, scans)"},
+    "lists": {"quad": "k_cell_rows + k_cont_scatter + k_conf_waves",
+              "planar": "k_cell_rows + k_cont_scatter + k_conf_waves"},
     "walk": {"quad": "k_pre_nodes + k_resolve_ticketed",
              "planar": "k_pre_nodes + k_resolve_ticketed"},
 }
@@ -420,7 +420,7 @@ def main():
     pairs = counts["pairs"]
     value = pairs * args.steps / elapsed
 
-    # Per-stage and per-kernel-group device time from HIP events recorded on
+    # Per-stage and per-kernel-group device time from the device clock, read on
     # the expansion stream, over as many further steps.
     stage = {"applicability": [], "surrogate": [], "check": [], "resolve": [], "total": []}
     detail = {k: [] for k in ("applicability", "surrogate", "check_pre", "check_main", "check_post", "lists", "walk")}
