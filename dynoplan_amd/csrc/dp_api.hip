@@ -1044,9 +1044,12 @@ int dp_expand_batch(dp_ctx* c, const double* nodes, const double* g_parent, int3
   return DP_OK;
 }
 
+// Selects the context's device even when the counters are at hand: what the
+// callers allocate and launch afterwards (the end of a batch the device left
+// unfinished, a larger visited set) belongs there.
 static int read_counters(dp_ctx* c, long long* h) {
+  HIP_CHECK(hipSetDevice(c->device));
   if (!c->counts_fresh) {
-    HIP_CHECK(hipSetDevice(c->device));
     int rc = settle(c);
     if (rc) return rc;
     dp_put_counters(c, c->stream);

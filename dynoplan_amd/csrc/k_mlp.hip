@@ -996,6 +996,7 @@ int dp_surrogate_scores(dp_ctx* c, float* out, int64_t n) {
     dp_set_error("invalid argument or no scores");
     return DP_ERR_ARG;
   }
+  DP_HIP_RET(hipSetDevice(c->device));
   DP_HIP_RET(hipDeviceSynchronize());
   DP_HIP_RET(hipMemcpy(out, c->mlp.score, sizeof(float) * n, hipMemcpyDeviceToHost));
   return DP_OK;
