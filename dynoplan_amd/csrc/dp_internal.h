@@ -229,7 +229,9 @@ struct dp_ctx {
   // visited set (T_n)
   int64_t nv = 0, nv_cap = 0;
   int64_t nv_sorted = 0;           // states the grid holds; [nv_sorted, nv) lie behind them, unsorted, and every
-                                   // duplicate test reads them as one more run
+                                   // duplicate test and radius query reads them as one more run
+  int64_t nv_ready = 0;            // states at the last expansion or radius query: the allocation-free query
+                                   // answers for these
   double* d_vis = nullptr;         // [nx][nv_cap] append order
   double* d_vis_sorted = nullptr;  // [nx][nv_cap] sorted by cell
   int32_t* d_vis_cell = nullptr;   // scratch [nv_cap]

@@ -1196,6 +1196,7 @@ int dp_launch_expand(dp_ctx* c, const dp_expand_params* p, hipStream_t s) {
     int rc = dp_launch_visited_rebuild(c, r_dup, s);
     if (rc) return rc;
   }
+  if (!c->select_mode) c->nv_ready = c->nv;
 
   // The check stage counts the contenders into their grid cells as it finds
   // them; limit 0 takes pairs out again after it (k_precap_first), so there

@@ -50,7 +50,8 @@ struct radius_args {
   const int32_t* vstart;   // [nslots] visited grid cell offsets
   const double* vis;       // [nx][vstride] visited states sorted by cell
   int64_t vstride;
-  const int32_t* vperm;    // [nv] sorted position -> append index
+  const int32_t* vperm;    // [nv_sorted] sorted position -> append index
+  int64_t nv, nv_sorted;   // states behind the sorted ones lie in append order
   const double* queries;   // [n][nx] row-major
   int64_t n;
   double r;
@@ -62,8 +63,9 @@ struct radius_args {
 
 // One wave per query.  Lanes 0..8 locate the 9 runs of the 27-cell block
 // (rows c1-1..c1+1, layers c2-1..c2+1, x from c0-1 to c0+1 clipped: the rules
-// of dp_cell_neighbor), then the candidates of all runs are numbered 0..K-1
-// and lane l tests l, l+64, ...; hits are ballot-compacted.
+// of dp_cell_neighbor), lane 9 the unsorted tail of the visited set, then the
+// candidates of all runs are numbered 0..K-1 and lane l tests l, l+64, ...;
+// hits are ballot-compacted.
 template <int NX, bool FILL>
 __global__ __launch_bounds__(256) void k_radius(radius_args a) {
   const dp_dev_sys& S = *a.sys;
@@ -99,6 +101,9 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
         st = a.vstart[row + x0];
         len = a.vstart[row + x1 + 1] - st;
       }
+    } else if (lane == 9) {
+      st = (int)a.nv_sorted;
+      len = (int)(a.nv - a.nv_sorted);
     }
     int incl = len;
 #pragma unroll
@@ -106,13 +111,13 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       const int v = __shfl_up(incl, d, 64);
       if (lane >= d) incl += v;
     }
-    int32_t rs[9], rp[9];
+    int32_t rs[10], rp[10];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
+    for (int k = 0; k < 10; ++k) {
       rs[k] = __builtin_amdgcn_readlane(st, k);
       rp[k] = __builtin_amdgcn_readlane(incl - len, k);
     }
-    const int K = __builtin_amdgcn_readlane(incl, 8);
+    const int K = __builtin_amdgcn_readlane(incl, 9);
     const int64_t base = FILL ? a.offsets[q] : 0;
     const int64_t total = FILL ? a.offsets[q + 1] - base : 0;
     // a list that fits a lane per entry is gathered in LDS and sorted here: a
@@ -127,10 +132,10 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       if (j < K) {
         int k = 0;
 #pragma unroll
-        for (int kk = 1; kk < 9; ++kk) k += j >= rp[kk] ? 1 : 0;
+        for (int kk = 1; kk < 10; ++kk) k += j >= rp[kk] ? 1 : 0;
         int32_t sk = rs[0], pk = rp[0];
 #pragma unroll
-        for (int kk = 1; kk < 9; ++kk)
+        for (int kk = 1; kk < 10; ++kk)
           if (k == kk) sk = rs[kk], pk = rp[kk];
         t = sk + (j - pk);
         hit = dp_within_col_pf<NX>(S, x, a.vis, a.vstride, t, a.r, T);
@@ -138,8 +143,9 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       const uint64_t m = __ballot(hit);
       if (FILL && hit) {
         const int64_t at = cnt + __popcll(m & lt);
-        if (own) list[at] = a.vperm[t];
-        else if (base + at < a.idx_cap) a.idx[base + at] = a.vperm[t];
+        const int32_t v = t < a.nv_sorted ? a.vperm[t] : t;
+        if (own) list[at] = v;
+        else if (base + at < a.idx_cap) a.idx[base + at] = v;
       }
       cnt += __popcll(m);
     }
@@ -267,6 +273,8 @@ int launch_radius(const dp_ctx* c, const double* d_queries, int64_t n, double ra
   a.vis = c->d_vis_sorted;
   a.vstride = c->nv_cap;
   a.vperm = c->d_vis_perm;
+  a.nv = c->nv;
+  a.nv_sorted = c->nv_sorted;
   a.queries = d_queries;
   a.n = n;
   a.r = radius;
@@ -386,6 +394,7 @@ int dp_visited_radius(dp_ctx* c, const double* queries, int64_t n, double radius
     int rc = dp_launch_visited_rebuild(c, radius, s);
     if (rc) return rc;
   }
+  c->nv_ready = c->nv;
   if (c->nv == 0) {
     for (int64_t q = 0; q <= n; ++q) out_offsets[q] = 0;
     return DP_OK;
@@ -441,7 +450,7 @@ int dp_visited_radius_noalloc(dp_ctx* c, const double* d_queries, int64_t n, dou
     dp_set_error("radius must be finite and >= 0");
     return DP_ERR_ARG;
   }
-  if (c->nv > 0 && (c->grid_dirty || c->nv != c->nv_sorted || !(c->grid_radius >= radius))) {
+  if (c->nv > 0 && (c->grid_dirty || c->nv != c->nv_ready || !(c->grid_radius >= radius))) {
     dp_set_error("the visited grid is not built for this radius: call dp_visited_radius or dp_expand once "
                  "after the last change of the visited set");
     return DP_ERR_STATE;
