@@ -2006,7 +2006,12 @@ int dp_launch_resolve_again(dp_ctx* c, hipStream_t s) {
                                                                            c->d_res, c->d_counters);
   DP_HIP_RET(hipGetLastError());
   const dp_expand_params p = c->round_params;
-  return dp_launch_resolve(c, &p, c->round_r_dup, false, s);
+  // the stage marks belong to the expansion, not to its completion by the host
+  const bool quiet = c->no_events;
+  c->no_events = true;
+  const int rc = dp_launch_resolve(c, &p, c->round_r_dup, false, s);
+  c->no_events = quiet;
+  return rc;
 }
 
 int dp_launch_more_rounds(dp_ctx* c, int rounds, hipStream_t s) {
