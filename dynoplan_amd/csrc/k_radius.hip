@@ -144,8 +144,13 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       if (FILL && hit) {
         const int64_t at = cnt + __popcll(m & lt);
         const int32_t v = t < a.nv_sorted ? a.vperm[t] : t;
-        if (own) list[at] = v;
-        else if (base + at < a.idx_cap) a.idx[base + at] = v;
+        // (a capacity of its own for the LDS list: calls that overlap on one
+        // device race on the counts, and `total` may not be this scan's)
+        if (own) {
+          if (at < 64) list[at] = v;
+        } else if (base + at < a.idx_cap) {
+          a.idx[base + at] = v;
+        }
       }
       cnt += __popcll(m);
     }
