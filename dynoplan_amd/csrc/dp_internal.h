@@ -512,18 +512,30 @@ int dp_prepare_goal_index(dp_ctx* c, const dp_expand_params* p, hipStream_t s);
 // compute them again.  A launch that is captured must not be told.
 int dp_size_pairs(dp_ctx* c, const dp_expand_params* p, hipStream_t s, bool* counted = nullptr);
 
+// Visited states an expansion may leave unsorted: every FREE pair tests each
+// of them, a rebuild of the grid is four launches (20 us).
+//
+// Planar: the check deals the tail over its lanes, so what counts is the tail
+// times the combinations.  At 1000 combinations and 20 new states per batch,
+// 524 states at most cost 7 us a batch on average and 262 cost 3.5, against 1
+// and 2 us of rebuilding.  Batches of few combinations have few waves to share
+// a long tail (up to 13k states at 1 x 20: 81 to 156 us a step of expansion
+// and append, where a rebuild each time takes 79 to 101); past 1024 states a
+// rebuild costs less than 0.5 us a batch.
+// Quadrotor: the FP64 pass walks the tail in each lane, 0.2 us a state whatever
+// the combinations, so 64 states cost as much as the rebuilds they save (one
+// node of 100 primitives, 92% FREE, up to 2621 states: 318 us a step, 128 with
+// a rebuild each time).
+inline bool dp_tail_fits(const dp_ctx* c) {
+  const int64_t tail = c->nv - c->nv_sorted;
+  if (tail > (c->desc.system == DP_SYS_QUADROTOR ? 64 : 1024)) return false;
+  return tail * (int64_t)c->N * c->P <= (1ll << 18);
+}
+
 // Any visited state within r of x in run k (0..8) of x's 27-cell block?  The
 // block is 9 runs of 3 cells adjacent in memory (x is the fastest grid axis):
 // run k covers rows c1 + k%3 - 1 and layers c2 + k/3 - 1 (the rules of
 // dp_cell_neighbor), x from c0 - 1 to c0 + 1 clipped to the grid.
-// Visited states an expansion may leave unsorted: the tail costs every FREE
-// pair one test per state, a rebuild of the grid four launches (20 us).  At
-// 1000 combinations and 20 new states per batch, 524 states at most cost 7 us
-// a batch on average and 262 cost 3.5, against 1 and 2 us of rebuilding.
-inline bool dp_tail_fits(const dp_ctx* c) {
-  return (c->nv - c->nv_sorted) * (int64_t)c->N * c->P <= (1ll << 18);
-}
-
 template <int NX>
 __device__ __forceinline__ bool dp_grid_run_any(const dp_dev_sys& S, const dp_grid_geom& G, const int32_t* start,
                                              const double* pts, int64_t stride, const double* x, int k, double r,
