@@ -491,6 +491,7 @@ __device__ __forceinline__ void load_translated(const dp_check_args& a, int64_t 
 // another and dealt to the 64 lanes in turn.  A bitmap of the segments' first
 // items gives an item's segment by a bit count, kItemWindow items at a time.
 constexpr int kItemWindow = 4096;
+constexpr int kPairItems = 1 << 20;  // visited candidates of a pair past which it is a list of its own
 
 // Per-wave LDS of k_check_planar (6 KB for three components, 7 KB for five).
 template <int NX>
@@ -880,38 +881,47 @@ __global__ __launch_bounds__(256) void k_check_planar(dp_check_args a) {
           nr += rn[k] > 0 ? 1 : 0;
         }
       }
-      const int incl = wave_incl_scan(K, lane), run0 = wave_incl_scan(nr, lane) - nr;
-      const int T = __builtin_amdgcn_readlane(incl, 63);
-      {
-        int f = incl - K, at = run0;
-#pragma unroll
-        for (int k = 0; k < 10; ++k)
-          if (rn[k] > 0) {
-            W.vis.run[at++] = make_int2(lane, rb[k] - f);
-            f += rn[k];
-          }
-      }
       W.bad[lane] = 0;
 #pragma unroll
       for (int c = 0; c < NX; ++c) W.vis.x[c][lane] = xf[c];
-      for_items(
-          W.head, T, lane,
-          [&](int w0) {
-            int f = incl - K;
+      // The items of 64 pairs are numbered in 31 bits.  A pair of more than
+      // kPairItems candidates (a set of that many states within a block) could
+      // take the sum past them: then the wave's pairs go one after another.
+      const bool alone = __ballot(K > kPairItems) != 0;
+      for (uint64_t left = alone ? __ballot(K > 0) : 1ull; left; left &= left - 1ull) {
+        const bool in = !alone || lane == __ffsll((long long)left) - 1;
+        const int n = in ? K : 0, runs = in ? nr : 0;
+        const int incl = wave_incl_scan(n, lane), run0 = wave_incl_scan(runs, lane) - runs;
+        const int T = __builtin_amdgcn_readlane(incl, 63);
+        if (in) {
+          int f = incl - n, at = run0;
 #pragma unroll
-            for (int k = 0; k < 10; ++k)
-              if (rn[k] > 0) {
-                mark_item(W.head, f, w0);
-                f += rn[k];
-              }
-          },
-          [&](int run, int f) {
-            const int2 r = W.vis.run[run];
-            double x[NX];
+          for (int k = 0; k < 10; ++k)
+            if (rn[k] > 0) {
+              W.vis.run[at++] = make_int2(lane, rb[k] - f);
+              f += rn[k];
+            }
+        }
+        for_items(
+            W.head, T, lane,
+            [&](int w0) {
+              if (!in) return;
+              int f = incl - n;
 #pragma unroll
-            for (int c = 0; c < NX; ++c) x[c] = W.vis.x[c][r.x];
-            if (dp_within_col_pf<NX>(S, x, a.vis, a.vstride, (int64_t)f + r.y, a.r_dup, Tdup)) W.bad[r.x] = 1;
-          });
+              for (int k = 0; k < 10; ++k)
+                if (rn[k] > 0) {
+                  mark_item(W.head, f, w0);
+                  f += rn[k];
+                }
+            },
+            [&](int run, int f) {
+              const int2 r = W.vis.run[run];
+              double x[NX];
+#pragma unroll
+              for (int c = 0; c < NX; ++c) x[c] = W.vis.x[c][r.x];
+              if (dp_within_col_pf<NX>(S, x, a.vis, a.vstride, (int64_t)f + r.y, a.r_dup, Tdup)) W.bad[r.x] = 1;
+            });
+      }
       dupv = fr && W.bad[lane] != 0;
       wave_lds_sync();
     }
