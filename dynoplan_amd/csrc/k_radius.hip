@@ -5,11 +5,11 @@
 // For each query state: the indices (append order of the visited set) of
 // every visited state within `radius` under the system metric, ascending,
 // as CSR.  Three kernels:
-//   k_radius<NX, false>  one wave per query over the 9 x-contiguous runs of
+//   k_radius (count)     one wave per query over the 9 x-contiguous runs of
 //                        the query's 27-cell block: the hit count
 //   k_radius_offsets     one workgroup: exclusive scan of the counts into
 //                        the CSR offsets, plus total and longest list
-//   k_radius<NX, true>   the same scan again, hits written at their offsets;
+//   k_radius (fill)      the same scan again, hits written at their offsets;
 //                        lists of up to 64 are sorted by their wave first
 //   k_radius_sort        one workgroup per query: longer lists sorted in LDS,
 //                        launched when there is one
@@ -51,22 +51,28 @@ struct radius_args {
   const double* vis;       // [nx][vstride] visited states sorted by cell
   int64_t vstride;
   const int32_t* vperm;    // [nv_sorted] sorted position -> append index
-  int64_t nv, nv_sorted;   // states behind the sorted ones lie in append order
   const double* queries;   // [n][nx] row-major
   int64_t n;
   double r;
-  int32_t* counts;         // [n]
-  const int64_t* offsets;  // [n+1] (fill pass)
+  union {
+    int32_t* counts;         // [n] (count pass)
+    const int64_t* offsets;  // [n+1] (fill pass)
+  };
   int64_t* idx;            // [idx_cap] (fill pass)
   int64_t idx_cap;
+  int32_t nv, nv_sorted;   // states behind the sorted ones lie in append order
 };
+// The launch sizes behind the arguments end with their third cache line: read
+// from a fourth they cost each pass 0.26 us of 7.
+static_assert(sizeof(radius_args) <= 176, "k_radius's arguments fit three cache lines with the launch sizes");
 
 // One wave per query.  Lanes 0..8 locate the 9 runs of the 27-cell block
 // (rows c1-1..c1+1, layers c2-1..c2+1, x from c0-1 to c0+1 clipped: the rules
-// of dp_cell_neighbor), lane 9 the unsorted tail of the visited set, then the
-// candidates of all runs are numbered 0..K-1 and lane l tests l, l+64, ...;
-// hits are ballot-compacted.
-template <int NX, bool FILL>
+// of dp_cell_neighbor), then the candidates of all runs are numbered 0..K-1
+// and lane l tests l, l+64, ...; hits are ballot-compacted.  TAIL: the
+// unsorted tail of the visited set behind them, in a kernel of its own so that
+// queries without one do not pay for the loop.
+template <int NX, bool FILL, bool TAIL>
 __global__ __launch_bounds__(256) void k_radius(radius_args a) {
   const dp_dev_sys& S = *a.sys;
   const dp_grid_geom& G = a.grid;
@@ -101,9 +107,6 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
         st = a.vstart[row + x0];
         len = a.vstart[row + x1 + 1] - st;
       }
-    } else if (lane == 9) {
-      st = (int)a.nv_sorted;
-      len = (int)(a.nv - a.nv_sorted);
     }
     int incl = len;
 #pragma unroll
@@ -111,13 +114,13 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       const int v = __shfl_up(incl, d, 64);
       if (lane >= d) incl += v;
     }
-    int32_t rs[10], rp[10];
+    int32_t rs[9], rp[9];
 #pragma unroll
-    for (int k = 0; k < 10; ++k) {
+    for (int k = 0; k < 9; ++k) {
       rs[k] = __builtin_amdgcn_readlane(st, k);
       rp[k] = __builtin_amdgcn_readlane(incl - len, k);
     }
-    const int K = __builtin_amdgcn_readlane(incl, 9);
+    const int K = __builtin_amdgcn_readlane(incl, 8);
     const int64_t base = FILL ? a.offsets[q] : 0;
     const int64_t total = FILL ? a.offsets[q + 1] - base : 0;
     // a list that fits a lane per entry is gathered in LDS and sorted here: a
@@ -125,6 +128,16 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
     const bool own = FILL && total <= 64 && base + total <= a.idx_cap;
     int32_t* const list = hits[threadIdx.x / 64];
     int64_t cnt = 0;
+    // a hit's place in the query's list, its append index v there
+    auto put = [&](int64_t at, int32_t v) {
+      // (a bound of its own for the LDS list: calls that overlap on one device
+      // race on the counts, and `total` may not be this scan's)
+      if (own) {
+        if (at < 64) list[at] = v;
+      } else if (base + at < a.idx_cap) {
+        a.idx[base + at] = v;
+      }
+    };
     for (int j0 = 0; j0 < K; j0 += 64) {
       const int j = j0 + lane;
       bool hit = false;
@@ -132,26 +145,23 @@ __global__ __launch_bounds__(256) void k_radius(radius_args a) {
       if (j < K) {
         int k = 0;
 #pragma unroll
-        for (int kk = 1; kk < 10; ++kk) k += j >= rp[kk] ? 1 : 0;
+        for (int kk = 1; kk < 9; ++kk) k += j >= rp[kk] ? 1 : 0;
         int32_t sk = rs[0], pk = rp[0];
 #pragma unroll
-        for (int kk = 1; kk < 10; ++kk)
+        for (int kk = 1; kk < 9; ++kk)
           if (k == kk) sk = rs[kk], pk = rp[kk];
         t = sk + (j - pk);
         hit = dp_within_col_pf<NX>(S, x, a.vis, a.vstride, t, a.r, T);
       }
       const uint64_t m = __ballot(hit);
-      if (FILL && hit) {
-        const int64_t at = cnt + __popcll(m & lt);
-        const int32_t v = t < a.nv_sorted ? a.vperm[t] : t;
-        // (a capacity of its own for the LDS list: calls that overlap on one
-        // device race on the counts, and `total` may not be this scan's)
-        if (own) {
-          if (at < 64) list[at] = v;
-        } else if (base + at < a.idx_cap) {
-          a.idx[base + at] = v;
-        }
-      }
+      if (FILL && hit) put(cnt + __popcll(m & lt), a.vperm[t]);
+      cnt += __popcll(m);
+    }
+    for (int64_t t0 = a.nv_sorted; TAIL && t0 < (int64_t)a.nv; t0 += 64) {
+      const int64_t t = t0 + lane;
+      const bool hit = t < (int64_t)a.nv && dp_within_col_pf<NX>(S, x, a.vis, a.vstride, t, a.r, T);
+      const uint64_t m = __ballot(hit);
+      if (FILL && hit) put(cnt + __popcll(m & lt), (int32_t)t);
       cnt += __popcll(m);
     }
     if (own && total > 0) {
@@ -278,23 +288,26 @@ int launch_radius(const dp_ctx* c, const double* d_queries, int64_t n, double ra
   a.vis = c->d_vis_sorted;
   a.vstride = c->nv_cap;
   a.vperm = c->d_vis_perm;
-  a.nv = c->nv;
-  a.nv_sorted = c->nv_sorted;
+  a.nv = (int32_t)c->nv;
+  a.nv_sorted = (int32_t)c->nv_sorted;
   a.queries = d_queries;
   a.n = n;
   a.r = radius;
-  a.counts = d_counts;
-  a.offsets = d_offsets;
+  if (fill_only) a.offsets = d_offsets;
+  else a.counts = d_counts;
   a.idx = d_idx;
   a.idx_cap = idx_cap;
   const int blocks = dp_grid_blocks(n, 4, 8192);
   return radius_dispatch(c->desc.nx, [&](auto NXc) -> int {
     constexpr int NX = decltype(NXc)::value;
+    const bool tail = a.nv > a.nv_sorted;
     if (!fill_only) {
-      k_radius<NX, false><<<blocks, 256, 0, s>>>(a);
+      if (tail) k_radius<NX, false, true><<<blocks, 256, 0, s>>>(a);
+      else k_radius<NX, false, false><<<blocks, 256, 0, s>>>(a);
       k_radius_offsets<<<1, 1024, 0, s>>>(d_counts, n, d_offsets, d_status);
     } else {
-      k_radius<NX, true><<<blocks, 256, 0, s>>>(a);
+      if (tail) k_radius<NX, true, true><<<blocks, 256, 0, s>>>(a);
+      else k_radius<NX, true, false><<<blocks, 256, 0, s>>>(a);
     }
     DP_HIP_RET(hipGetLastError());
     return DP_OK;
