@@ -28,13 +28,6 @@
 // Pair flag (limit_branching_factor == 0): a FREE pair after its node's
 // first FREE pair, CAPPED before the walk.
 #define DP_F_PRECAP 0x40
-// Pair flag (planar systems, limit_branching_factor > 0): a FREE pair past
-// its node's list window.  It stays a contender (later pairs test against
-// it) but gets no stored list of earlier conflicts; the walk scans the
-// contender grid for it if its node's cap does not fall before it.  (The
-// quadrotor's check stage uses this bit for its own state before it writes
-// the final flags, and never sets it for the walk.)
-#define DP_F_NOLIST 0x08
 // FP64 window of a quadrotor node, in FREE pairs: enough for the
 // cap of limit NOVEL pairs with a wide margin for duplicates.
 #define DP_FP64_WINDOW(limit) ((limit) < (1 << 28) ? 3 * (limit) + 32 : INT32_MAX)
@@ -63,8 +56,6 @@
 // Largest pinned staging buffer: three of them per context at most, and large
 // enough that a piece takes far longer on the host link than its launch.
 #define DP_STAGE_MAX (8ll << 20)
-// LDS per workgroup on gfx950
-#define DP_LDS_MAX 163840
 #define DP_SPIN_LIMIT_WAITING (1 << 10)
 // Earlier-conflict entries stored inline per pair (longer lists continue in
 // the overflow pool).

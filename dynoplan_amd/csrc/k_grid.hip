@@ -293,15 +293,14 @@ __device__ __forceinline__ void put_record(const double* fin, int64_t pcap, int3
 
 // Contender records into cell order, and the list window (planar systems,
 // limit > 0, window > 0): the contenders of a node after its first W in
-// canonical order are flagged DP_F_NOLIST, and their list length is set to
-// -(1 + rank) (rank among the node's contenders, at most 32766); the walk
-// scans the grid if it reaches one before the cap, which is slow (per lane,
-// and again on every retry).  The walks of the context's batches record in
-// need[0] the most contenders one of them went through; W is need + need / 4
-// + 16 (at least `least`), or `window` before the first batch: generous (20 * limit + 32, where
-// walks of 4096 unicycle1 nodes reach 79 contenders at the median and 342 at
-// most), since a first batch with W = 92 spent 13 to 17 ms scanning.  A fixed
-// window (need == null) is used as given.
+// canonical order get no list (bit 31 of their record, list length -1); the
+// walk scans the grid if it reaches one before the cap, which is slow (per
+// lane, and again on every retry).  The walks of the context's batches record
+// in need[0] the most contenders one of them went through; W is need + need / 4
+// + 16 (at least `least`), or `window` before the first batch: generous
+// (20 * limit + 32, where walks of 4096 unicycle1 nodes reach 79 contenders at
+// the median and 342 at most), since a first batch with W = 92 spent 13 to
+// 17 ms scanning.  A fixed window (need == null) is used as given.
 //
 // One wave per node, four nodes per workgroup, four chunks of 64 pairs per
 // step with their loads issued together (indices clamped into the node).
@@ -313,7 +312,8 @@ __device__ __forceinline__ void put_record(const double* fin, int64_t pcap, int3
 template <int NX>
 __global__ __launch_bounds__(256) void k_cont_scatter(int32_t N, const int32_t* __restrict__ app,
                                                       const int32_t* __restrict__ total,
-                                                      const int8_t* __restrict__ verdict, int8_t* __restrict__ flags,
+                                                      const int8_t* __restrict__ verdict,
+                                                      const int8_t* __restrict__ flags,
                                                       const double* __restrict__ fin, int64_t pcap,
                                                       const int32_t* __restrict__ count,
                                                       const int32_t* __restrict__ start,
@@ -358,8 +358,7 @@ __global__ __launch_bounds__(256) void k_cont_scatter(int32_t N, const int32_t* 
       if (!con) continue;
       bool nolist = (fl & 2) != 0;  // goal-forced: NOVEL without a list
       if (window > 0 && r >= window) {
-        flags[p] = (int8_t)(fl | DP_F_NOLIST);
-        conf_cnt[p] = (int16_t)(-1 - (r < 32766 ? r : 32766));
+        conf_cnt[p] = -1;
         nolist = true;
       }
       const int32_t cell = cell_u[u];
