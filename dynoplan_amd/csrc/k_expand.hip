@@ -433,7 +433,7 @@ struct dp_check_args {
   const double4* st4;    // [boxes][S] per state: (x, y, cos, sin) of the body, then the trailer's (offset x, y, cos, sin)
   const double* prec;    // [P][DP_PREC] what a pair reads of its primitive
   double reach[4];       // union of the swept boxes relative to a node (lo x, hi x, lo y, hi y)
-  int32_t ppw;           // pairs per wave, 1 to 64 (0: from the pair count)
+  int32_t ppw;           // pairs per wave, 2 to 64 (0: from the pair count)
   int32_t P;
   const int32_t* goalidx;
   int32_t num_goal, check_goal;
@@ -493,7 +493,10 @@ __device__ __forceinline__ void load_translated(const dp_check_args& a, int64_t 
 constexpr int kItemWindow = 4096;
 constexpr int kPairItems = 1 << 20;  // visited candidates of a pair past which it is a list of its own
 
-// Per-wave LDS of k_check_planar (6 KB for three components, 7 KB for five).
+// Per-wave LDS of k_check_planar: 9.5 KB for three components, 10.5 KB for
+// five.  A workgroup takes four of them, 0.9 KB of constants and 40 bytes per
+// obstacle, so three workgroups fit a CU (as many as the registers allow) up
+// to some 370 obstacles, with five components up to 270, and two up to 950.
 template <int NX>
 struct check_wave {
   uint64_t head[kItemWindow / 64];
@@ -514,6 +517,8 @@ struct check_wave {
     } vis;
   };
 };
+static_assert(sizeof(check_wave<3>) == 9728 && sizeof(check_wave<4>) == 10240 && sizeof(check_wave<5>) == 10752,
+              "the figures above");
 
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll

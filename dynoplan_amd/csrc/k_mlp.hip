@@ -180,8 +180,8 @@ constexpr int kInferWaves = 8;
 constexpr int kActStride = 256 + 8;   // bf16 per pair: rows 4 banks apart
 constexpr int kProdStride = 64 + 4;   // floats per pair
 struct infer_lds {
-  uint16_t act[2][2][32 * kActStride];  // [layer input][tile parity]
-  float prod[10][32 * kProdStride];     // wave 4 + w: w + 1 tiles
+  alignas(16) uint16_t act[2][2][32 * kActStride];  // [layer input][tile parity], read 16 bytes at a time
+  alignas(16) float prod[10][32 * kProdStride];     // wave 4 + w: w + 1 tiles
   float z[2][4][32];                    // [step parity][wave]
 };
 
