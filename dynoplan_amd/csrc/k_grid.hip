@@ -884,7 +884,9 @@ __device__ __forceinline__ void poll_pause(int32_t w, int32_t cap) {
 //
 // The quadrotor's pairs are mostly not FREE (4% of 550 per node): there the
 // FREE pairs are taken from a queue in LDS, filled from 256 pairs per step, so
-// a node is one chunk instead of nine (walk of 2048 nodes 55 -> 24 us).
+// a node is one chunk instead of nine (walk of 2048 nodes 55 -> 24 us).  With
+// balanced thrusts 92% of them are FREE, and that walk (with k_pre_nodes) is
+// not slower either: 104 -> 94 us.
 constexpr int kWalkQueue = 64 + 256;
 
 template <int NX>
@@ -1438,7 +1440,12 @@ __global__ __launch_bounds__(64) void k_round(round_args a) {
 // wave takes the lowest undecided lane as NOVEL, strikes its conflicts out
 // and so on: at most `limit` steps per node.  The grid, lists, pre-pass and
 // walk of a large batch are six launches and about 45 us at any size; this
-// takes 6.5-9 us for one node of 100 pairs, 4 us more per further node.
+// takes 6.5-9 us for one node of 100 pairs and 4 to 15 us more per further node
+// (its chunks, and up to `limit` steps).  Whole calls at a cap of 20, this
+// against the general path: unicycle1 (1000 primitives) 98 against 97 us with
+// five nodes and 108 against 99 with six, quadrotor with balanced thrusts
+// (2000) 269 against 265 with five, car (3000) 95 against 104 with five and 103
+// against 106 with six: four nodes are always on this side, five are not.
 constexpr int kSmallNodes = 4, kSmallNovel = 160;
 
 struct small_args {

@@ -195,7 +195,8 @@ class GpuExpander:
         return {"applicability": ms[0], "check": ms[1], "resolve": ms[2], "total": ms[3], "surrogate": ms[4]}
 
     def timing_detail(self):
-        """Device ms of the last expansion per kernel group (HIP events)."""
+        """Device ms of the last expansion per kernel group (the device clock at
+        each stage's first kernel)."""
         ms = (C.c_float * 7)()
         N.check(self.lib.dp_last_timing_detail(self.ctx, ms))
         keys = ("applicability", "surrogate", "check_pre", "check_main", "check_post", "lists", "walk")
